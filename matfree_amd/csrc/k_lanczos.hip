@@ -688,6 +688,28 @@ __device__ __forceinline__ int plane_group(int c4, int perm) {
 template <int V>
 __device__ __forceinline__ void store_planes(const PlaneOut& pl, int64_t p, int64_t i,
                                              const float (&v)[V]) {
+  if (pl.three) {
+    // the FP32 matvec's planes: 8 columns of a probe per 16-byte word
+    // (k_split3_probes); i % V == 0, so a group lies in one word
+    const int64_t word = (((i / 32) * (pl.Ppad / 32) + p / 32) * 2 + ((i >> 4) & 1)) * 64 +
+                         (p & 31) + 32 * ((i >> 3) & 1);
+    __bf16* dst = pl.hi + word * 8 + (i & 7);
+    struct __attribute__((aligned(2 * V))) Group {
+      __bf16 b[V];
+    } q[3];
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      // every second run of tiles holds -V (k_matvec_f32)
+      const float x = (i / (32 * kPlaneSignRun)) & 1 ? -v[u] : v[u];
+      q[0].b[u] = __bf16(x);
+      const float r = x - float(q[0].b[u]);
+      q[1].b[u] = __bf16(r);
+      q[2].b[u] = __bf16(r - float(q[1].b[u]));
+    }
+#pragma unroll
+    for (int w = 0; w < 3; ++w) *reinterpret_cast<Group*>(dst + w * pl.plane) = q[w];
+    return;
+  }
   if constexpr (V == 4) {  // i % 4 == 0: one group of four, one 8-byte store per plane
     const int64_t dst = ((i / 32) * pl.Ppad + p) * 32 + 4 * plane_group(int((i % 32) / 4), pl.perm);
     __bf16 h[4], l[4];

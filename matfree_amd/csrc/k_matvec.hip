@@ -2,29 +2,21 @@
 // (decomp.py:460), vmapped over probes (stochtrace.py:49), becomes one dense
 // contraction W[p][i] = sum_m A[i][m] V[p][m] on the matrix cores.
 //
-// FP32 path: v_mfma_f32_32x32x2f32 with D[i][p] (rows = output elements,
-// columns = probes).  A workgroup of 4 waves owns 128 output elements; each
-// wave owns 32 of them for 32 * NACC probes (NACC 32x32 accumulators).
+// FP32 path, D[i][p] on the matrix cores (rows = output elements, columns =
+// probes), in three forms (which one: launch_f32):
 //
-//  * A operand: each lane builds its own fragment in registers -- row
-//    i = i0 + 32 * wave + (lane & 31), contraction indices
-//    m0 + 16 * (lane >> 5) + s, s = 0..15 of the current BK = 32 tile.  For a
-//    stored matrix the 16 values are one contiguous 64-byte load (prefetched a
-//    tile ahead); for the RBF kernel they are generated in place from the
-//    lane's own point and the tile's 32 points, so every kernel entry is
-//    evaluated exactly once per matvec and never touches LDS.
-//  * B operand: the probe tile V[p0 .. p0 + 32 NACC)[m0 .. m0 + 32) is shared
-//    by the four waves through a double-buffered LDS tile (one barrier per
-//    tile; the next tile's global loads are in flight during the MFMAs).
-//  * Blocked summation: every tile accumulates into fresh registers that are
-//    then added to the running sums, so rounding grows with BK + n / BK rather
-//    than n (as in a blocked CPU GEMM).
-//
-// Within an MFMA the two lane halves carry two different contraction indices;
-// lane half h walks m in [16 h, 16 h + 16) of the tile, for both operands.
+//  * workgroup form (more than 32 probes): 128 rows x 64 or 128 probes, six
+//    products of three BF16 parts per factor; the probes' parts and the
+//    matrix tiles (or the tile's points) pass through LDS, an entry is formed
+//    once and used for every probe;
+//  * wave form (RBF, up to 32 probes): the same products, four waves sharing
+//    32 rows by tiles, no LDS sharing and no barrier in the loop;
+//  * stream form (stored matrix, up to 32 probes): v_mfma_f32_32x32x2f32 with
+//    the matrix loaded to LDS by a wave of its own.
 //
 // RBF: K_im = exp2(c |x_i - x_m|^2), c = -log2(e) / (2 l^2); the nugget
 // s2 * v is added in FP32 in the epilogue (never folded into a tile).
+#include <algorithm>
 #include <cmath>
 
 #include "slq_internal.h"
@@ -36,7 +28,6 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int BI = 128;      // output elements per workgroup
 constexpr int BK = 32;       // contraction tile
-constexpr int LDK = BK + 4;  // padded LDS row (floats)
 constexpr int kThreads = 256;
 
 struct RBFParams {
@@ -66,87 +57,17 @@ __device__ __forceinline__ void store4u(float* p, const float4& v) {
   __builtin_memcpy(p, &v, sizeof(v));
 }
 
-// V tile: (32 NACC) probes x 32 m = 8 NACC float4, NACC per thread.
-template <int NACC, bool VEC>
-__device__ __forceinline__ void load_v_tile(const float* __restrict__ V, int64_t P, int64_t n,
-                                            int64_t p0, int64_t m0, float4 (&reg)[NACC]) {
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int u = 0; u < NACC; ++u) {
-    const int f = t + u * kThreads;
-    const int row = f >> 3, c4 = f & 7;
-    const int64_t p = p0 + row, m = m0 + 4 * c4;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (p < P) {
-      const float* src = V + p * n + m;
-      if (VEC) {
-        if (m < n) v = *reinterpret_cast<const float4*>(src);
-      } else if (m + 4 <= n) {
-        v = load4u(src);
-      } else {
-        if (m + 0 < n) v.x = src[0];
-        if (m + 1 < n) v.y = src[1];
-        if (m + 2 < n) v.z = src[2];
-        if (m + 3 < n) v.w = src[3];
-      }
-    }
-    reg[u] = v;
-  }
-}
-
-template <int NACC>
-__device__ __forceinline__ void store_v_tile(float* Vs, const float4 (&reg)[NACC]) {
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int u = 0; u < NACC; ++u) {
-    const int f = t + u * kThreads;
-    const int row = f >> 3, c4 = f & 7;
-    *reinterpret_cast<float4*>(Vs + row * LDK + 4 * c4) = reg[u];
-  }
-}
-
-// The lane's 16 stored-matrix values A[row][m0 + 16 h + 0..15].
-template <bool VEC>
-__device__ __forceinline__ void load_a_frag(const float* __restrict__ A, int64_t n, int64_t row,
-                                            int64_t m0, int h, float (&a)[16]) {
-  const int64_t m = m0 + 16 * h;
-  if (row < n) {
-    const float* src = A + row * n + m;
-    if (m + 16 <= n) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float4 v = VEC ? *reinterpret_cast<const float4*>(src + 4 * q) : load4u(src + 4 * q);
-        a[4 * q + 0] = v.x;
-        a[4 * q + 1] = v.y;
-        a[4 * q + 2] = v.z;
-        a[4 * q + 3] = v.w;
-      }
-    } else {
-#pragma unroll
-      for (int s = 0; s < 16; ++s) a[s] = (m + s < n) ? src[s] : 0.f;
-    }
-  } else {
-#pragma unroll
-    for (int s = 0; s < 16; ++s) a[s] = 0.f;
-  }
-}
-
-// The lane's 16 generated RBF values exp2(-|x~_row - x~_m|^2) from scaled
-// coordinates x~ = s x, s = sqrt(log2(e) / (2 l^2)) (points past n staged at
-// kFarPoint, which gives exactly 0).
+// One generated RBF value exp2(-|x~_i - x~_m|^2) from scaled coordinates
+// x~ = s x, s = sqrt(log2(e) / (2 l^2)) (points past n staged at kFarPoint,
+// which gives exactly 0).
 template <int DIM>
-__device__ __forceinline__ void gen_rbf_frag(const float4* Xs, const float (&xr)[4], int h,
-                                             float (&a)[16]) {
-#pragma unroll
-  for (int s = 0; s < 16; ++s) {
-    const float4 xm = Xs[16 * h + s];
-    float d = xr[0] - xm.x;
-    float d2 = d * d;
-    if (DIM > 1) { d = xr[1] - xm.y; d2 = fmaf(d, d, d2); }
-    if (DIM > 2) { d = xr[2] - xm.z; d2 = fmaf(d, d, d2); }
-    if (DIM > 3) { d = xr[3] - xm.w; d2 = fmaf(d, d, d2); }
-    a[s] = __builtin_amdgcn_exp2f(-d2);
-  }
+__device__ __forceinline__ float rbf_entry(const float (&xr)[4], const float4& xm) {
+  float d = xr[0] - xm.x;
+  float d2 = d * d;
+  if (DIM > 1) { d = xr[1] - xm.y; d2 = fmaf(d, d, d2); }
+  if (DIM > 2) { d = xr[2] - xm.z; d2 = fmaf(d, d, d2); }
+  if (DIM > 3) { d = xr[3] - xm.w; d2 = fmaf(d, d, d2); }
+  return __builtin_amdgcn_exp2f(-d2);
 }
 
 // Epilogue: lane l of a 32x32 accumulator holds column (l & 31) and rows
@@ -196,131 +117,6 @@ __device__ __forceinline__ void store_out(float* __restrict__ W, const float* __
       }
     }
   }
-}
-
-template <int NACC, bool RBF, int DIM, bool VEC>
-__global__ void __launch_bounds__(kThreads)
-    k_matvec_f32(const float* __restrict__ A, RBFParams prm, const float* __restrict__ V,
-                 int64_t P, int64_t n, float* __restrict__ W) {
-  constexpr int BPW = 32 * NACC;  // probes per workgroup
-  __shared__ __attribute__((aligned(16))) float Vs[2][BPW * LDK];
-  __shared__ float4 Xs[2][BK];
-  const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6, r = lane & 31, h = lane >> 5;
-  const int64_t i0w = int64_t(blockIdx.x) * BI + 32 * wave;
-  const int64_t row = i0w + r;
-  const int64_t p0 = int64_t(blockIdx.y) * BPW;
-  // split-K: slice z of gridDim.z covers tiles [kt_begin, kt_end)
-  const int64_t all_tiles = (n + BK - 1) / BK;
-  const int64_t kt_begin = all_tiles * blockIdx.z / gridDim.z;
-  const int64_t kt_end = all_tiles * (blockIdx.z + 1) / gridDim.z;
-  const int64_t ntiles = kt_end - kt_begin;
-  const int64_t mbase = kt_begin * BK;
-  const bool split = gridDim.z > 1;
-  float* Wout = split ? W + int64_t(blockIdx.z) * P * n : W;
-
-  floatx16 acc[NACC];
-#pragma unroll
-  for (int c = 0; c < NACC; ++c)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[c][e] = 0.f;
-
-  // points relative to point 0 (translation invariance; both sides form the
-  // same FP32 difference), scaled
-  float x0[4] = {0.f, 0.f, 0.f, 0.f};
-  float xr[4] = {0.f, 0.f, 0.f, 0.f};
-  if (RBF && n > 0) {
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) x0[d] = prm.X[d];
-  }
-  if (RBF && row < n) {
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) xr[d] = (prm.X[row * DIM + d] - x0[d]) * prm.scale;
-  }
-  auto load_x = [&](int64_t m0) {
-    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    const int64_t m = m0 + t;
-    if (m < n) {
-      const float* src = prm.X + m * DIM;
-      x.x = (src[0] - x0[0]) * prm.scale;
-      if (DIM > 1) x.y = (src[1] - x0[1]) * prm.scale;
-      if (DIM > 2) x.z = (src[2] - x0[2]) * prm.scale;
-      if (DIM > 3) x.w = (src[3] - x0[3]) * prm.scale;
-    } else {
-      x = make_float4(kFarPoint, kFarPoint, kFarPoint, kFarPoint);
-    }
-    return x;
-  };
-
-  float4 vreg[NACC];
-  float areg[16];
-  float4 xnext = make_float4(0.f, 0.f, 0.f, 0.f);
-  load_v_tile<NACC, VEC>(V, P, n, p0, mbase, vreg);
-  store_v_tile<NACC>(Vs[0], vreg);
-  if (RBF) {
-    if (t < BK) Xs[0][t] = load_x(mbase);
-  } else {
-    load_a_frag<VEC>(A, n, row, mbase, h, areg);
-  }
-  __syncthreads();
-
-  for (int64_t kt = 0; kt < ntiles; ++kt) {
-    const int buf = int(kt & 1);
-    const int64_t m0 = mbase + kt * BK;
-    const bool more = kt + 1 < ntiles;
-    if (more) {
-      load_v_tile<NACC, VEC>(V, P, n, p0, m0 + BK, vreg);
-      if (RBF && t < BK) xnext = load_x(m0 + BK);
-    }
-    float a[16];
-    if (RBF) {
-      gen_rbf_frag<DIM>(Xs[buf], xr, h, a);
-    } else {
-#pragma unroll
-      for (int s = 0; s < 16; ++s) a[s] = areg[s];
-      if (more) load_a_frag<VEC>(A, n, row, m0 + BK, h, areg);
-    }
-
-    floatx16 tmp[NACC];
-#pragma unroll
-    for (int c = 0; c < NACC; ++c)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) tmp[c][e] = 0.f;
-    const float* vb = Vs[buf] + r * LDK + 16 * h;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      float4 b[NACC];
-#pragma unroll
-      for (int c = 0; c < NACC; ++c)
-        b[c] = *reinterpret_cast<const float4*>(vb + 32 * c * LDK + 4 * q);
-#pragma unroll
-      for (int c = 0; c < NACC; ++c)
-        tmp[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[4 * q + 0], b[c].x, tmp[c], 0, 0, 0);
-#pragma unroll
-      for (int c = 0; c < NACC; ++c)
-        tmp[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[4 * q + 1], b[c].y, tmp[c], 0, 0, 0);
-#pragma unroll
-      for (int c = 0; c < NACC; ++c)
-        tmp[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[4 * q + 2], b[c].z, tmp[c], 0, 0, 0);
-#pragma unroll
-      for (int c = 0; c < NACC; ++c)
-        tmp[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[4 * q + 3], b[c].w, tmp[c], 0, 0, 0);
-    }
-#pragma unroll
-    for (int c = 0; c < NACC; ++c)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[c][e] += tmp[c][e];
-
-    if (more) {
-      store_v_tile<NACC>(Vs[buf ^ 1], vreg);
-      if (RBF && t < BK) Xs[buf ^ 1][t] = xnext;
-    }
-    __syncthreads();
-  }
-  if (split)
-    store_out<NACC, VEC, false>(Wout, V, P, n, i0w, p0, acc, 0.f);
-  else
-    store_out<NACC, VEC, RBF>(Wout, V, P, n, i0w, p0, acc, prm.noise);
 }
 
 // ---------------------------------------------------------------------------
@@ -529,6 +325,953 @@ __device__ __forceinline__ void split_frag(const float (&a)[16], u32x4 (&hi)[2],
 __device__ __forceinline__ floatx16 mfma_bf16(const u32x4& a, const u32x4& b, const floatx16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
                                                  __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// ---------------------------------------------------------------------------
+// FP32 path on the BF16 matrix cores.
+// ---------------------------------------------------------------------------
+typedef __attribute__((address_space(1))) const void* GlobalPtr;
+typedef __attribute__((address_space(3))) void* LdsPtr;
+
+// Split two floats into three packed BF16 words: x = hi + mid + lo, exactly
+// for finite x below 2^127 (each part takes the next 8 significant bits,
+// round to nearest).
+__device__ __forceinline__ void split3_pair(float x0, float x1, uint32_t& hi, uint32_t& mid,
+                                            uint32_t& lo) {
+  auto unpack = [](uint32_t w) {
+    return f32x2{__builtin_bit_cast(float, w << 16), __builtin_bit_cast(float, w & 0xffff0000u)};
+  };
+  const f32x2 x = {x0, x1};
+  hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2));
+  const f32x2 r = x - unpack(hi);
+  mid = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+  lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(r - unpack(mid), bf16x2));
+}
+
+__device__ __forceinline__ uint32_t pack_bf16(float x0, float x1) {
+  const f32x2 x = {x0, x1};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2));
+}
+
+// One part of the split: word = bf16(x), returns x - word (exact).
+__device__ __forceinline__ float split_part(float x0, float x1, uint32_t& word, float& r1) {
+  const uint32_t w = pack_bf16(x0, x1);
+  word = w;
+  r1 = x1 - __builtin_bit_cast(float, w & 0xffff0000u);
+  return x0 - __builtin_bit_cast(float, w << 16);
+}
+
+// Wait until at most N of the wave's vector loads (to registers or LDS, which
+// finish in the order of issue) are in flight.
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  static_assert(N < 64, "vmcnt has six bits (3:0 and 15:14)");
+  __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | (N >> 4 << 14));
+}
+
+// Tiles of one plane sign (see k_matvec_f32).
+constexpr int kSignRun = kPlaneSignRun;
+__device__ __forceinline__ float tile_sign(int64_t kt) {
+  return (kt / kSignRun) & 1 ? -1.f : 1.f;
+}
+
+// The three BF16 planes of V, zero-padded to npad columns and Ppad probes, in
+// the order the MFMA B fragments are read: word (16 bytes, 8 columns)
+// ((kt * Ppad / 32 + p / 32) * 2 + kb) * 64 + (p % 32) + 32 h of a plane holds
+// columns 32 kt + 16 kb + 8 h .. + 7 of probe p, so that a workgroup's probe
+// tile is contiguous and a wave's fragment is 64 consecutive words (no bank
+// conflicts without padding).  One word per thread.
+__global__ void __launch_bounds__(256)
+    k_split3_probes(const float* __restrict__ V, int64_t P, int64_t n, int64_t npb, int64_t words,
+                    u32x4* __restrict__ planes) {
+  const int64_t stride = int64_t(gridDim.x) * blockDim.x;
+  for (int64_t w = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; w < words; w += stride) {
+    const int lane = int(w & 63), kb = int(w >> 6) & 1;
+    const int64_t blk = w >> 7;
+    const int64_t kt = blk / npb, p = (blk - kt * npb) * 32 + (lane & 31);
+    const int64_t m = kt * BK + 16 * kb + 8 * (lane >> 5);
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = 0.f;
+    if (p < P) {
+      const float* src = V + p * n + m;
+      if (m + 8 <= n) {
+        const float4 v0 = load4u(src), v1 = load4u(src + 4);
+        x[0] = v0.x; x[1] = v0.y; x[2] = v0.z; x[3] = v0.w;
+        x[4] = v1.x; x[5] = v1.y; x[6] = v1.z; x[7] = v1.w;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (m + e < n) x[e] = src[e];
+      }
+    }
+    const float sgn = tile_sign(kt);
+    u32x4 q[3];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      uint32_t hi, mid, lo;
+      split3_pair(sgn * x[2 * e], sgn * x[2 * e + 1], hi, mid, lo);
+      q[0][e] = hi;
+      q[1][e] = mid;
+      q[2][e] = lo;
+    }
+#pragma unroll
+    for (int u = 0; u < 3; ++u) planes[u * words + w] = q[u];
+  }
+}
+
+// The product of one 32-probe block on the FP32 matrix cores, straight from
+// global memory (tiles [kt0, kt1) of row `row`, probe p of the lane): taken by
+// a wave whose split product came out non-finite, so that infinities, NaN and
+// values that overflow BF16 give what FP32 arithmetic gives.
+template <bool RBF, int DIM>
+__device__ floatx16 f32_block(const float* __restrict__ A, const RBFParams& prm,
+                              const float (&x0)[4], const float (&xr)[4],
+                              const float* __restrict__ V, int64_t P, int64_t n, int64_t row,
+                              int64_t p, int64_t kt0, int64_t kt1) {
+  const int h = (threadIdx.x & 63) >> 5;
+  const float* arow = RBF ? nullptr : A + (row < n ? row : n - 1) * n;
+  const float* vrow = V + (p < P ? p : P - 1) * n;
+  // columns m .. m + 3 of a row, zero past n
+  auto load = [&](const float* src, int64_t m) {
+    if (m + 4 <= n) return load4u(src + m);
+    return make_float4(m < n ? src[m] : 0.f, m + 1 < n ? src[m + 1] : 0.f,
+                       m + 2 < n ? src[m + 2] : 0.f, 0.f);
+  };
+  auto rbf = [&](int64_t m) {
+    float4 xm = make_float4(kFarPoint, kFarPoint, kFarPoint, kFarPoint);
+    if (m < n) {
+      const float* src = prm.X + m * DIM;
+      xm.x = (src[0] - x0[0]) * prm.scale;
+      if (DIM > 1) xm.y = (src[1] - x0[1]) * prm.scale;
+      if (DIM > 2) xm.z = (src[2] - x0[2]) * prm.scale;
+      if (DIM > 3) xm.w = (src[3] - x0[3]) * prm.scale;
+    }
+    return rbf_entry<DIM>(xr, xm);
+  };
+  floatx16 sum;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) sum[e] = 0.f;
+#pragma unroll 1
+  for (int64_t kt = kt0; kt < kt1; ++kt) {
+    floatx16 tmp;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) tmp[e] = 0.f;
+    float4 a[4], v[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int64_t m = kt * BK + 16 * h + 4 * g;
+      v[g] = load(vrow, m);
+      if (RBF)
+        a[g] = make_float4(rbf(m), rbf(m + 1), rbf(m + 2), rbf(m + 3));
+      else
+        a[g] = load(arow, m);
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].x, v[g].x, tmp, 0, 0, 0);
+      tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].y, v[g].y, tmp, 0, 0, 0);
+      tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].z, v[g].z, tmp, 0, 0, 0);
+      tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].w, v[g].w, tmp, 0, 0, 0);
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sum[e] += tmp[e];
+  }
+  return sum;
+}
+
+// W = A V in FP32 from six BF16 products.  With a = a_h + a_m + a_l and
+// v = v_h + v_m + v_l (exact), a v = a_h v_h + (a_h v_m + a_m v_h) + (a_m v_m
+// + a_h v_l + a_l v_h) + dropped parts of at most 2^-26 |a v|, below the
+// rounding of one FP32 product; BF16 products are exact in FP32.  (Operands
+// below 2^-110 lose the parts that fall under BF16's subnormals.)  v_mfma
+// 32x32x16 BF16 runs 16 times the FP32 matrix rate, so six products take 3/8
+// of the FP32 form's matrix cycles.  The stored row (or the generated RBF
+// entries) is split in registers, once per wave and tile; the probes' planes
+// are split once per matvec (or by k_normalize).
+//
+// Rounding.  The MFMA aligns its eight products of a lane half to the largest
+// and drops the bits below it towards minus infinity (then adds the sum to C
+// rounded to nearest): a bias of one sign in every output, which a recursion
+// adds up (a decomposition's start-vector cotangent lost a factor of five).
+// So the planes hold V and -V in turns of kSignRun tiles, whose products are
+// added with that sign, and the biases cancel.  Sums are kept in levels (a
+// tile or a pair of tiles, 16 tiles, the slice), smallest products first:
+// against 64 bits the result is 1.2x (n = 1001) to 3x (n = 32768) nearer than
+// the FP32 MFMA chain's.
+constexpr int kTileRun = 16;
+
+
+// Workgroup form, for more than 32 probes: 128 rows x 32 NACC probes, 32 rows
+// per wave.  The matrix cores bound it (48 products of 32 cycles a tile and
+// wave at 128 probes); the vector instructions that form the next tile's parts
+// are dealt out between the products, since in one run they and the products
+// of the SIMD's other wave took turns.  Whole calls, FP32 MFMAs before: RBF
+// n = 32768, 128 probes 2446 -> 1390 us; stored n = 16384, 256 probes 1189 ->
+// 751, 128 probes 607 -> 410, 64 probes 351 -> 271 us.
+template <int NACC, bool RBF, int DIM>
+__global__ void __launch_bounds__(kThreads, 2)
+    k_matvec_f32(const float* __restrict__ A, RBFParams prm, const u32x4* __restrict__ planes,
+                 int64_t plane_words, int64_t npb, const float* __restrict__ V, int64_t P,
+                 int64_t n, float* __restrict__ W, int64_t wstride) {
+  constexpr int TW = 128 * NACC;  // words of one plane's tile
+  constexpr int kPieces = 3 * TW;
+  constexpr int PT = kPieces / kThreads;
+  // LDS, all double-buffered: the planes' tile; then the matrix tiles (per wave
+  // 32 rows x 8 pieces of 16 bytes, piece q of row r in slot q ^ (r & 7)) or,
+  // RBF, the coordinates of the tile's points.  One array, so that two
+  // workgroups with a 128-probe tile fill the CU's 160 KB exactly.
+  constexpr int kBytesB = 2 * kPieces * 16;
+  __shared__ __attribute__((aligned(16))) char lds[kBytesB + (RBF ? 2 * DIM * BK * 4 : 2 * 16384)];
+  u32x4* const Bs = reinterpret_cast<u32x4*>(lds);                // [2][kPieces]
+  float4* const As = reinterpret_cast<float4*>(lds + kBytesB);    // [2][4][256]
+  float* const Xs = reinterpret_cast<float*>(lds + kBytesB);      // [2][DIM][BK]
+  const int t = threadIdx.x;
+  const int lane = t & 63, wave = t >> 6, r = lane & 31, h = lane >> 5;
+  const int64_t i0w = int64_t(blockIdx.x) * BI + 32 * wave;
+  const int64_t row = i0w + r;
+  const int64_t p0 = int64_t(blockIdx.y) * 32 * NACC;
+  // split-K: slice z of gridDim.z covers tiles [kt_begin, kt_end), whole runs of
+  // one plane sign
+  const int64_t all_tiles = (n + BK - 1) / BK;
+  const int64_t runs = (all_tiles + kSignRun - 1) / kSignRun;
+  const int64_t kt_begin = runs * blockIdx.z / gridDim.z * kSignRun;
+  int64_t kt_end = runs * (blockIdx.z + 1) / gridDim.z * kSignRun;
+  if (kt_end > all_tiles) kt_end = all_tiles;
+  const int64_t ntiles = kt_end - kt_begin;
+  const bool split = gridDim.z > 1;
+  float* Wout = W + int64_t(blockIdx.z) * wstride;
+
+  floatx16 acc[NACC], sum[NACC];
+#pragma unroll
+  for (int c = 0; c < NACC; ++c)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[c][e] = sum[c][e] = 0.f;
+  // the sums of the last tiles move to the running sums
+  auto flush = [&](float sgn) {
+#pragma unroll
+    for (int c = 0; c < NACC; ++c)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        sum[c][e] = fmaf(sgn, acc[c][e], sum[c][e]);
+        if (!RBF) acc[c][e] = 0.f;
+      }
+  };
+
+  // points relative to point 0 (translation invariance; both sides form the
+  // same FP32 difference), scaled
+  float x0[4] = {0.f, 0.f, 0.f, 0.f};
+  float xr[4] = {0.f, 0.f, 0.f, 0.f};
+  if (RBF) {
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) x0[d] = prm.X[d];
+    if (row < n) {
+#pragma unroll
+      for (int d = 0; d < DIM; ++d) xr[d] = (prm.X[row * DIM + d] - x0[d]) * prm.scale;
+    }
+  }
+  // The loop runs over the slice's whole tiles (for RBF every tile: points
+  // past n are staged far away); the matrix's last, partial tile follows by
+  // itself with masked loads.  Loads past the last whole tile are clamped, so
+  // that the loop body is one basic block and the order pinned below holds.
+  const bool part = !RBF && kt_end == all_tiles && n % BK != 0;
+  const int64_t nwhole = part ? ntiles - 1 : ntiles;
+  auto clamp = [&](int64_t kt) { return kt < nwhole ? kt : nwhole - 1; };
+  // coordinate (t / 32) % DIM of point t % 32 of tile kt (the threads past
+  // 32 DIM load and write some of them again)
+  const int xd = (t >> 5) % DIM;
+  const float xo = RBF ? prm.X[xd] : 0.f;
+  auto load_x = [&](int64_t kt) {
+    const int64_t m = (kt_begin + kt) * BK + (t & (BK - 1));
+    return prm.X[(m < n ? m : n - 1) * DIM + xd];
+  };
+  auto store_x = [&](int64_t kt, int buf, float x) {
+    const bool ok = (kt_begin + kt) * BK + (t & (BK - 1)) < n;
+    Xs[(buf * DIM + xd) * BK + (t & (BK - 1))] = ok ? (x - xo) * prm.scale : kFarPoint;
+  };
+  const int uwave = __builtin_amdgcn_readfirstlane(wave);
+  // the wave's matrix tile kt into LDS: instruction u loads rows 8 u .. 8 u + 7,
+  // eight lanes per 128-byte row segment; rows past n read row n - 1 (their
+  // results are not stored)
+  const char* const abase =
+      RBF ? nullptr
+          : reinterpret_cast<const char*>(A + int64_t(blockIdx.x) * BI * n + kt_begin * BK);
+  uint32_t aoff[4];  // bytes from the workgroup's first row (128 n < 2^30 floats)
+  if (!RBF) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t i = i0w + 8 * u + (lane >> 3);
+      aoff[u] = uint32_t(((i < n ? i : n - 1) - int64_t(blockIdx.x) * BI) * n * 4 +
+                         16 * ((lane & 7) ^ (lane >> 3)));
+    }
+  }
+  auto load_a = [&](int64_t kt, int buf) {
+    const char* src = abase + kt * (BK * 4);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      __builtin_amdgcn_global_load_lds((GlobalPtr)(src + aoff[u]),
+                                       (LdsPtr)(As + (4 * buf + uwave) * 256 + 64 * u), 16, 0, 0);
+  };
+  // the planes' tile kt into LDS buffer buf, by direct loads to LDS (64
+  // consecutive words per wave and instruction, no registers); complete after
+  // wait_loads() and a barrier
+  const u32x4* pbase = planes + (kt_begin * npb + p0 / 32) * 128 + lane;
+  auto load_b = [&](int64_t kt, int buf) {
+    const u32x4* ptile = pbase + kt * npb * 128;
+#pragma unroll
+    for (int u = 0; u < PT; ++u) {
+      const int f = 64 * uwave + u * kThreads;  // uniform
+      __builtin_amdgcn_global_load_lds(
+          (GlobalPtr)(ptile + (u * kThreads / TW) * plane_words + f % TW), (LdsPtr)(Bs + buf * kPieces + f),
+          16, 0, 0);
+    }
+  };
+
+  // A fragments (three parts, two 16-deep halves) of the current / next tile;
+  // slots 8 kb + 0..7 of a lane: columns 16 kb + 8 h + 0..7
+  u32x4 fA[3][2], fB[3][2];
+  // Group g (slots 4 g .. 4 g + 3) of the next tile's fragment: four matrix
+  // entries (ga[0]) or the coordinates of four points (ga[d]) from LDS, the
+  // entries, and their parts, in eight pieces of about six instructions that
+  // go between the products.
+  auto read_group = [&](int buf, int g, float4 (&ga)[DIM]) {
+    if (RBF) {
+#pragma unroll
+      for (int d = 0; d < DIM; ++d)
+        ga[d] = *reinterpret_cast<const float4*>(Xs + (buf * DIM + d) * BK + 16 * (g >> 1) +
+                                                 8 * h + 4 * (g & 1));
+    } else {
+      const int q = 4 * (g >> 1) + 2 * h + (g & 1);
+      ga[0] = As[(4 * buf + wave) * 256 + r * 8 + (q ^ (r & 7))];
+    }
+  };
+  float ev[4];
+  auto piece = [&](int g, int m, const float4 (&ga)[DIM], u32x4 (&nxt)[3][2]) {
+    auto comp = [](const float4& v, int i) {
+      return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
+    };
+    if (m < 4) {
+      if (RBF) {
+        float4 xm = make_float4(comp(ga[0], m), 0.f, 0.f, 0.f);
+        if (DIM > 1) xm.y = comp(ga[DIM > 1 ? 1 : 0], m);
+        if (DIM > 2) xm.z = comp(ga[DIM > 2 ? 2 : 0], m);
+        if (DIM > 3) xm.w = comp(ga[DIM > 3 ? 3 : 0], m);
+        ev[m] = rbf_entry<DIM>(xr, xm);
+      } else {
+        ev[m] = comp(ga[0], m);
+      }
+      return;
+    }
+    const int e = 2 * ((m - 4) >> 1);  // pair of the group
+    const int kb = g >> 1, word = 2 * (g & 1) + e / 2;
+    uint32_t w;
+    ev[e] = split_part(ev[e], ev[e + 1], w, ev[e + 1]);
+    if ((m & 1) == 0) {
+      nxt[0][kb][word] = w;
+    } else {
+      nxt[1][kb][word] = w;
+      nxt[2][kb][word] = pack_bf16(ev[e], ev[e + 1]);
+    }
+  };
+
+  const u32x4* bsrc = Bs + lane;
+  auto read_b = [&](int buf, int q, int c, u32x4 (&d)[2]) {
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) d[kb] = bsrc[buf * kPieces + q * TW + c * 128 + kb * 64];
+  };
+
+  // acc += the products of the staged tile `buf` with fragment f; `first` is
+  // issued after the LDS reads of the first probe block, between(i) after MFMA
+  // i.  The probes' parts are taken in the order l, m, h, so that each part's
+  // registers are refilled for the next probe block as soon as its products
+  // are issued.  RBF: the run's first tile (fresh) starts the accumulators.
+  // Dense: every tile accumulates in fresh registers.
+  auto products = [&](int buf, float sgn, bool fresh, const u32x4 (&f)[3][2], auto first,
+                      auto between) {
+    u32x4 bl[2], bm[2], bh[2];
+    read_b(buf, 2, 0, bl);
+    read_b(buf, 1, 0, bm);
+    read_b(buf, 0, 0, bh);
+    __builtin_amdgcn_sched_barrier(0);
+    first();
+    __builtin_amdgcn_sched_barrier(0);
+    floatx16 tmp;
+#pragma unroll
+    for (int c = 0; c < NACC; ++c) {
+      floatx16& t0 = RBF ? acc[c] : tmp;
+      if (!RBF || fresh) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) t0[e] = 0.f;
+      }
+#pragma unroll
+      for (int i = 0; i < 12; ++i) {
+        const int kb = i & 1;
+        const u32x4 fa = i < 2 ? f[0][kb] : i < 4 ? f[1][kb] : i < 6 ? f[0][kb]
+                       : i < 8 ? f[2][kb] : i < 10 ? f[1][kb] : f[0][kb];
+        t0 = mfma_bf16(fa, i < 2 ? bl[kb] : i < 6 ? bm[kb] : bh[kb], t0);
+        if (c + 1 < NACC) {
+          if (i == 1) read_b(buf, 2, c + 1, bl);
+          if (i == 5) read_b(buf, 1, c + 1, bm);
+          if (i == 11) read_b(buf, 0, c + 1, bh);
+        }
+        between(12 * c + i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (!RBF) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[c][e] = fmaf(sgn, tmp[e], acc[c][e]);
+      }
+    }
+  };
+
+  if (nwhole > 0) {
+    // prologue: tile 0 staged and its fragment formed, the matrix (points) of
+    // tile 1 staged
+    load_b(0, 0);
+    if (RBF) {
+      const float a = load_x(0), b = load_x(clamp(1));
+      store_x(0, 0, a);
+      store_x(clamp(1), 1, b);
+    } else {
+      load_a(0, 0);
+      load_a(clamp(1), 1);
+    }
+    wait_loads<0>();
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float4 ga[DIM];
+      read_group(0, g, ga);
+#pragma unroll
+      for (int m = 0; m < 8; ++m) piece(g, m, ga, fA);
+    }
+    __syncthreads();  // the first buffers are refilled by step 0
+  }
+  // Step kt: the loads of the planes of tile kt + 1 and of the matrix (points)
+  // of tile kt + 2 are issued, then the products of tile kt, each followed by
+  // a piece of the fragment of tile kt + 1, so that the vector instructions
+  // issue while the matrix cores run (with the pieces in one run before the
+  // products the two units took turns).
+  auto step = [&](int64_t kt, int buf, const u32x4 (&cur)[3][2], u32x4 (&nxt)[3][2]) {
+    float xn = 0.f;
+    float4 ga[2][DIM];
+    constexpr int kSlots = 12 * NACC;
+    constexpr int kLead = 3;  // products before the first piece
+    products(
+        buf, tile_sign(kt_begin + kt), buf == 0, cur,
+        [&] {
+          load_b(clamp(kt + 1), buf ^ 1);
+          __builtin_amdgcn_sched_barrier(0);
+          if (RBF)
+            xn = load_x(clamp(kt + 2));
+          else
+            load_a(clamp(kt + 2), buf);
+        },
+        [&](int i) {
+          if (i == 0) {
+            if (!RBF) wait_loads<PT + 4>();  // the matrix tile kt + 1
+            read_group(buf ^ 1, 0, ga[0]);
+          }
+#pragma unroll
+          for (int m = 0; m < 32; ++m) {
+            if (kLead + m * (kSlots - kLead) / 32 != i) continue;
+            const int g = m >> 3;
+            if ((m & 7) == 0 && g < 3) read_group(buf ^ 1, g + 1, ga[(g + 1) & 1]);
+            piece(g, m & 7, ga[g & 1], nxt);
+          }
+        });
+    if (RBF) store_x(clamp(kt + 2), buf, xn);
+    // the planes of tile kt + 1 (the matrix tile kt + 2, issued last, may
+    // still be in flight)
+    wait_loads<RBF ? 0 : 4>();
+    __syncthreads();
+  };
+
+  int64_t kt = 0;
+  if constexpr (RBF) {
+    for (; kt + 1 < nwhole; kt += 2) {
+      step(kt, 0, fA, fB);
+      step(kt + 1, 1, fB, fA);
+      flush(tile_sign(kt_begin + kt));
+    }
+    if (kt < nwhole) {
+      step(kt, 0, fA, fB);
+      flush(tile_sign(kt_begin + kt));
+    }
+  } else {
+    while (kt + 1 < nwhole) {
+      const int64_t stop = kt + kTileRun < nwhole ? kt + kTileRun : nwhole;
+      for (; kt + 1 < stop; kt += 2) {
+        step(kt, 0, fA, fB);
+        step(kt + 1, 1, fB, fA);
+      }
+      flush(1.f);
+    }
+    if (kt < nwhole) step(kt, 0, fA, fB);
+  }
+  if (part) {
+    load_b(nwhole, 0);
+    const float* src = A + (row < n ? row : n - 1) * n;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int64_t m = (all_tiles - 1) * BK + 16 * (g >> 1) + 8 * h + 4 * (g & 1);
+      float4 ga[DIM];
+      ga[0].x = m < n ? src[m] : 0.f;
+      ga[0].y = m + 1 < n ? src[m + 1] : 0.f;
+      ga[0].z = m + 2 < n ? src[m + 2] : 0.f;
+      ga[0].w = m + 3 < n ? src[m + 3] : 0.f;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) piece(g, q, ga, fA);
+    }
+    wait_loads<0>();
+    __syncthreads();
+    products(0, tile_sign(all_tiles - 1), true, fA, [] {}, [](int) {});
+  }
+  if (!RBF) flush(1.f);
+  wait_loads<0>();  // no load to LDS in flight past here
+
+#pragma unroll
+  for (int c = 0; c < NACC; ++c) {
+    bool bad = false;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) bad |= !(fabsf(sum[c][e]) <= 3.4028235e38f);
+    if (__any(bad && p0 + 32 * c + r < P))
+      sum[c] = f32_block<RBF, DIM>(A, prm, x0, xr, V, P, n, row, p0 + 32 * c + r, kt_begin,
+                                   kt_end);
+  }
+  if (split)
+    store_out<NACC, false, false>(Wout, V, P, n, i0w, p0, sum, 0.f);
+  else
+    store_out<NACC, false, RBF>(Wout, V, P, n, i0w, p0, sum, prm.noise);
+}
+
+// The split A fragment of 16 values times sgn.
+__device__ __forceinline__ void split16(const float (&a)[16], float sgn, u32x4 (&f)[3][2]) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    uint32_t hi, mid, lo;
+    split3_pair(sgn * a[2 * e], sgn * a[2 * e + 1], hi, mid, lo);
+    f[0][e / 4][e % 4] = hi;
+    f[1][e / 4][e % 4] = mid;
+    f[2][e / 4][e % 4] = lo;
+  }
+}
+
+// acc + sgn times the six products of one tile with one block of 32 probes,
+// the tile's products in fresh registers (smallest first).
+__device__ __forceinline__ floatx16 block_products(const u32x4 (&f)[3][2], const u32x4 (&b)[3][2],
+                                                   float sgn, floatx16 acc) {
+  floatx16 tmp;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) tmp[e] = 0.f;
+  constexpr int pa[6] = {0, 1, 2, 0, 1, 0}, pb[6] = {2, 1, 0, 1, 0, 0};
+#pragma unroll
+  for (int i = 0; i < 12; ++i) tmp = mfma_bf16(f[pa[i / 2]][i & 1], b[pb[i / 2]][i & 1], tmp);
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = fmaf(sgn, tmp[e], acc[e]);
+  return acc;
+}
+
+// The end of a 32-row, 32-probe workgroup: the sums of waves 0-3 are added in
+// the order of the waves (red: 16 KB of LDS, free) and written, with the nugget
+// where asked; check(o) may replace a thread's four values in between.
+template <typename Check>
+__device__ __forceinline__ void store_block(float* red, const floatx16& sum, const RBFParams& prm,
+                                            bool nugget, const float* __restrict__ V, int64_t P,
+                                            int64_t n, int64_t i0, float* __restrict__ W,
+                                            int64_t wstride, Check check) {
+  const int t = threadIdx.x;
+  const int lane = t & 63, wave = t >> 6, r = lane & 31, h = lane >> 5;
+  __syncthreads();
+  if (wave < 4) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) red[(wave * 16 + e) * 64 + lane] = sum[e];
+  }
+  __syncthreads();
+  // thread t (waves 0-3): rows 8 wave + 4 h + 0..3 of probe r
+  float o[4] = {0.f, 0.f, 0.f, 0.f};
+  if (wave < 4) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = 4 * wave + u;
+      o[u] = red[e * 64 + lane];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) o[u] += red[(w * 16 + e) * 64 + lane];
+    }
+  }
+  check(o);
+  float* out = W + int64_t(blockIdx.z) * wstride + int64_t(r) * n;
+  const int64_t io = i0 + 8 * wave + 4 * h;
+  if (wave < 4 && r < P) {
+    const float* vp = V + int64_t(r) * n;
+    if (io + 4 <= n) {
+      if (nugget) {
+        const float4 v = load4u(vp + io);
+        o[0] = fmaf(prm.noise, v.x, o[0]);
+        o[1] = fmaf(prm.noise, v.y, o[1]);
+        o[2] = fmaf(prm.noise, v.z, o[2]);
+        o[3] = fmaf(prm.noise, v.w, o[3]);
+      }
+      store4u(out + io, make_float4(o[0], o[1], o[2], o[3]));
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (io + u < n) out[io + u] = nugget ? fmaf(prm.noise, vp[io + u], o[u]) : o[u];
+    }
+  }
+}
+
+// Wave form, for the RBF kernel and up to 32 probes, where forming the entries
+// on the vector units is the bound: a workgroup owns 32 rows, its four waves
+// take every fourth tile of the slice and their sums are added at the end, so
+// that small problems still give every CU work.  PLANES: the probes' parts
+// come from the planes, one tile ahead in registers; otherwise (small n, where
+// a launch of its own for the planes would cost more) the wave reads and
+// splits them itself.  Whole calls, FP32 MFMAs before: n = 10413, 2-D, 32
+// probes 95.5 -> 70.6 us; n = 32768, 3-D 792 -> 615; n = 2048, 16 probes
+// 16.4 -> 14.6 us.
+template <int DIM, bool PLANES>
+__global__ void __launch_bounds__(kThreads, 3)
+    k_matvec_f32_wave(RBFParams prm, const u32x4* __restrict__ planes, int64_t plane_words,
+                      const float* __restrict__ V, int64_t P, int64_t n,
+                      float* __restrict__ W, int64_t wstride) {
+  constexpr int kXW = (32 * DIM + 63) / 64;  // point coordinates per lane and tile
+  __shared__ __attribute__((aligned(16))) float lds[4096];
+  const int t = threadIdx.x;
+  const int lane = t & 63, wave = t >> 6, r = lane & 31, h = lane >> 5;
+  const int uwave = __builtin_amdgcn_readfirstlane(wave);
+  const int64_t i0 = int64_t(blockIdx.x) * 32;
+  const int64_t row = i0 + r;
+  const int64_t all_tiles = (n + BK - 1) / BK;
+  const int64_t runs = (all_tiles + kSignRun - 1) / kSignRun;
+  const int64_t kt_begin = runs * blockIdx.z / gridDim.z * kSignRun;
+  int64_t kt_end = runs * (blockIdx.z + 1) / gridDim.z * kSignRun;
+  if (kt_end > all_tiles) kt_end = all_tiles;
+  // the wave's tiles: kt_begin + uwave + 4 i, i < nw; without planes the last,
+  // partial tile of the vectors follows by itself with masked loads
+  const bool part = !PLANES && kt_end == all_tiles && n % BK != 0;
+  const int64_t kt_whole = part ? kt_end - 1 : kt_end;
+  const int64_t kt0 = kt_begin + uwave;
+  const int64_t nw = kt_whole > kt0 ? (kt_whole - kt0 + 3) / 4 : 0;
+  auto tile = [&](int64_t i) { return kt0 + 4 * (i < nw ? i : nw - 1); };
+
+  floatx16 acc, sum;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = sum[e] = 0.f;
+
+  // points relative to point 0, scaled (as in k_matvec_f32)
+  float x0[4] = {0.f, 0.f, 0.f, 0.f};
+  float xr[4] = {0.f, 0.f, 0.f, 0.f};
+  float xo[kXW];
+  float* xs = lds + wave * (2 * DIM * BK);  // the wave's tile points, two buffers
+#pragma unroll
+  for (int d = 0; d < DIM; ++d) x0[d] = prm.X[d];
+  if (row < n) {
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) xr[d] = (prm.X[row * DIM + d] - x0[d]) * prm.scale;
+  }
+#pragma unroll
+  for (int u = 0; u < kXW; ++u) xo[u] = prm.X[((64 * u + lane) >> 5) % DIM];
+  // coordinate ((64 u + lane) / 32) % DIM of point lane % 32 of tile kt
+  auto load_x = [&](int64_t kt, float (&x)[kXW]) {
+    const int64_t m = kt * BK + r;
+#pragma unroll
+    for (int u = 0; u < kXW; ++u)
+      x[u] = prm.X[(m < n ? m : n - 1) * DIM + ((64 * u + lane) >> 5) % DIM];
+  };
+  auto store_x = [&](int64_t kt, int buf, const float (&x)[kXW]) {
+    const bool ok = kt * BK + r < n;
+#pragma unroll
+    for (int u = 0; u < kXW; ++u)
+      xs[(buf * DIM + ((64 * u + lane) >> 5) % DIM) * BK + r] =
+          ok ? (x[u] - xo[u]) * prm.scale : kFarPoint;
+  };
+  // slots 8 kb + 0..7 of a lane: columns 16 kb + 8 h + 0..7 of tile kt; probes
+  // past P read probe P - 1 (not stored)
+  const float* vrow = V + (r < P ? r : P - 1) * n + 8 * h;
+  auto load_v = [&](int64_t kt, float (&a)[16]) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float4 v = load4u(vrow + kt * BK + 16 * (g >> 1) + 4 * (g & 1));
+      a[4 * g + 0] = v.x;
+      a[4 * g + 1] = v.y;
+      a[4 * g + 2] = v.z;
+      a[4 * g + 3] = v.w;
+    }
+  };
+  auto load_b = [&](int64_t kt, u32x4 (&b)[3][2]) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+        b[q][kb] = planes[q * plane_words + kt * 128 + kb * 64 + lane];
+  };
+  // the split fragment of the tile in point buffer buf
+  auto fragment = [&](int buf, u32x4 (&f)[3][2]) {
+    float a[16];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float4 c[DIM];
+#pragma unroll
+      for (int d = 0; d < DIM; ++d)
+        c[d] = *reinterpret_cast<const float4*>(xs + (buf * DIM + d) * BK + 16 * (g >> 1) + 8 * h +
+                                                4 * (g & 1));
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        auto comp = [&](int d) {
+          const float4 v = c[d < DIM ? d : 0];
+          return m == 0 ? v.x : m == 1 ? v.y : m == 2 ? v.z : v.w;
+        };
+        a[4 * g + m] = rbf_entry<DIM>(xr, make_float4(comp(0), comp(1), comp(2), comp(3)));
+      }
+    }
+    split16(a, 1.f, f);
+  };
+  auto flush = [&] {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      sum[e] += acc[e];
+      acc[e] = 0.f;
+    }
+  };
+
+  u32x4 bA[3][2], bB[3][2];
+  float va[16], vb[16], xn[kXW];
+  if (nw > 0) {
+    if (PLANES)
+      load_b(tile(0), bA);
+    else
+      load_v(tile(0), va);
+    load_x(tile(0), xn);
+    store_x(tile(0), 0, xn);
+  }
+  // Step i: the loads of the next tile are issued, then tile i's entries are
+  // formed, split and multiplied.
+  auto step = [&](int64_t i, int buf, u32x4 (&bc)[3][2], u32x4 (&bn)[3][2], const float (&vc)[16],
+                  float (&vn)[16]) {
+    if (PLANES)
+      load_b(tile(i + 1), bn);
+    else
+      load_v(tile(i + 1), vn);
+    load_x(tile(i + 1), xn);
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 f[3][2];
+    const float sgn = tile_sign(kt0 + 4 * i);
+    fragment(buf, f);
+    if (!PLANES) split16(vc, sgn, bc);
+    acc = block_products(f, bc, sgn, acc);
+    store_x(tile(i + 1), buf ^ 1, xn);
+  };
+  int64_t i = 0;
+  while (i + 1 < nw) {
+    const int64_t stop = i + kTileRun < nw ? i + kTileRun : nw;
+    for (; i + 1 < stop; i += 2) {
+      step(i, 0, bA, bB, va, vb);
+      step(i + 1, 1, bB, bA, vb, va);
+    }
+    flush();
+  }
+  if (i < nw) step(i, 0, bA, bB, va, vb);
+  if (part && (all_tiles - 1 - kt_begin) % 4 == uwave) {
+    const int64_t kt = all_tiles - 1;
+    const float sgn = tile_sign(kt);
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      const int col = 16 * (s >> 3) + (s & 7);
+      va[s] = kt * BK + 8 * h + col < n ? vrow[kt * BK + col] : 0.f;
+    }
+    load_x(kt, xn);
+    store_x(kt, 0, xn);
+    u32x4 f[3][2];
+    fragment(0, f);
+    split16(va, sgn, bA);
+    acc = block_products(f, bA, sgn, acc);
+  }
+  flush();
+
+  store_block(lds, sum, prm, gridDim.z == 1, V, P, n, i0, W, wstride, [&](float (&o)[4]) {
+    bool bad = false;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) bad |= !(fabsf(o[u]) <= 3.4028235e38f);
+    if (__syncthreads_or(bad && r < P)) {
+      const floatx16 full = f32_block<true, DIM>(nullptr, prm, x0, xr, V, P, n, row, r, kt_begin,
+                                                 kt_end);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        o[u] = wave == 0 ? full[u] : wave == 1 ? full[4 + u] : wave == 2 ? full[8 + u]
+                                                                          : full[12 + u];
+    }
+  });
+}
+
+// Stream form, for a stored matrix and up to 32 probes: the matrix's bytes are
+// the bound, and with one probe block per entry the FP32 matrix cores (1024
+// cycles a tile) keep up with HBM while splitting the entries for the BF16
+// ones does not.  A workgroup owns 32 rows, four waves multiply one tile each
+// of a block of 32 rows x 128 columns, and a fifth wave does nothing but load
+// the blocks to LDS, four ahead of the one in use.  Loads finish in the order
+// of issue within a wave, so a wave that loads both the matrix and the vectors
+// would wait for all of its matrix loads whenever it needs a vector; the
+// loader keeps up to 64 KB per workgroup in flight (two workgroups fill the
+// CU's LDS).  A row's piece of a block is 512 contiguous bytes: unaligned rows
+// read in the 128-byte rows of a tile reach 4.2 TB/s, in these pieces 4.9.
+// Whole calls with 32 probes, each wave loading its own rows before: n = 10413
+// 149 -> 117 us, 15001 271 -> 216, 4096 23.6 -> 19.7, 16384 225 -> 232 us.
+constexpr int kStreamWaves = 5;
+constexpr int kStreamStages = 5;
+__global__ void __launch_bounds__(64 * kStreamWaves, 3)
+    k_matvec_f32_stream(const float* __restrict__ A, const float* __restrict__ V, int64_t P,
+                        int64_t n, float* __restrict__ W, int64_t wstride) {
+  constexpr int kBlockTiles = 4;
+  __shared__ __attribute__((aligned(16))) float4 as[kStreamStages * 1024];
+  const int t = threadIdx.x;
+  const int lane = t & 63, wave = t >> 6, r = lane & 31, h = lane >> 5;
+  const int uwave = __builtin_amdgcn_readfirstlane(wave);
+  const int64_t i0 = int64_t(blockIdx.x) * 32;
+  const int64_t all_tiles = (n + BK - 1) / BK;
+  const int64_t runs = (all_tiles + kBlockTiles - 1) / kBlockTiles;
+  const int64_t kt_begin = runs * blockIdx.z / gridDim.z * kBlockTiles;
+  int64_t kt_end = runs * (blockIdx.z + 1) / gridDim.z * kBlockTiles;
+  if (kt_end > all_tiles) kt_end = all_tiles;
+  // the matrix's last, partial tile follows by itself with masked loads
+  const bool part = kt_end == all_tiles && n % BK != 0;
+  const int64_t nwhole = kt_end - kt_begin - (part ? 1 : 0);
+  const int64_t nblocks = (nwhole + kBlockTiles - 1) / kBlockTiles;
+
+  // The i-th block in the workgroup's order: every row block starts at another
+  // one, since rows a multiple of 4 KB apart have a column of every row on the
+  // same memory channel (32 probes, n = 16384: 258 -> 232 us, 12288: 148 -> 139,
+  // other n the same).
+  const int64_t rot = nblocks > 1 ? int64_t(blockIdx.x) % nblocks : 0;
+  auto order = [&](int64_t i) {
+    const int64_t b = i + rot;
+    return b < nblocks ? b : b - nblocks;
+  };
+
+  floatx16 sum;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) sum[e] = 0.f;
+  if (uwave == kStreamWaves - 1) {
+    // instruction u of a block: rows 2 u, 2 u + 1; piece q of a row goes to
+    // slot q ^ (row & 7) (conflict-free fragment reads).  Pieces past the
+    // row's last whole one are clamped (their tile is not whole), rows past n
+    // read row n - 1, blocks past the last one the last.
+    const uint32_t last = uint32_t(n - 4 - kt_begin * BK) * 4;
+    const int rr = lane >> 5;
+    auto load_block = [&](int64_t b, int stage) {
+      const uint32_t c0 = uint32_t(order(b < nblocks ? b : nblocks - 1)) * (kBlockTiles * BK * 4);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const int64_t i = i0 + 2 * u + rr;
+        const uint32_t c = c0 + 16u * uint32_t((lane & 31) ^ ((2 * u + rr) & 7));
+        const char* src = reinterpret_cast<const char*>(A + (i < n ? i : n - 1) * n +
+                                                        kt_begin * BK);
+        __builtin_amdgcn_global_load_lds((GlobalPtr)(src + (c < last ? c : last)),
+                                         (LdsPtr)(as + stage * 1024 + 64 * u), 16, 0, 0);
+      }
+    };
+    if (nblocks > 0) {
+#pragma unroll
+      for (int b = 0; b < kStreamStages - 1; ++b) load_block(b, b);
+      int stage = kStreamStages - 1;
+      for (int64_t b = 0; b < nblocks; ++b) {
+        wait_loads<16 * (kStreamStages - 2)>();  // block b is in LDS
+        // (a bare barrier: __syncthreads() waits for every load to LDS)
+        __builtin_amdgcn_s_barrier();  // and block b - 1 is free
+        __builtin_amdgcn_sched_barrier(0);
+        load_block(b + kStreamStages - 1, stage);
+        stage = stage == kStreamStages - 1 ? 0 : stage + 1;
+      }
+    }
+    wait_loads<0>();
+  } else {
+    // An MFMA carries two contraction indices, one per lane half: half h walks
+    // columns 16 h .. 16 h + 15 of the tile for both operands.  Probes past P
+    // read probe P - 1 (not stored).
+    floatx16 acc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+    const float* vrow = V + (r < P ? r : P - 1) * n + kt_begin * BK + 16 * h;
+    auto load_v = [&](int64_t kt, float4 (&v)[4]) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) v[g] = load4u(vrow + kt * BK + 4 * g);
+    };
+    auto tile_products = [&](const float4 (&a)[4], const float4 (&v)[4]) {
+      floatx16 tmp;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) tmp[e] = 0.f;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].x, v[g].x, tmp, 0, 0, 0);
+        tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].y, v[g].y, tmp, 0, 0, 0);
+        tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].z, v[g].z, tmp, 0, 0, 0);
+        tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].w, v[g].w, tmp, 0, 0, 0);
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[e] += tmp[e];
+    };
+    // Block b: its fragment is read from LDS and its vectors loaded while the
+    // products of the block before run.
+    float4 aA[4], aB[4], vA[4], vB[4];
+    bool live = false;  // the tile read last exists (the last block may miss some)
+    auto block = [&](int64_t b, int stage, const float4 (&ac)[4], float4 (&an)[4],
+                     const float4 (&vc)[4], float4 (&vn)[4]) {
+      const int64_t kt = order(b) * kBlockTiles + uwave;
+      __syncthreads();
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int q = 8 * uwave + 4 * h + g;
+        an[g] = as[stage * 1024 + r * 32 + (q ^ (r & 7))];
+      }
+      load_v(kt < nwhole ? kt : nwhole - 1, vn);
+      __builtin_amdgcn_sched_barrier(0);
+      if (live) tile_products(ac, vc);
+      live = kt < nwhole;
+    };
+    int stage = 0;
+    int64_t b = 0;
+    auto next = [&] { stage = stage == kStreamStages - 1 ? 0 : stage + 1; };
+    while (b < nblocks) {
+      const int64_t stop = b + kTileRun < nblocks ? b + kTileRun : nblocks;
+      for (; b + 1 < stop; b += 2) {
+        block(b, stage, aB, aA, vB, vA);
+        next();
+        block(b + 1, stage, aA, aB, vA, vB);
+        next();
+      }
+      if (b < stop) break;  // the slice's odd last block
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        sum[e] += acc[e];
+        acc[e] = 0.f;
+      }
+    }
+    if (b < nblocks) {
+      block(b, stage, aB, aA, vB, vA);
+      if (live) tile_products(aA, vA);
+    } else if (nblocks > 0 && live) {
+      tile_products(aB, vB);
+    }
+    if (part && (all_tiles - 1) % 4 == uwave) {
+      const int64_t m0 = (all_tiles - 1) * BK + 16 * h;
+      const float* src = A + (i0 + r < n ? i0 + r : n - 1) * n;
+      const float* vp = V + (r < P ? r : P - 1) * n;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int64_t m = m0 + 4 * g;
+        aA[g] = make_float4(m < n ? src[m] : 0.f, m + 1 < n ? src[m + 1] : 0.f,
+                           m + 2 < n ? src[m + 2] : 0.f, m + 3 < n ? src[m + 3] : 0.f);
+        vA[g] = make_float4(m < n ? vp[m] : 0.f, m + 1 < n ? vp[m + 1] : 0.f,
+                            m + 2 < n ? vp[m + 2] : 0.f, m + 3 < n ? vp[m + 3] : 0.f);
+      }
+      tile_products(aA, vA);
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sum[e] += acc[e];
+  }
+  RBFParams prm{};
+  store_block(reinterpret_cast<float*>(as), sum, prm, false, V, P, n, i0, W, wstride,
+              [](float (&)[4]) {});
 }
 
 // RBF exponents for the BF16 kernels.  The base-2 exponent of a 32 x 32 tile,
@@ -1679,29 +2422,69 @@ hipError_t launch_tpl_bf16(hipStream_t s, const float* A, const u32x4* rec, cons
   return launch_tpl_bf16_n<NACC, RBF, 1>(s, A, rec, prm, Vhi, Vlo, Ppad, V, P, n, W, vec, S);
 }
 
-template <int NACC, bool RBF, int DIM>
-hipError_t launch_tpl(hipStream_t s, const float* A, const RBFParams& prm, const float* V,
-                      int64_t P, int64_t n, float* W, bool vec, int S) {
-  const dim3 grid(unsigned((n + BI - 1) / BI), unsigned((P + 32 * NACC - 1) / (32 * NACC)),
+int nacc_for(int64_t P) { return P <= 32 ? 1 : (P <= 64 ? 2 : 4); }
+
+// Whether the FP32 matvec of P vectors reads planes: not the stream form of a
+// stored matrix (up to 32 probes), and not the wave form at small n, where the
+// waves split the vectors themselves (the launch that writes the planes costs
+// about 3.5 us, splitting in the waves 0.2 us per 1000 columns).
+bool f32_planes(int64_t n, int64_t P, bool rbf) {
+  return nacc_for(P) > 1 || (rbf && n >= 4096);
+}
+
+// The FP32 matvec of P vectors (a group of the launch's probes) from planes
+// of npb blocks of 32 probes; out: W, or the first of S partial planes of
+// wstride floats.
+template <bool RBF, int DIM>
+hipError_t launch_f32(hipStream_t s, const float* A, const RBFParams& prm, const u32x4* planes,
+                      int64_t plane_words, int64_t npb, const float* V, int64_t P, int64_t n,
+                      float* out, int64_t wstride, int S) {
+  const int nacc = nacc_for(P);
+  const dim3 grid(unsigned((n + BI - 1) / BI), unsigned((P + 32 * nacc - 1) / (32 * nacc)),
                   unsigned(S));
-  if (vec)
-    hipLaunchKernelGGL((k_matvec_f32<NACC, RBF, DIM, true>), grid, dim3(kThreads), 0, s, A, prm,
-                       V, P, n, W);
-  else
-    hipLaunchKernelGGL((k_matvec_f32<NACC, RBF, DIM, false>), grid, dim3(kThreads), 0, s, A, prm,
-                       V, P, n, W);
+  if (nacc == 1) {
+    const dim3 wgrid(unsigned((n + 31) / 32), 1, unsigned(S));
+    if constexpr (!RBF)
+      hipLaunchKernelGGL(k_matvec_f32_stream, wgrid, dim3(64 * kStreamWaves), 0, s, A, V, P, n,
+                         out, wstride);
+    else if (f32_planes(n, P, true))
+      hipLaunchKernelGGL((k_matvec_f32_wave<DIM, true>), wgrid, dim3(kThreads), 0, s, prm, planes,
+                         plane_words, V, P, n, out, wstride);
+    else
+      hipLaunchKernelGGL((k_matvec_f32_wave<DIM, false>), wgrid, dim3(kThreads), 0, s, prm,
+                         planes, plane_words, V, P, n, out, wstride);
+  } else if (nacc == 2) {
+    hipLaunchKernelGGL((k_matvec_f32<2, RBF, DIM>), grid, dim3(kThreads), 0, s, A, prm, planes,
+                       plane_words, npb, V, P, n, out, wstride);
+  } else {
+    hipLaunchKernelGGL((k_matvec_f32<4, RBF, DIM>), grid, dim3(kThreads), 0, s, A, prm, planes,
+                       plane_words, npb, V, P, n, out, wstride);
+  }
   return hipGetLastError();
 }
 
-template <bool RBF, int DIM>
-hipError_t launch_f32(hipStream_t s, const float* A, const RBFParams& prm, const float* V,
-                      int64_t P, int64_t n, float* W, bool vec, int S) {
-  if (P <= 32) return launch_tpl<1, RBF, DIM>(s, A, prm, V, P, n, W, vec, S);
-  if (P <= 64) return launch_tpl<2, RBF, DIM>(s, A, prm, V, P, n, W, vec, S);
-  return launch_tpl<4, RBF, DIM>(s, A, prm, V, P, n, W, vec, S);
+hipError_t launch_f32_any(hipStream_t s, const slq_operator& op, const RBFParams& prm,
+                          const u32x4* planes, int64_t plane_words, int64_t npb, const float* V,
+                          int64_t P, float* out, int64_t wstride, int S) {
+  const int64_t n = op.n;
+  if (op.kind == SLQ_OP_DENSE)
+    return launch_f32<false, 1>(s, op.matrix, prm, planes, plane_words, npb, V, P, n, out, wstride,
+                                S);
+  switch (op.dim) {
+    case 1:
+      return launch_f32<true, 1>(s, nullptr, prm, planes, plane_words, npb, V, P, n, out, wstride,
+                                 S);
+    case 2:
+      return launch_f32<true, 2>(s, nullptr, prm, planes, plane_words, npb, V, P, n, out, wstride,
+                                 S);
+    case 3:
+      return launch_f32<true, 3>(s, nullptr, prm, planes, plane_words, npb, V, P, n, out, wstride,
+                                 S);
+    default:
+      return launch_f32<true, 4>(s, nullptr, prm, planes, plane_words, npb, V, P, n, out, wstride,
+                                 S);
+  }
 }
-
-int nacc_for(int64_t P) { return P <= 32 ? 1 : (P <= 64 ? 2 : 4); }
 
 // Ring depth of the packed matvec: 8 KB of tile planes in flight per wave
 // (BF16 planes 2 KB per tile, FP8 planes 1 KB).
@@ -1781,6 +2564,33 @@ int choose_splitk(int64_t n, int64_t P, int64_t avail_floats, bool fp32) {
   return S;
 }
 
+// Column slices of the FP32 matvec, up to the factor above (which sizes the
+// scratch).  Workgroup form: the last round of resident workgroups (two per
+// CU) filled best.  Wave form: three per CU.  Stream form: one per CU runs
+// faster than two that share the CU's part of the bandwidth (n = 4096, 32
+// probes: 20 us in 256 workgroups, 27 in 512), so rounds of 256, by up to
+// three slices (10413: 1, 2, 3 slices take 143, 121, 117 us).
+int choose_splitk_f32(int64_t n, int64_t P, bool rbf) {
+  const int most = choose_splitk(n, P, int64_t(1) << 60, true);
+  const int64_t nacc = nacc_for(P);
+  const bool stream = nacc == 1 && !rbf;
+  const int64_t wgs = nacc == 1 ? (n + 31) / 32
+                                : (n + BI - 1) / BI * ((P + 32 * nacc - 1) / (32 * nacc));
+  const int64_t resident = stream ? 256 : (nacc == 1 ? 768 : 512);
+  if (stream && wgs <= resident) return int(std::min<int64_t>(most, resident / wgs));
+  int best = 1;
+  double fill = 0.0;
+  for (int S = 1; S <= (stream ? std::min(most, 3) : most); ++S) {
+    const double rounds = double(wgs * S) / double(resident);
+    const double f = rounds / std::ceil(rounds);
+    if (f > fill + 0.02) {
+      fill = f;
+      best = S;
+    }
+  }
+  return best;
+}
+
 // Derivative-kernel contraction: columns in launches of G column blocks of
 // 128 (NACC = 4; planes of 128 G x npad split-BF16 values, G <= 8) and S
 // column slices (the slices add to the partial sums, so they need no partial
@@ -1854,10 +2664,34 @@ hipError_t launch_pack_matrix(hipStream_t s, const float* A, int64_t n, int stor
   return hipGetLastError();
 }
 
-int64_t matvec_scratch_floats(int64_t n, int64_t P) {
-  const int64_t bpw = 32 * nacc_for(P);
-  const int64_t Ppad = (P + bpw - 1) / bpw * bpw;
-  const int64_t npad = (n + BK - 1) / BK * BK;
+namespace {
+
+// Padded sizes of the planes of P probes.
+struct PlaneSizes {
+  int64_t npad, Ppad;
+  PlaneSizes(int64_t n, int64_t P) {
+    const int64_t bpw = 32 * nacc_for(P);
+    npad = (n + BK - 1) / BK * BK;
+    Ppad = (P + bpw - 1) / bpw * bpw;
+  }
+};
+
+bool rows_kernel(const slq_operator& op, int64_t P) {
+  return op.kind == SLQ_OP_RBF && P <= kRowsMaxP && op.dim >= 1 && op.dim <= 4;
+}
+bool packed_op(const slq_operator& op) {
+  return op.kind == SLQ_OP_DENSE && op.storage != SLQ_STORE_FP32;
+}
+bool fp32_op(const slq_operator& op) { return op.precision == SLQ_PREC_FP32 && !packed_op(op); }
+
+// Floats of the FP32 matvec's three BF16 planes of `probes` (padded) probes.
+int64_t f32_plane_floats(int64_t npad, int64_t probes) { return 3 * npad * probes / 2; }
+
+}  // namespace
+
+int64_t matvec_scratch_floats(const slq_operator& op, int64_t P, bool lean) {
+  const int64_t n = op.n;
+  const PlaneSizes z(n, P);
   // the split-K slices a launch takes when scratch does not limit them (the
   // larger of the FP32 and the BF16 choice, and the few-vector row kernel's)
   const int64_t unlimited = int64_t(1) << 60;
@@ -1868,20 +2702,35 @@ int64_t matvec_scratch_floats(int64_t n, int64_t P) {
     const int Sr = choose_rows_splitk(n, P, unlimited);
     if (Sr > S) S = Sr;
   }
-  // partial sums + two BF16 planes + the RBF point records (16 floats each)
-  return int64_t(S) * P * n + Ppad * npad + 16 * npad;
+  // partial sums + two BF16 planes + the RBF point records (16 floats each);
+  // the FP32 matvec takes a third plane (for up to 32 probes it fits the
+  // records' place)
+  int64_t planes = z.Ppad * z.npad + 16 * z.npad;
+  if (!lean && fp32_op(op) && !rows_kernel(op, P)) {
+    const int64_t three = f32_plane_floats(z.npad, z.Ppad);
+    if (three > planes) planes = three;
+  }
+  return int64_t(S) * P * n + planes;
 }
 
-PlaneOut matvec_planes(const slq_operator& op, int64_t P, float* scratch) {
+PlaneOut matvec_planes(const slq_operator& op, int64_t P, float* scratch, int64_t scratch_floats) {
   PlaneOut out;
-  const bool rows = op.kind == SLQ_OP_RBF && P <= kRowsMaxP && op.dim >= 1 && op.dim <= 4;
-  const bool packed = op.kind == SLQ_OP_DENSE && op.storage != SLQ_STORE_FP32;
-  if (rows || (op.precision == SLQ_PREC_FP32 && !packed) || !scratch) return out;
-  const int64_t npad = (op.n + BK - 1) / BK * BK;
-  const int64_t bpw = 32 * nacc_for(P);
-  out.Ppad = (P + bpw - 1) / bpw * bpw;
+  if (rows_kernel(op, P) || !scratch) return out;
+  const PlaneSizes z(op.n, P);
+  if (fp32_op(op)) {
+    // with less scratch the launch splits groups of probes by itself
+    if (!f32_planes(op.n, P, op.kind == SLQ_OP_RBF)) return out;
+    const int64_t S = choose_splitk_f32(op.n, P, op.kind == SLQ_OP_RBF);
+    if (f32_plane_floats(z.npad, z.Ppad) + S * P * op.n > scratch_floats) return out;
+    out.Ppad = z.Ppad;
+    out.hi = reinterpret_cast<__bf16*>(scratch);
+    out.plane = z.Ppad * z.npad;
+    out.three = 1;
+    return out;
+  }
+  out.Ppad = z.Ppad;
   out.hi = reinterpret_cast<__bf16*>(scratch);
-  out.lo = (!packed && op.precision == SLQ_PREC_BF16X3) ? out.hi + out.Ppad * npad : nullptr;
+  out.lo = (!packed_op(op) && op.precision == SLQ_PREC_BF16X3) ? out.hi + z.Ppad * z.npad : nullptr;
   out.perm = op.kind == SLQ_OP_RBF ? 1 : 0;
   return out;
 }
@@ -1892,7 +2741,7 @@ hipError_t launch_matvec(hipStream_t s, const slq_operator& op, const float* V, 
   if (defer) *defer = MvSplitSum{};
   const int64_t n = op.n;
   if (n <= 0 || P <= 0) return hipSuccess;
-  if (op.kind == SLQ_OP_RBF && P <= kRowsMaxP && op.dim >= 1 && op.dim <= 4) {
+  if (rows_kernel(op, P)) {
     // a few vectors: the row kernels in FP32 (every precision gets FP32
     // here); for dimension <= 3 with the exponents from the matrix cores,
     // the point records at the start of the scratch, the partial sums after
@@ -1954,27 +2803,66 @@ hipError_t launch_matvec(hipStream_t s, const slq_operator& op, const float* V, 
     return hipGetLastError();
   }
   const bool vec = (n % 4 == 0) && aligned16(V) && aligned16(W);
-  const bool packed = op.kind == SLQ_OP_DENSE && op.storage != SLQ_STORE_FP32;
-  const bool fp32 = op.precision == SLQ_PREC_FP32 && !packed;
+  const bool packed = packed_op(op);
+  const bool fp32 = fp32_op(op);
   const int nprod = packed ? 1
                            : (op.precision == SLQ_PREC_BF16X3
                                   ? 3
                                   : (op.precision == SLQ_PREC_BF16X2 ? 2 : 1));
-  // scratch layout: [BF16 planes, RBF point records (bf16 path only)]
-  // [split-K partial sums]
-  int64_t planes_floats = 0;
-  __bf16 *Vhi = nullptr, *Vlo = nullptr;
-  u32x4* rec = nullptr;
-  const int64_t npad = (n + BK - 1) / BK * BK;
-  const int64_t bpw = 32 * nacc_for(P);
-  const int64_t Ppad = (P + bpw - 1) / bpw * bpw;
-  if (!fp32) {
-    if (!scratch) return hipErrorInvalidValue;
-    planes_floats = Ppad * npad + 16 * npad;
+  if (!scratch) return hipErrorInvalidValue;
+  const int64_t npad = PlaneSizes(n, P).npad, Ppad = PlaneSizes(n, P).Ppad;
+  RBFParams prm{};
+  hipError_t err = hipSuccess;
+  const float rbf_coef = float(-1.4426950408889634 / (2.0 * op.lengthscale * op.lengthscale));
+  const float rbf_scale = float(sqrt(1.4426950408889634 / (2.0 * op.lengthscale * op.lengthscale)));
+  if (op.kind == SLQ_OP_RBF) {
+    prm.X = op.points;
+    prm.dim = op.dim;
+    prm.coef = rbf_coef;
+    prm.scale = rbf_scale;
+    prm.noise = float(op.noise);
+  }
+  float* partial = nullptr;
+  int S = 1;
+  if (fp32) {
+    // scratch layout: [three BF16 planes of a group of probes][split-K
+    // partial sums].  The group is every probe unless the scratch is the lean
+    // size, where the planes of a part of them fit at a time; a probe's
+    // result does not depend on the grouping.
+    S = choose_splitk_f32(n, P, op.kind == SLQ_OP_RBF);
+    const int64_t sums = S > 1 ? int64_t(S) * P * n : 0;
+    int64_t group = Ppad;
+    if (f32_plane_floats(npad, Ppad) + sums > scratch_floats) {
+      group = (scratch_floats - sums) / f32_plane_floats(npad, 1);
+      group = group >= 128 ? group / 128 * 128 : (group >= 64 ? 64 : group / 32 * 32);
+      if (group <= 0) return hipErrorInvalidValue;
+    }
+    u32x4* planes = reinterpret_cast<u32x4*>(scratch);
+    partial = scratch + f32_plane_floats(npad, group);
+    const bool ready = !f32_planes(n, P, op.kind == SLQ_OP_RBF) || ((flags & kMvPlanesReady) && group == Ppad);
+    if (ready && ev0) (void)hipEventRecord(ev0, s);
+    for (int64_t p0 = 0; p0 < P && err == hipSuccess; p0 += group) {
+      const int64_t Pg = P - p0 < group ? P - p0 : group;
+      const PlaneSizes zg(n, Pg);
+      const int64_t words = zg.Ppad * npad / 8;
+      if (!ready) {
+        int64_t blocks = (words + 255) / 256;
+        if (blocks > 8192) blocks = 8192;
+        hipLaunchKernelGGL(k_split3_probes, dim3(unsigned(blocks)), dim3(256), 0, s, V + p0 * n,
+                           Pg, n, zg.Ppad / 32, words, planes);
+        if ((err = hipGetLastError()) != hipSuccess) break;
+        if (p0 == 0 && ev0) (void)hipEventRecord(ev0, s);
+      }
+      err = launch_f32_any(s, op, prm, planes, words, zg.Ppad / 32, V + p0 * n, Pg,
+                           (S > 1 ? partial : W) + p0 * n, P * n, S);
+    }
+  } else {
+    // scratch layout: [BF16 planes, RBF point records][split-K partial sums]
+    const int64_t planes_floats = Ppad * npad + 16 * npad;
     if (planes_floats > scratch_floats) return hipErrorInvalidValue;
-    Vhi = reinterpret_cast<__bf16*>(scratch);
-    Vlo = Vhi + Ppad * npad;
-    rec = reinterpret_cast<u32x4*>(scratch + Ppad * npad);
+    __bf16* Vhi = reinterpret_cast<__bf16*>(scratch);
+    __bf16* Vlo = Vhi + Ppad * npad;
+    u32x4* rec = reinterpret_cast<u32x4*>(scratch + Ppad * npad);
     if (!(flags & kMvPlanesReady)) {
       int64_t blocks = (Ppad * npad / 4 + 255) / 256;
       if (blocks > 8192) blocks = 8192;
@@ -1985,53 +2873,31 @@ hipError_t launch_matvec(hipStream_t s, const slq_operator& op, const float* V, 
       else
         hipLaunchKernelGGL(k_split_probes<false>, dim3(unsigned(blocks)), dim3(256), 0, s, V, P,
                            n, Ppad, npad, Vhi, lo);
-      hipError_t e = hipGetLastError();
-      if (e != hipSuccess) return e;
+      if ((err = hipGetLastError()) != hipSuccess) return err;
     }
-  }
-  float* partial = scratch ? scratch + planes_floats : nullptr;
-  const int S = partial ? choose_splitk(n, P, scratch_floats - planes_floats, fp32) : 1;
-  float* out = (S > 1) ? partial : W;
-  RBFParams prm{};
-  hipError_t err;
-  const float rbf_coef = float(-1.4426950408889634 / (2.0 * op.lengthscale * op.lengthscale));
-  const float rbf_scale = float(sqrt(1.4426950408889634 / (2.0 * op.lengthscale * op.lengthscale)));
-  if (op.kind == SLQ_OP_RBF && !fp32 && !(flags & kMvPointsReady)) {
-    const dim3 pgrid(unsigned((npad + 255) / 256));
-    if (exponent_slot_count(nprod, false) == 16)
-      hipLaunchKernelGGL(k_prep_points<16>, pgrid, dim3(256), 0, s, op.points, op.dim, rbf_coef,
-                         rbf_scale, n, npad, rec);
-    else
-      hipLaunchKernelGGL(k_prep_points<32>, pgrid, dim3(256), 0, s, op.points, op.dim, rbf_coef,
-                         rbf_scale, n, npad, rec);
-    err = hipGetLastError();
-    if (err != hipSuccess) return err;
-  }
-  if (ev0) (void)hipEventRecord(ev0, s);
-  if (packed) {
-    err = launch_packed(s, op.storage, static_cast<const uint8_t*>(op.packed), op.tile_scales,
-                        npad / BK, Vhi, Ppad, V, P, n, out, vec, S);
-  } else if (op.kind == SLQ_OP_DENSE) {
-    const bool v2 = vec && aligned16(op.matrix);
-    err = fp32 ? launch_f32<false, 1>(s, op.matrix, prm, V, P, n, out, v2, S)
-               : launch_bf16<false>(s, op.matrix, nullptr, prm, Vhi, Vlo, Ppad, V, P, n, out, v2,
-                                    nprod, S);
-  } else {
-    prm.X = op.points;
-    prm.dim = op.dim;
-    prm.coef = rbf_coef;
-    prm.scale = rbf_scale;
-    prm.noise = float(op.noise);
-    if (!fp32) {
+    partial = scratch + planes_floats;
+    S = choose_splitk(n, P, scratch_floats - planes_floats, false);
+    float* out = (S > 1) ? partial : W;
+    if (op.kind == SLQ_OP_RBF && !(flags & kMvPointsReady)) {
+      const dim3 pgrid(unsigned((npad + 255) / 256));
+      if (exponent_slot_count(nprod, false) == 16)
+        hipLaunchKernelGGL(k_prep_points<16>, pgrid, dim3(256), 0, s, op.points, op.dim, rbf_coef,
+                           rbf_scale, n, npad, rec);
+      else
+        hipLaunchKernelGGL(k_prep_points<32>, pgrid, dim3(256), 0, s, op.points, op.dim, rbf_coef,
+                           rbf_scale, n, npad, rec);
+      if ((err = hipGetLastError()) != hipSuccess) return err;
+    }
+    if (ev0) (void)hipEventRecord(ev0, s);
+    if (packed) {
+      err = launch_packed(s, op.storage, static_cast<const uint8_t*>(op.packed), op.tile_scales,
+                          npad / BK, Vhi, Ppad, V, P, n, out, vec, S);
+    } else if (op.kind == SLQ_OP_DENSE) {
+      err = launch_bf16<false>(s, op.matrix, nullptr, prm, Vhi, Vlo, Ppad, V, P, n, out,
+                               vec && aligned16(op.matrix), nprod, S);
+    } else {
       if (op.dim > 3) return hipErrorInvalidValue;  // rejected by the API before launch
       err = launch_bf16<true>(s, nullptr, rec, prm, Vhi, Vlo, Ppad, V, P, n, out, vec, nprod, S);
-    } else {
-      switch (op.dim) {
-        case 1: err = launch_f32<true, 1>(s, nullptr, prm, V, P, n, out, vec, S); break;
-        case 2: err = launch_f32<true, 2>(s, nullptr, prm, V, P, n, out, vec, S); break;
-        case 3: err = launch_f32<true, 3>(s, nullptr, prm, V, P, n, out, vec, S); break;
-        default: err = launch_f32<true, 4>(s, nullptr, prm, V, P, n, out, vec, S); break;
-      }
     }
   }
   if (ev1) (void)hipEventRecord(ev1, s);

@@ -51,6 +51,8 @@ struct slq_context {
   // arena mode: bytes of the buffers that were replaced by larger ones (a
   // dry run seeded with a pool's sizes: the pool frees them when it grows)
   size_t arena_replaced = 0;
+  // matvec scratch of the least size (matvec_scratch_floats)
+  bool lean = false;
   // measurement hooks: event pairs per kernel class, reused across reads
   unsigned profile_mask = 0;  // bit kc: kernel class kc is bracketed by events
   std::vector<std::pair<hipEvent_t, hipEvent_t>> events[SLQ_KC_COUNT];
@@ -256,7 +258,7 @@ int hessenberg_core(slq_context* ctx, const slq_operator& op, const float* V0, i
   const int64_t nb = num_chunks(n);
   const int pstride = int(k > 0 ? k : 1);
   float *part1, *part2, *norm2, *w, *w2, *mvs;
-  const int64_t mv_floats = matvec_scratch_floats(n, P);
+  const int64_t mv_floats = matvec_scratch_floats(op, P, ctx->lean);
   SLQ_TRY(ensure_t(ctx, ctx->splitk, size_t(mv_floats), &mvs));
   SLQ_TRY(ensure_t(ctx, ctx->partial1, size_t(P * nb * pstride), &part1));
   SLQ_TRY(ensure_t(ctx, ctx->partial2, size_t(P * nb * pstride), &part2));
@@ -277,7 +279,7 @@ int hessenberg_core(slq_context* ctx, const slq_operator& op, const float* V0, i
   SLQ_HIP(ctx, launch_normalize(s, V0, Q, P, n, norm2, nullptr, nullptr, 0, c));
   // after the first matvec (which splits its input and prepares the point
   // records) the normalisation writes the next input's BF16 planes itself
-  const PlaneOut planes = matvec_planes(op, P, mvs);
+  const PlaneOut planes = matvec_planes(op, P, mvs, mv_floats);
   MvSplitSum pend;
   for (int64_t j = 0; j < k; ++j) {
     const float* qj = Q + j * ldc;
@@ -353,7 +355,7 @@ int lanczos_core(slq_context* ctx, const slq_operator& op, const float* V0, int6
   hipStream_t s = ctx->stream;
   const int64_t nb = num_chunks(n);
   float *apart, *norm2, *w, *r, *ring, *mvs;
-  const int64_t mv_floats = matvec_scratch_floats(n, P);
+  const int64_t mv_floats = matvec_scratch_floats(op, P, ctx->lean);
   SLQ_TRY(ensure_t(ctx, ctx->splitk, size_t(mv_floats), &mvs));
   SLQ_TRY(ensure_t(ctx, ctx->partial1, size_t(P * nb), &apart));
   SLQ_TRY(ensure_t(ctx, ctx->norm2, size_t(P * nb), &norm2));
@@ -370,7 +372,7 @@ int lanczos_core(slq_context* ctx, const slq_operator& op, const float* V0, int6
   SLQ_HIP(ctx, launch_dots(s, nullptr, 0, V0, P, n, 1, norm2, 1));
   SLQ_HIP(ctx, launch_normalize(s, V0, vec(0), P, n, norm2, nullptr, nullptr, 0, c));
   const int64_t steps = k > 0 ? k : 1;
-  const PlaneOut planes = matvec_planes(op, P, mvs);
+  const PlaneOut planes = matvec_planes(op, P, mvs, mv_floats);
   MvSplitSum pend;
   for (int64_t j = 0; j < steps; ++j) {
     const float* q = vec(j);
@@ -535,7 +537,7 @@ int logdet_reverse(slq_context* ctx, const slq_operator& op, int64_t P, int64_t 
   const int64_t nb = num_chunks(n);
   float *dH, *Gam, *coef, *Lam, *lam, *lam2, *vm, *part1, *part2, *mvs;
   double* vwork = nullptr;
-  const int64_t mv_floats = matvec_scratch_floats(n, P);
+  const int64_t mv_floats = matvec_scratch_floats(op, P, ctx->lean);
   SLQ_TRY(ensure_t(ctx, ctx->splitk, size_t(mv_floats), &mvs));
   SLQ_TRY(ensure_t(ctx, ctx->partial1, size_t(P * nb * pstride), &part1));
   SLQ_TRY(ensure_t(ctx, ctx->partial2, size_t(P * nb * pstride), &part2));
@@ -619,7 +621,7 @@ int arnoldi_reverse(slq_context* ctx, const slq_operator& op, int64_t P, int64_t
   const int pstride = int(k);
   const int64_t nb = num_chunks(n);
   float *dH, *Gam, *coef, *Lam, *lam, *lam2, *vm, *part1, *part2, *mvs, *Pg, *gam;
-  const int64_t mv_floats = matvec_scratch_floats(n, P);
+  const int64_t mv_floats = matvec_scratch_floats(op, P, ctx->lean);
   SLQ_TRY(ensure_t(ctx, ctx->splitk, size_t(mv_floats), &mvs));
   SLQ_TRY(ensure_t(ctx, ctx->partial1, size_t(P * nb * pstride), &part1));
   SLQ_TRY(ensure_t(ctx, ctx->partial2, size_t(P * nb * pstride), &part2));
@@ -693,7 +695,7 @@ int lanczos_reverse(slq_context* ctx, const slq_operator& op, int64_t P, int64_t
   hipStream_t s = ctx->stream;
   const int64_t nb = num_chunks(n);
   float *db, *Lam, *xi, *W, *part1, *part2, *mvs;
-  const int64_t mv_floats = matvec_scratch_floats(n, P);
+  const int64_t mv_floats = matvec_scratch_floats(op, P, ctx->lean);
   SLQ_TRY(ensure_t(ctx, ctx->splitk, size_t(mv_floats), &mvs));
   SLQ_TRY(ensure_t(ctx, ctx->partial1, size_t(P * nb * 3), &part1));
   SLQ_TRY(ensure_t(ctx, ctx->partial2, size_t(P * nb * 3), &part2));
@@ -799,7 +801,7 @@ int logdet_lanczos_reverse(slq_context* ctx, const slq_operator& op, int64_t P, 
   const int64_t nb = num_chunks(n);
   float *dH, *Lam, *xi, *W, *part1, *part2, *mvs;
   double* vwork = nullptr;
-  const int64_t mv_floats = matvec_scratch_floats(n, P);
+  const int64_t mv_floats = matvec_scratch_floats(op, P, ctx->lean);
   SLQ_TRY(ensure_t(ctx, ctx->splitk, size_t(mv_floats), &mvs));
   SLQ_TRY(ensure_t(ctx, ctx->partial1, size_t(P * nb * 3), &part1));
   SLQ_TRY(ensure_t(ctx, ctx->partial2, size_t(P * nb * 3), &part2));
@@ -955,7 +957,7 @@ int slq_matvec(slq_context* ctx, const slq_operator* op, const float* V, int64_t
   if (!V || !W) return fail(ctx, SLQ_EINVAL, "input or output pointer is NULL");
   SLQ_TRY(set_device(ctx));
   float* mvs;
-  const int64_t mv_floats = matvec_scratch_floats(op->n, P);
+  const int64_t mv_floats = matvec_scratch_floats(*op, P, ctx->lean);
   SLQ_TRY(ensure_t(ctx, ctx->splitk, size_t(mv_floats), &mvs));
   SLQ_HIP(ctx, launch_matvec(ctx->stream, *op, V, P, W, mvs, mv_floats));
   return SLQ_OK;
@@ -1098,6 +1100,21 @@ int slq_logdet_noalloc(slq_context* ctx, const slq_operator* op, const float* Z,
   sizing.arena_size = SIZE_MAX / 2;
   ForwardState st;
   int rc = logdet_forward(&sizing, *op, Z, P, k, per_probe, mean, alpha, beta, st);
+  if (rc == SLQ_OK && sizing.arena_off > size_t(SLQ_NOALLOC_SCRATCH_BYTES)) {
+    // the least scratch: the same results
+    slq_context least;
+    least.device = ctx->device;
+    least.stream = ctx->stream;
+    least.arena_mode = true;
+    least.dry_run = true;
+    least.lean = true;
+    least.arena = base;
+    least.arena_size = SIZE_MAX / 2;
+    rc = logdet_forward(&least, *op, Z, P, k, per_probe, mean, alpha, beta, st);
+    sizing.lean = true;
+    sizing.arena_off = least.arena_off;
+    sizing.error = least.error;
+  }
   if (rc != SLQ_OK) return fail(ctx, rc, sizing.error);
   if (sizing.arena_off > size_t(SLQ_NOALLOC_SCRATCH_BYTES))
     return fail(ctx, SLQ_EINVAL,
@@ -1109,6 +1126,7 @@ int slq_logdet_noalloc(slq_context* ctx, const slq_operator* op, const float* Z,
   run.device = ctx->device;
   run.stream = ctx->stream;
   run.arena_mode = true;
+  run.lean = sizing.lean;
   run.arena = base;
   run.arena_size = size_t(SLQ_NOALLOC_SCRATCH_BYTES);
   rc = set_device(&run);
@@ -1319,7 +1337,7 @@ int slq_cg(slq_context* ctx, const slq_operator* op, const float* B, int64_t P, 
   // scalars: gamma (2 generations), atol2 (floats), iters (int64), active
   // (2 generations), the count (ints); 16 words per column plus the count
   SLQ_TRY(ensure_t(ctx, ctx->cg_scal, size_t(16 * P + 64), &scal));
-  const int64_t mv_floats = matvec_scratch_floats(n, P);
+  const int64_t mv_floats = matvec_scratch_floats(*op, P, ctx->lean);
   SLQ_TRY(ensure_t(ctx, ctx->splitk, size_t(mv_floats), &mvs));
   float *pq = parts, *rr = parts + P * nb, *rz = parts + 2 * P * nb, *bb = parts + 3 * P * nb;
   CgScalars sc;

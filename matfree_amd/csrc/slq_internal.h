@@ -48,6 +48,9 @@ __device__ __forceinline__ float ordered_sum(const float* __restrict__ v, int64_
 // ---- probes (k_probes.hip) -------------------------------------------------
 hipError_t launch_rademacher(hipStream_t s, uint32_t k0, uint32_t k1, int64_t count, float* out);
 
+// The FP32 matvec's planes hold V and -V in turns of this many 32-column tiles.
+constexpr int kPlaneSignRun = 2;
+
 // BF16 planes of the block matvec's input (tile-major, zero-padded; see
 // k_matvec.hip), written by the kernel that produces the input so that the
 // matvec can skip its own split pass (kMvPlanesReady).  hi == nullptr: the
@@ -57,6 +60,10 @@ struct PlaneOut {
   __bf16* lo = nullptr;  // null when the matvec does not read the low plane
   int64_t Ppad = 0;
   int perm = 0;  // RBF fragment order of the columns within a tile
+  // three: the FP32 matvec's planes instead (x = hi + mid + lo, `plane`
+  // elements apart, in the fragment order of k_split3_probes)
+  int three = 0;
+  int64_t plane = 0;
 };
 
 // A split-K sum left to the consumer: W = sum_{z < S} partial[z * P * n + .]
@@ -161,12 +168,14 @@ hipError_t launch_lanczos_adj_xi(hipStream_t s, const float* W, const float* lam
 
 // ---- block matvec (k_matvec.hip) -------------------------------------------
 // Largest split-K factor of the block matvec; its partial sums need up to
-// kMaxSplitK * P * n floats of scratch (split-K is off when scratch is null;
-// matvec_scratch_floats sizes it for the factor the launch will take).
+// kMaxSplitK * P * n floats of scratch (matvec_scratch_floats sizes it for
+// the factor the launch will take).
 constexpr int kMaxSplitK = 16;
-// Scratch (in floats) the block matvec can use for P vectors of length n:
-// the split-K partial sums and the BF16 hi/lo planes of the vectors.
-int64_t matvec_scratch_floats(int64_t n, int64_t P);
+// Scratch (in floats) the block matvec of op can use for P vectors: the
+// split-K partial sums and the BF16 planes of the vectors.  lean: the least
+// it works with (the FP32 matvec then splits its probes in groups, with the
+// same results).
+int64_t matvec_scratch_floats(const slq_operator& op, int64_t P, bool lean = false);
 // ev0 / ev1 (optional) are recorded on s right before and after the block
 // matvec kernel (the launches around it excluded).
 // flags: kMvPlanesReady -- the scratch planes already hold V (written by a
@@ -181,8 +190,8 @@ hipError_t launch_matvec(hipStream_t s, const slq_operator& op, const float* V, 
                          float* W, float* scratch, int64_t scratch_floats,
                          hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr, int flags = 0,
                          MvSplitSum* defer = nullptr);
-// The planes launch_matvec reads for (op, P) in scratch.
-PlaneOut matvec_planes(const slq_operator& op, int64_t P, float* scratch);
+// The planes launch_matvec reads for (op, P) in a scratch of this size.
+PlaneOut matvec_planes(const slq_operator& op, int64_t P, float* scratch, int64_t scratch_floats);
 // Packed storage of a stored matrix (slq_storage): sizes (false for FP32 or
 // an unknown storage) and the packing kernel.
 bool packed_size(int64_t n, int storage, int64_t* bytes, int64_t* scale_count);
