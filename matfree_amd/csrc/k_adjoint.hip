@@ -6,9 +6,9 @@
 //
 // Kernels:
 //  * the eigen cotangent dH comes from k_tridiag.hip (k_tridiag_vjp);
-//  * k_adjoint_coef / k_adjoint_combine: one step of the backward
-//    recursion (decomp.py:587-599) given the reductions of the streaming
-//    kernels (k_lanczos.hip).
+//  * k_adjoint_combine: one step of the backward recursion
+//    (decomp.py:587-599) given the reductions of the streaming kernels
+//    (k_lanczos.hip).
 //  * k_outer_sum: the parameter cotangents from S = sum lambda q^T -- the
 //    stored matrix's dA = S, or the RBF contractions <S, dK/dl>, <S, I> of
 //    FP32 operators (for BF16 operators the block matvec's derivative mode
@@ -22,8 +22,8 @@ namespace slq {
 namespace {
 
 // ---------------------------------------------------------------------------
-// Coefficients of one backward step idx (decomp.py:592-599), one block per
-// probe.  With s_j = q_j^T (A^T lambda) (sum of the partials over chunks):
+// Coefficients of one backward step idx (decomp.py:592-599) of probe p, formed
+// by every block that uses them.  With s_j = q_j^T (A^T lambda) (sum of the partials over chunks):
 //   Gamma[idx, j] = lower_mask[idx, j] (Pi_gamma[idx, j] - s_j), j <= idx,
 //     lower_mask = tril(1) with 1/2 on the diagonal (decomp.py:490-495),
 //     Pi_gamma = H dH^T (dQ = dc = 0, decomp.py:506), dH tridiagonal;
@@ -33,31 +33,35 @@ namespace {
 //     with gamma = dH[:, k-1] (dr = 0, decomp.py:498, 505),
 //     beta_minus = (1, H[1,0], H[2,1], ...) (decomp.py:513) and beta_plus
 //     the strict upper part of H beyond the diagonal (decomp.py:515).
-// Output per probe (stride cs = 2 k + 4): gq[0..k), gl[k..2k), and
-// (cr, cl, cv, scale) for r, lambda, A^T lambda and the final division.
+// Output in LDS: gq[0..k), gl[k..2k), and (cr, cl, cv, scale) for r, lambda,
+// A^T lambda and the final division; Gamma[idx, :] is written by the block
+// with `write`, and only entries of earlier steps are read from it.
+//
+// A launch of its own for these few sums took 3.7 to 4.3 us a step (n = 4096
+// and 8192, 32 probes); formed by every block of k_adjoint_combine they add
+// about 1 us to it.
 // ---------------------------------------------------------------------------
 //
 // General cotangents (decomp.py:497-506): Pg (P x k x k, column-major) holds
 // Pi_gamma = -dc c e_1 e_1^T + H dH^T - dQ^T Q and gam (P x k) the vector
 // gamma = dH e_K - Q^T dr; when they are null, dQ = dr = dc = 0 and dH is
 // tridiagonal (the SLQ composition) and both are formed here.
-__global__ void __launch_bounds__(256)
-    k_adjoint_coef(const float* __restrict__ H, const float* __restrict__ dH,
-                   float* __restrict__ Gam, const float* __restrict__ part, int64_t nb,
-                   int pstride, int64_t k, int64_t idx, float* __restrict__ coef,
-                   const float* __restrict__ Pg, const float* __restrict__ gam) {
-  extern __shared__ float grow[];  // Gamma[idx, 0..idx]
-  const int64_t p = blockIdx.x;
-  const float* Hp = H + p * k * k;    // column-major: H[row + col * k]
-  const float* dHp = dH + p * k * k;  // column-major
-  float* Gp = Gam + p * k * k;        // column-major
-  float* cp = coef + p * (2 * k + 4);
-  for (int64_t j = threadIdx.x; j <= idx; j += blockDim.x) {
-    float s = 0.f;
-    s = ordered_sum(part + p * nb * pstride + j, nb, pstride);
+__device__ __forceinline__ void step_coefficients(const AdjointStep& st, int64_t p, int64_t nb,
+                                                  int64_t k, bool write, float* cs) {
+  const float* Hp = st.H + p * k * k;    // column-major: H[row + col * k]
+  const float* dHp = st.dH + p * k * k;  // column-major
+  float* Gp = st.Gam + p * k * k;        // column-major
+  const int64_t idx = st.idx;
+  for (int64_t j = threadIdx.x; j < k; j += blockDim.x) {
+    if (j > idx) {
+      cs[j] = Gp[j + idx * k];  // Gamma[j, idx], set at step j
+      cs[k + j] = -Hp[idx + j * k];
+      continue;
+    }
+    const float s = ordered_sum(st.part + p * nb * st.pstride + j, nb, st.pstride);
     float pg;
-    if (Pg) {
-      pg = Pg[p * k * k + idx + j * k];
+    if (st.Pg) {
+      pg = st.Pg[p * k * k + idx + j * k];
     } else {
       pg = Hp[idx + j * k] * dHp[j + j * k];
       if (j > 0) pg += Hp[idx + (j - 1) * k] * dHp[j + (j - 1) * k];
@@ -65,51 +69,45 @@ __global__ void __launch_bounds__(256)
     }
     const float w = (j < idx) ? 1.f : 0.5f;
     const float g = w * (pg - s);
-    grow[j] = g;
-    Gp[idx + j * k] = g;
-  }
-  __syncthreads();
-  for (int64_t j = threadIdx.x; j < k; j += blockDim.x) {
-    float gq;
-    if (j < idx)
-      gq = grow[j];
-    else if (j == idx)
-      gq = 2.f * grow[j];
-    else
-      gq = Gp[j + idx * k];  // Gamma[j, idx], set at step j
-    cp[j] = gq;
-    cp[k + j] = (j > idx) ? -Hp[idx + j * k] : 0.f;
+    if (write) Gp[idx + j * k] = g;
+    cs[j] = j < idx ? g : 2.f * g;
+    cs[k + j] = 0.f;
   }
   if (threadIdx.x == 0) {
-    cp[2 * k + 0] = gam ? gam[p * k + idx] : dHp[idx + (k - 1) * k];  // gamma_idx
-    cp[2 * k + 1] = -Hp[idx + idx * k];      // -alpha_idx
-    cp[2 * k + 2] = 1.f;                     // + A^T lambda
-    cp[2 * k + 3] = 1.f / (idx == 0 ? 1.f : Hp[idx + (idx - 1) * k]);
+    cs[2 * k + 0] = st.gam ? st.gam[p * k + idx] : dHp[idx + (k - 1) * k];  // gamma_idx
+    cs[2 * k + 1] = -Hp[idx + idx * k];                                     // -alpha_idx
+    cs[2 * k + 2] = 1.f;                                                    // + A^T lambda
+    cs[2 * k + 3] = 1.f / (idx == 0 ? 1.f : Hp[idx + (idx - 1) * k]);
   }
+  __syncthreads();
 }
 
 // y = scale (cr r + cl x + cv v + d + sum_{j < ncq} gq_j Q_j + sum_{jl0 <= j < k} gl_j L_j)
-// per probe, coefficients from coef (stride 2 k + 4); r, x, v, d may be null
-// (their terms are skipped).  With save (non-null) x is also copied there.
+// per probe, coefficients from coef (stride 2 k + 4), or (STEP) those of the
+// backward step st; r, x, v, d may be null (their terms are skipped).  With save (non-null) x is also copied there.
 // V consecutive elements per thread (V = 4: 16-byte loads and stores at any
 // dword alignment, which gfx950 code issues as single dwordx4 accesses, so
 // rows of any length n stream as float4 groups, the last group of a row
 // element by element; V = 1 for small P n, where one element per thread
 // gives the launch four times the waves); the basis columns eight at a time,
 // their loads in flight together.
-template <int V>
+template <int V, bool STEP>
 __global__ void __launch_bounds__(kStreamThreads)
     k_adjoint_combine(const float* __restrict__ Q, const float* __restrict__ Lam, int64_t ldc,
                       const float* __restrict__ r, const float* __restrict__ x,
                       const float* __restrict__ v, float* __restrict__ y, float* __restrict__ save,
                       int64_t n, int64_t k, int ncq, int jl0, const float* __restrict__ coef,
-                      const float* __restrict__ d) {
+                      const float* __restrict__ d, AdjointStep st, int64_t nb) {
   extern __shared__ float cs[];
   const int64_t p = blockIdx.y;
   const int t = threadIdx.x;
-  const float* cp = coef + p * (2 * k + 4);
-  for (int64_t j = t; j < 2 * k + 4; j += blockDim.x) cs[j] = cp[j];
-  __syncthreads();
+  if constexpr (STEP) {
+    step_coefficients(st, p, nb, k, blockIdx.x == 0, cs);
+  } else {
+    const float* cp = coef + p * (2 * k + 4);
+    for (int64_t j = t; j < 2 * k + 4; j += blockDim.x) cs[j] = cp[j];
+    __syncthreads();
+  }
   const float cr = cs[2 * k], cl = cs[2 * k + 1], cv = cs[2 * k + 2], sc = cs[2 * k + 3];
   const int64_t i = (int64_t(blockIdx.x) * kStreamThreads + t) * V;
   if (i >= n) return;
@@ -204,26 +202,25 @@ __global__ void k_adjoint_init_coef(const float* __restrict__ dH, int64_t k,
   }
 }
 
-// Row i of Pi_gamma = -dc c e_1 e_1^T + H dH^T - dQ^T Q (decomp.py:506) per
-// probe: (H dH^T)[i, j] = sum_m H[i, m] dH[j, m] (both column-major), and
-// (dQ^T Q)[i, j] = dQ_i . q_j from the chunk partials of launch_dots with
-// x = dQ_i (null: dQ = 0); dc / c per probe (dc null: 0).  Pg column-major.
+// Rows i0 + blockIdx.y of Pi_gamma = -dc c e_1 e_1^T + H dH^T - dQ^T Q
+// (decomp.py:506) per probe: (H dH^T)[i, j] = sum_m H[i, m] dH[j, m] (both
+// column-major), and (dQ^T Q)[i, j] = dQ_i . q_j from the chunk partials of
+// launch_dots with x = dQ_i (null: dQ = 0); dc / c per probe (dc null: 0).  Pg
+// column-major.  All rows in one launch: a launch per row and one per row's
+// dots took 12.5 us a row at n = 4096, 32 probes, 32 rows, nearly all of it
+// latency.
 __global__ void __launch_bounds__(256)
-    k_adjoint_pigamma_row(const float* __restrict__ H, const float* __restrict__ dH,
-                          const float* __restrict__ part, int64_t nb, int pstride,
-                          const float* __restrict__ c, const float* __restrict__ dc, int64_t k,
-                          int64_t i, float* __restrict__ Pg) {
-  const int64_t p = blockIdx.x;
+    k_adjoint_pigamma(const float* __restrict__ H, const float* __restrict__ dH,
+                      const float* __restrict__ part, int64_t prow, int64_t nb, int pstride,
+                      const float* __restrict__ c, const float* __restrict__ dc, int64_t k,
+                      int64_t i0, float* __restrict__ Pg) {
+  const int64_t p = blockIdx.x, i = i0 + blockIdx.y;
   const float* Hp = H + p * k * k;
   const float* dHp = dH + p * k * k;
   for (int64_t j = threadIdx.x; j < k; j += blockDim.x) {
     float v = 0.f;
     for (int64_t m = 0; m < k; ++m) v = fmaf(Hp[i + m * k], dHp[j + m * k], v);
-    if (part) {
-      float g = 0.f;
-      g = ordered_sum(part + p * nb * pstride + j, nb, pstride);
-      v -= g;
-    }
+    if (part) v -= ordered_sum(part + blockIdx.y * prow + p * nb * pstride + j, nb, pstride);
     if (dc && i == 0 && j == 0) v -= dc[p] * c[p];
     Pg[p * k * k + i + j * k] = v;
   }
@@ -514,21 +511,12 @@ hipError_t launch_outer_rbf_contract(hipStream_t s, const float* L, const float*
   return hipGetLastError();
 }
 
-hipError_t launch_adjoint_coef(hipStream_t s, const float* H, const float* dH, float* Gam,
-                               const float* part, int pstride, int64_t P, int64_t n, int64_t k,
-                               int64_t idx, float* coef, const float* Pg, const float* gam) {
-  const size_t shmem = size_t(idx + 1) * sizeof(float);
-  hipLaunchKernelGGL(k_adjoint_coef, dim3(unsigned(P)), dim3(256), shmem, s, H, dH, Gam, part,
-                     num_chunks(n), pstride, k, idx, coef, Pg, gam);
-  return hipGetLastError();
-}
-
-hipError_t launch_adjoint_pigamma_row(hipStream_t s, const float* H, const float* dH,
-                                      const float* part, int pstride, const float* c,
-                                      const float* dc, int64_t P, int64_t n, int64_t k, int64_t i,
-                                      float* Pg) {
-  hipLaunchKernelGGL(k_adjoint_pigamma_row, dim3(unsigned(P)), dim3(256), 0, s, H, dH, part,
-                     num_chunks(n), pstride, c, dc, k, i, Pg);
+hipError_t launch_adjoint_pigamma(hipStream_t s, const float* H, const float* dH,
+                                  const float* part, int64_t prow, int pstride, const float* c,
+                                  const float* dc, int64_t P, int64_t n, int64_t k, int64_t i0,
+                                  int64_t rows, float* Pg) {
+  hipLaunchKernelGGL(k_adjoint_pigamma, dim3(unsigned(P), unsigned(rows)), dim3(256), 0, s, H, dH,
+                     part, prow, num_chunks(n), pstride, c, dc, k, i0, Pg);
   return hipGetLastError();
 }
 
@@ -539,22 +527,42 @@ hipError_t launch_adjoint_gamma_init(hipStream_t s, const float* dH, const float
   return hipGetLastError();
 }
 
+namespace {
+
+template <bool STEP>
+hipError_t launch_combine(hipStream_t s, const float* Q, const float* Lam, int64_t ldc,
+                          const float* r, const float* x, const float* v, float* y, float* save,
+                          int64_t P, int64_t n, int64_t k, int ncq, int jl0, const float* coef,
+                          const float* d, const AdjointStep& st) {
+  const bool vec = P * n >= (int64_t(1) << 20);
+  const int64_t per_block = int64_t(kStreamThreads) * (vec ? 4 : 1);
+  const dim3 grid(unsigned((n + per_block - 1) / per_block), unsigned(P));
+  const size_t shmem = size_t(2 * k + 4) * sizeof(float);
+  if (vec)
+    hipLaunchKernelGGL((k_adjoint_combine<4, STEP>), grid, dim3(kStreamThreads), shmem, s, Q, Lam,
+                       ldc, r, x, v, y, save, n, k, ncq, jl0, coef, d, st, num_chunks(n));
+  else
+    hipLaunchKernelGGL((k_adjoint_combine<1, STEP>), grid, dim3(kStreamThreads), shmem, s, Q, Lam,
+                       ldc, r, x, v, y, save, n, k, ncq, jl0, coef, d, st, num_chunks(n));
+  return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_adjoint_combine(hipStream_t s, const float* Q, const float* Lam, int64_t ldc,
                                   const float* r, const float* x, const float* v, float* y,
                                   float* save, int64_t P, int64_t n, int64_t k, int ncq, int jl0,
                                   const float* coef, const float* d) {
-  const bool vec = P * n >= (int64_t(1) << 20);
-  const int V = vec ? 4 : 1;
-  const int64_t per_block = int64_t(kStreamThreads) * V;
-  const dim3 grid(unsigned((n + per_block - 1) / per_block), unsigned(P));
-  const size_t shmem = size_t(2 * k + 4) * sizeof(float);
-  if (vec)
-    hipLaunchKernelGGL(k_adjoint_combine<4>, grid, dim3(kStreamThreads), shmem, s, Q, Lam, ldc, r,
-                       x, v, y, save, n, k, ncq, jl0, coef, d);
-  else
-    hipLaunchKernelGGL(k_adjoint_combine<1>, grid, dim3(kStreamThreads), shmem, s, Q, Lam, ldc, r,
-                       x, v, y, save, n, k, ncq, jl0, coef, d);
-  return hipGetLastError();
+  return launch_combine<false>(s, Q, Lam, ldc, r, x, v, y, save, P, n, k, ncq, jl0, coef, d,
+                               AdjointStep{});
+}
+
+hipError_t launch_adjoint_step(hipStream_t s, const float* Q, const float* Lam, int64_t ldc,
+                               const float* r, const float* x, const float* v, float* y,
+                               float* save, int64_t P, int64_t n, int64_t k,
+                               const AdjointStep& st, const float* d) {
+  return launch_combine<true>(s, Q, Lam, ldc, r, x, v, y, save, P, n, k, int(k), int(st.idx + 1),
+                              nullptr, d, st);
 }
 
 hipError_t launch_sum_fixed(hipStream_t s, const double* partial, int64_t count, int nout,

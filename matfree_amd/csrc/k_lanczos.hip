@@ -173,7 +173,8 @@ constexpr int kColBatch = 8;
 template <int V, int NC, bool SUM>
 __global__ void __launch_bounds__(kStreamThreads)
     k_dots(const float* __restrict__ Q, int64_t ldc, const float* __restrict__ x, float* xw,
-           int64_t n, int ncols, float* __restrict__ partial, int pstride, MvSplitSum sm) {
+           int64_t n, int ncols, float* __restrict__ partial, int pstride, int64_t xrow,
+           int64_t prow, MvSplitSum sm) {
   constexpr int NE = Layout<V>::NE;
   constexpr int CB = NC < kColBatch ? NC : kColBatch;
   __shared__ float red[kWaves * NC];
@@ -182,6 +183,8 @@ __global__ void __launch_bounds__(kStreamThreads)
   const int64_t nb = gridDim.x;
   const int t = threadIdx.x;
   const int64_t base = b * kChunk;
+  x += blockIdx.z * xrow;
+  partial += blockIdx.z * prow;
 
   float xv[NE][V];
   int64_t off[NE];
@@ -265,14 +268,15 @@ template <int NC, bool SUM>
 __global__ void __launch_bounds__(kStreamThreads)
     k_dots_shifted(const float* __restrict__ Q, int64_t ldc, const float* __restrict__ x,
                    float* xw, int64_t n, int ncols, float* __restrict__ partial, int pstride,
-                   MvSplitSum sm) {
+                   int64_t xrow, int64_t prow, MvSplitSum sm) {
   constexpr int NE = Layout<4>::NE;
   constexpr int CB = NC < kColBatch ? NC : kColBatch;
   __shared__ float red[kWaves * NC];
   const int64_t p = blockIdx.y, b = blockIdx.x, nb = gridDim.x;
   const int t = threadIdx.x;
   const ShiftedRow row(p, n, b, t);
-  const float* xr = x + p * n;
+  const float* xr = x + blockIdx.z * xrow + p * n;
+  partial += blockIdx.z * prow;
   float xv[NE][4];
   int64_t off[NE];
 #pragma unroll
@@ -376,17 +380,76 @@ __device__ __forceinline__ void load_coeffs(const float* __restrict__ hpart, int
   __syncthreads();
 }
 
+// BF16 hi / lo planes of V elements i .. i + V - 1 of probe p, in the layout
+// of the block matvec's split pass (k_matvec.hip: tile-major, 32 columns per
+// tile and probe; RBF tiles with column groups of four ordered as the MFMA
+// fragments expect): hi = bf16(x), lo = bf16(x - hi), round to nearest.
+__device__ __forceinline__ int plane_group(int c4, int perm) {
+  return perm ? ((c4 & 4) | ((c4 & 1) << 1) | ((c4 & 2) >> 1)) : c4;
+}
+
+template <int V>
+__device__ __forceinline__ void store_planes(const PlaneOut& pl, int64_t p, int64_t i,
+                                             const float (&v)[V]) {
+  if (pl.three) {
+    // the FP32 matvec's planes: 8 columns of a probe per 16-byte word
+    // (k_split3_probes); i % V == 0, so a group lies in one word
+    const int64_t word = (((i / 32) * (pl.Ppad / 32) + p / 32) * 2 + ((i >> 4) & 1)) * 64 +
+                         (p & 31) + 32 * ((i >> 3) & 1);
+    __bf16* dst = pl.hi + word * 8 + (i & 7);
+    struct __attribute__((aligned(2 * V))) Group {
+      __bf16 b[V];
+    } q[3];
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      // every second run of tiles holds -V (k_matvec_f32)
+      const float x = (i / (32 * kPlaneSignRun)) & 1 ? -v[u] : v[u];
+      q[0].b[u] = __bf16(x);
+      const float r = x - float(q[0].b[u]);
+      q[1].b[u] = __bf16(r);
+      q[2].b[u] = __bf16(r - float(q[1].b[u]));
+    }
+#pragma unroll
+    for (int w = 0; w < 3; ++w) *reinterpret_cast<Group*>(dst + w * pl.plane) = q[w];
+    return;
+  }
+  if constexpr (V == 4) {  // i % 4 == 0: one group of four, one 8-byte store per plane
+    const int64_t dst = ((i / 32) * pl.Ppad + p) * 32 + 4 * plane_group(int((i % 32) / 4), pl.perm);
+    __bf16 h[4], l[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      h[u] = __bf16(v[u]);
+      l[u] = __bf16(v[u] - float(h[u]));
+    }
+    *reinterpret_cast<uint2*>(pl.hi + dst) = __builtin_bit_cast(uint2, h);
+    if (pl.lo) *reinterpret_cast<uint2*>(pl.lo + dst) = __builtin_bit_cast(uint2, l);
+  } else {
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      const int64_t m = i + u;
+      const int64_t dst =
+          ((m / 32) * pl.Ppad + p) * 32 + 4 * plane_group(int((m % 32) / 4), pl.perm) + (m % 4);
+      const __bf16 h = __bf16(v[u]);
+      pl.hi[dst] = h;
+      if (pl.lo) pl.lo[dst] = __bf16(v[u] - float(h));
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // project: y = x - Q h (h from partials); optional norm^2 partials of y.
 // Columns in batches of kColBatch loaded together, the last ncols % kColBatch
-// in batches of 4, 2 and 1 (no column is read twice).
+// in batches of 4, 2 and 1 (no column is read twice).  pl (V = 4): the planes
+// of y for the matvec that follows, which saves its split launch (3.3 us at
+// n = 8192, 32 probes).
 // ---------------------------------------------------------------------------
 template <int V>
 __global__ void __launch_bounds__(kStreamThreads)
     k_project(const float* __restrict__ Q, int64_t ldc, const float* __restrict__ x,
               float* __restrict__ y, int64_t n, int ncols, const float* __restrict__ hpart,
               int pstride, float* __restrict__ norm2part, float* __restrict__ hout,
-              int64_t hout_stride, const float* __restrict__ hsub, int64_t hsub_stride) {
+              int64_t hout_stride, const float* __restrict__ hsub, int64_t hsub_stride,
+              PlaneOut pl) {
   constexpr int NE = Layout<V>::NE;
   extern __shared__ float hs[];
   __shared__ float red[kWaves];
@@ -444,6 +507,8 @@ __global__ void __launch_bounds__(kStreamThreads)
         acc = fmaf(xv[v], xv[v], acc);
       }
       VecIO<V>::store(y + p * n + i, xv);
+      if constexpr (V == 4)
+        if (pl.hi) store_planes<V>(pl, p, i, xv);
     }
   }
   if (norm2part) {
@@ -677,62 +742,6 @@ __global__ void __launch_bounds__(kStreamThreads)
   }
 }
 
-// BF16 hi / lo planes of V elements i .. i + V - 1 of probe p, in the layout
-// of the block matvec's split pass (k_matvec.hip: tile-major, 32 columns per
-// tile and probe; RBF tiles with column groups of four ordered as the MFMA
-// fragments expect): hi = bf16(x), lo = bf16(x - hi), round to nearest.
-__device__ __forceinline__ int plane_group(int c4, int perm) {
-  return perm ? ((c4 & 4) | ((c4 & 1) << 1) | ((c4 & 2) >> 1)) : c4;
-}
-
-template <int V>
-__device__ __forceinline__ void store_planes(const PlaneOut& pl, int64_t p, int64_t i,
-                                             const float (&v)[V]) {
-  if (pl.three) {
-    // the FP32 matvec's planes: 8 columns of a probe per 16-byte word
-    // (k_split3_probes); i % V == 0, so a group lies in one word
-    const int64_t word = (((i / 32) * (pl.Ppad / 32) + p / 32) * 2 + ((i >> 4) & 1)) * 64 +
-                         (p & 31) + 32 * ((i >> 3) & 1);
-    __bf16* dst = pl.hi + word * 8 + (i & 7);
-    struct __attribute__((aligned(2 * V))) Group {
-      __bf16 b[V];
-    } q[3];
-#pragma unroll
-    for (int u = 0; u < V; ++u) {
-      // every second run of tiles holds -V (k_matvec_f32)
-      const float x = (i / (32 * kPlaneSignRun)) & 1 ? -v[u] : v[u];
-      q[0].b[u] = __bf16(x);
-      const float r = x - float(q[0].b[u]);
-      q[1].b[u] = __bf16(r);
-      q[2].b[u] = __bf16(r - float(q[1].b[u]));
-    }
-#pragma unroll
-    for (int w = 0; w < 3; ++w) *reinterpret_cast<Group*>(dst + w * pl.plane) = q[w];
-    return;
-  }
-  if constexpr (V == 4) {  // i % 4 == 0: one group of four, one 8-byte store per plane
-    const int64_t dst = ((i / 32) * pl.Ppad + p) * 32 + 4 * plane_group(int((i % 32) / 4), pl.perm);
-    __bf16 h[4], l[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      h[u] = __bf16(v[u]);
-      l[u] = __bf16(v[u] - float(h[u]));
-    }
-    *reinterpret_cast<uint2*>(pl.hi + dst) = __builtin_bit_cast(uint2, h);
-    if (pl.lo) *reinterpret_cast<uint2*>(pl.lo + dst) = __builtin_bit_cast(uint2, l);
-  } else {
-#pragma unroll
-    for (int u = 0; u < V; ++u) {
-      const int64_t m = i + u;
-      const int64_t dst =
-          ((m / 32) * pl.Ppad + p) * 32 + 4 * plane_group(int((m % 32) / 4), pl.perm) + (m % 4);
-      const __bf16 h = __bf16(v[u]);
-      pl.hi[dst] = h;
-      if (pl.lo) pl.lo[dst] = __bf16(v[u] - float(h));
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
 // normalize: out = x / sqrt(sum_b norm2part), plus bookkeeping of the norm
 // ---------------------------------------------------------------------------
@@ -801,29 +810,32 @@ inline int stream_width(int64_t n, int64_t ld, std::initializer_list<const void*
 
 template <int V>
 hipError_t launch_dots_v(hipStream_t s, const float* Q, int64_t ldc, const float* x, int64_t P,
-                         int64_t n, int ncols, float* partial, int pstride) {
-  const dim3 grid(unsigned(num_chunks(n)), unsigned(P));
+                         int64_t n, int ncols, float* partial, int pstride, int64_t rows,
+                         int64_t xrow, int64_t prow) {
+  const dim3 grid(unsigned(num_chunks(n)), unsigned(P), unsigned(rows));
   const dim3 block(kStreamThreads);
   const MvSplitSum sm;
   if (ncols <= 8)
     hipLaunchKernelGGL((k_dots<V, 8, false>), grid, block, 0, s, Q, ldc, x, nullptr, n, ncols,
-                       partial, pstride, sm);
+                       partial, pstride, xrow, prow, sm);
   else if (ncols <= 16)
     hipLaunchKernelGGL((k_dots<V, 16, false>), grid, block, 0, s, Q, ldc, x, nullptr, n, ncols,
-                       partial, pstride, sm);
+                       partial, pstride, xrow, prow, sm);
   else if (ncols <= 32)
     hipLaunchKernelGGL((k_dots<V, 32, false>), grid, block, 0, s, Q, ldc, x, nullptr, n, ncols,
-                       partial, pstride, sm);
+                       partial, pstride, xrow, prow, sm);
   else
     hipLaunchKernelGGL((k_dots<V, 64, false>), grid, block, 0, s, Q, ldc, x, nullptr, n, ncols,
-                       partial, pstride, sm);
+                       partial, pstride, xrow, prow, sm);
   return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t launch_dots(hipStream_t s, const float* Q, int64_t ldc, const float* x, int64_t P,
-                       int64_t n, int ncols, float* partial, int pstride) {
+                       int64_t n, int ncols, float* partial, int pstride, int64_t rows,
+                       int64_t xrow, int64_t prow) {
+  if (rows > 1 && xrow % 4 != 0) return hipErrorInvalidValue;  // one alignment for all rows
   const int V = Q ? stream_width(n, ldc, {x, Q}) : stream_width(n, n, {x});
   if (Q == nullptr) {
     const dim3 grid(unsigned(num_chunks(n)), unsigned(P));
@@ -835,26 +847,28 @@ hipError_t launch_dots(hipStream_t s, const float* Q, int64_t ldc, const float* 
       hipLaunchKernelGGL(k_sumsq<1>, grid, dim3(kStreamThreads), 0, s, x, n, partial);
     return hipGetLastError();
   }
-  if (V == 4) return launch_dots_v<4>(s, Q, ldc, x, P, n, ncols, partial, pstride);
+  if (V == 4)
+    return launch_dots_v<4>(s, Q, ldc, x, P, n, ncols, partial, pstride, rows, xrow, prow);
   if (shifted_ok(n, ldc, {x, Q})) {  // measured faster than the float2 kernels for even n
-    const dim3 grid(unsigned(num_chunks(n)), unsigned(P));
+    const dim3 grid(unsigned(num_chunks(n)), unsigned(P), unsigned(rows));
     const dim3 block(kStreamThreads);
     if (ncols <= 8)
       hipLaunchKernelGGL((k_dots_shifted<8, false>), grid, block, 0, s, Q, ldc, x, nullptr, n,
-                         ncols, partial, pstride, MvSplitSum{});
+                         ncols, partial, pstride, xrow, prow, MvSplitSum{});
     else if (ncols <= 16)
       hipLaunchKernelGGL((k_dots_shifted<16, false>), grid, block, 0, s, Q, ldc, x, nullptr, n,
-                         ncols, partial, pstride, MvSplitSum{});
+                         ncols, partial, pstride, xrow, prow, MvSplitSum{});
     else if (ncols <= 32)
       hipLaunchKernelGGL((k_dots_shifted<32, false>), grid, block, 0, s, Q, ldc, x, nullptr, n,
-                         ncols, partial, pstride, MvSplitSum{});
+                         ncols, partial, pstride, xrow, prow, MvSplitSum{});
     else
       hipLaunchKernelGGL((k_dots_shifted<64, false>), grid, block, 0, s, Q, ldc, x, nullptr, n,
-                         ncols, partial, pstride, MvSplitSum{});
+                         ncols, partial, pstride, xrow, prow, MvSplitSum{});
     return hipGetLastError();
   }
-  if (V == 2) return launch_dots_v<2>(s, Q, ldc, x, P, n, ncols, partial, pstride);
-  return launch_dots_v<1>(s, Q, ldc, x, P, n, ncols, partial, pstride);
+  if (V == 2)
+    return launch_dots_v<2>(s, Q, ldc, x, P, n, ncols, partial, pstride, rows, xrow, prow);
+  return launch_dots_v<1>(s, Q, ldc, x, P, n, ncols, partial, pstride, rows, xrow, prow);
 }
 
 hipError_t launch_dots_sum(hipStream_t s, const float* Q, int64_t ldc, const MvSplitSum& sum,
@@ -865,10 +879,10 @@ hipError_t launch_dots_sum(hipStream_t s, const float* Q, int64_t ldc, const MvS
   const int V = stream_width(n, ldc, ptrs);
 #define SLQ_DS(VV, NC)                                                                          \
   hipLaunchKernelGGL((k_dots<VV, NC, true>), grid, block, 0, s, Q, ldc, nullptr, x, n, ncols, \
-                     partial, pstride, sum)
+                     partial, pstride, 0, 0, sum)
 #define SLQ_DSH(NC)                                                                          \
   hipLaunchKernelGGL((k_dots_shifted<NC, true>), grid, block, 0, s, Q, ldc, nullptr, x, n, \
-                     ncols, partial, pstride, sum)
+                     ncols, partial, pstride, 0, 0, sum)
 #define SLQ_DS_NC(M)         \
   if (ncols <= 8) M(8);      \
   else if (ncols <= 16) M(16); \
@@ -898,22 +912,24 @@ hipError_t launch_dots_sum(hipStream_t s, const float* Q, int64_t ldc, const MvS
 hipError_t launch_project(hipStream_t s, const float* Q, int64_t ldc, const float* x, float* y,
                           int64_t P, int64_t n, int ncols, const float* hpart, int pstride,
                           float* norm2part, float* hout, int64_t hout_stride, const float* hsub,
-                          int64_t hsub_stride) {
+                          int64_t hsub_stride, const PlaneOut* planes) {
   const dim3 grid(unsigned(num_chunks(n)), unsigned(P));
   const size_t shmem = size_t(ncols > 0 ? ncols : 1) * sizeof(float);
   const int V = stream_width(n, ldc, {x, y, Q});
+  if (planes && V != 4) return hipErrorInvalidValue;
+  const PlaneOut pl = planes ? *planes : PlaneOut{};
   if (V == 4)
     hipLaunchKernelGGL(k_project<4>, grid, dim3(kStreamThreads), shmem, s, Q, ldc, x, y, n, ncols,
-                       hpart, pstride, norm2part, hout, hout_stride, hsub, hsub_stride);
+                       hpart, pstride, norm2part, hout, hout_stride, hsub, hsub_stride, pl);
   else if (shifted_ok(n, ldc, {x, y, Q}))  // measured faster than the float2 kernel for even n
     hipLaunchKernelGGL(k_project_shifted, grid, dim3(kStreamThreads), shmem, s, Q, ldc, x, y, n,
                        ncols, hpart, pstride, norm2part, hout, hout_stride, hsub, hsub_stride);
   else if (V == 2)
     hipLaunchKernelGGL(k_project<2>, grid, dim3(kStreamThreads), shmem, s, Q, ldc, x, y, n, ncols,
-                       hpart, pstride, norm2part, hout, hout_stride, hsub, hsub_stride);
+                       hpart, pstride, norm2part, hout, hout_stride, hsub, hsub_stride, pl);
   else
     hipLaunchKernelGGL(k_project<1>, grid, dim3(kStreamThreads), shmem, s, Q, ldc, x, y, n, ncols,
-                       hpart, pstride, norm2part, hout, hout_stride, hsub, hsub_stride);
+                       hpart, pstride, norm2part, hout, hout_stride, hsub, hsub_stride, pl);
   return hipGetLastError();
 }
 

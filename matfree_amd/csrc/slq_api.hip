@@ -526,6 +526,42 @@ int rbf_param_contract(slq_context* ctx, const slq_operator& op, const float* L,
   return SLQ_OK;
 }
 
+// The operator products of a reverse scan.  After the first, the point records
+// in the scratch are reused and the input's planes are written by the
+// projection that forms it (rows of whole float4 groups); a split-K sum is
+// left to the dots that read it.  Without these, the small launches around the
+// product took 12 us of a step at n = 8192, 32 probes.
+struct AdjointMatvec {
+  const slq_operator& op;
+  int64_t P;
+  float* mvs;
+  int64_t mv_floats;
+  PlaneOut planes;
+  bool first = true;
+  AdjointMatvec(const slq_operator& o, int64_t probes, float* scratch, int64_t floats)
+      : op(o), P(probes), mvs(scratch), mv_floats(floats),
+        planes(matvec_planes(o, probes, scratch, floats)) {}
+  // where the producer of the next input puts its planes (null: not at all)
+  const PlaneOut* planes_out() const {
+    return !first && planes.hi && op.n % 4 == 0 ? &planes : nullptr;
+  }
+  // w = A x and the chunk partials of its dots with ncols columns of Q;
+  // projected: x was formed with planes_out()
+  hipError_t run(hipStream_t s, const float* x, float* w, const float* Q, int64_t ldc, int ncols,
+                 float* part, int pstride, bool projected) {
+    int flags = first ? 0 : kMvPointsReady;
+    if (projected && planes_out()) flags |= kMvPlanesReady;
+    first = false;
+    MvSplitSum pend;
+    const hipError_t e =
+        launch_matvec(s, op, x, P, w, mvs, mv_floats, nullptr, nullptr, flags, &pend);
+    if (e != hipSuccess) return e;
+    if (pend.partial)
+      return launch_dots_sum(s, Q, ldc, pend, w, P, op.n, ncols, part, pstride);
+    return launch_dots(s, Q, ldc, w, P, op.n, ncols, part, pstride);
+  }
+};
+
 // The reverse pass: cotangent of the probe mean w.r.t. H (eigh VJP), the
 // Arnoldi adjoint recursion (decomp.py:480-600, reortho="full"), and the
 // operator parameters' cotangents (the matvec VJPs of decomp.py:587-589).
@@ -561,20 +597,20 @@ int logdet_reverse(slq_context* ctx, const slq_operator& op, int64_t P, int64_t 
   SLQ_HIP(ctx, launch_adjoint_combine(s, st.Q, nullptr, ldc, nullptr, nullptr, nullptr, lam,
                                       nullptr, P, n, k, int(k), int(k), coef));
   // reverse scan (decomp.py:538, 575-599)
+  AdjointMatvec mv(op, P, mvs, mv_floats);
   for (int64_t idx = k - 1; idx >= 0; --idx) {
     // lambda -= Q_m (Q_m^T lambda - dH[:, idx]_m), columns j <= idx + 1 (decomp.py:576-584)
     const int ncols = int(idx + 2 < k ? idx + 2 : k);
     SLQ_HIP(ctx, launch_dots(s, st.Q, ldc, lam, P, n, ncols, part1, pstride));
     SLQ_HIP(ctx, launch_project(s, st.Q, ldc, lam, lam2, P, n, ncols, part1, pstride, nullptr,
-                                nullptr, 0, dH + idx * k, k * k));
-    // A^T lambda (decomp.py:587-588; A symmetric)
-    SLQ_HIP(ctx, launch_matvec(s, op, lam2, P, vm, mvs, mv_floats));
-    // Q^T (A^T lambda) for Gamma[idx, :] (decomp.py:592-593)
-    SLQ_HIP(ctx, launch_dots(s, st.Q, ldc, vm, P, n, int(idx + 1), part2, pstride));
-    SLQ_HIP(ctx, launch_adjoint_coef(s, st.H, dH, Gam, part2, pstride, P, n, k, idx, coef));
+                                nullptr, 0, dH + idx * k, k * k, mv.planes_out()));
+    // A^T lambda (decomp.py:587-588; A symmetric) and Q^T (A^T lambda) for
+    // Gamma[idx, :] (decomp.py:592-593)
+    SLQ_HIP(ctx, mv.run(s, lam2, vm, st.Q, ldc, int(idx + 1), part2, pstride, true));
     // Lambda[:, idx] = lambda and the next lambda (decomp.py:596-599)
-    SLQ_HIP(ctx, launch_adjoint_combine(s, st.Q, Lam, ldc, st.R, lam2, vm, lam, Lam + idx * ldc,
-                                        P, n, k, int(k), int(idx + 1), coef));
+    const AdjointStep step{st.H, dH, Gam, part2, pstride, idx};
+    SLQ_HIP(ctx, launch_adjoint_step(s, st.Q, Lam, ldc, st.R, lam2, vm, lam, Lam + idx * ldc, P, n,
+                                     k, step));
   }
 
   // parameter cotangents: sum over steps and probes of the matvec VJPs
@@ -641,11 +677,19 @@ int arnoldi_reverse(slq_context* ctx, const slq_operator& op, int64_t P, int64_t
   else
     SLQ_HIP(ctx, launch_fill_zero(s, dH, P * k * k));
   SLQ_HIP(ctx, launch_fill_zero(s, Gam, P * k * k));
-  // Pi_gamma = -dc c e_1 e_1^T + H dH^T - dQ^T Q, row by row (decomp.py:506)
-  for (int64_t i = 0; i < k; ++i) {
-    if (dQ) SLQ_HIP(ctx, launch_dots(s, st.Q, ldc, dQ + i * ldq, P, n, int(k), part1, pstride));
-    SLQ_HIP(ctx, launch_adjoint_pigamma_row(s, st.H, dH, dQ ? part1 : nullptr, pstride, st.c, dc,
-                                            P, n, k, i, Pg));
+  // Pi_gamma = -dc c e_1 e_1^T + H dH^T - dQ^T Q (decomp.py:506), as many rows
+  // at a time as the partial dots dQ_i^T Q fit in Lambda's place (not yet in
+  // use) and a grid takes; one if the rows of dQ differ in alignment
+  const int64_t prow = P * nb * pstride;
+  const int64_t fit = std::min<int64_t>(std::min<int64_t>(k * ldc / prow, k), 65535);
+  const int64_t group = ldq % 4 == 0 || !dQ ? fit : 1;
+  for (int64_t i = 0; i < k; i += group) {
+    const int64_t rows = std::min(group, k - i);
+    if (dQ)
+      SLQ_HIP(ctx, launch_dots(s, st.Q, ldc, dQ + i * ldq, P, n, int(k), Lam, pstride, rows, ldq,
+                               prow));
+    SLQ_HIP(ctx, launch_adjoint_pigamma(s, st.H, dH, dQ ? Lam : nullptr, prow, pstride, st.c, dc,
+                                        P, n, k, i, rows, Pg));
   }
   // gamma = dH e_K - Q^T dr; lambda = dr + Q gamma (decomp.py:498-499)
   if (dr) SLQ_HIP(ctx, launch_dots(s, st.Q, ldc, dr, P, n, int(k), part1, pstride));
@@ -654,6 +698,7 @@ int arnoldi_reverse(slq_context* ctx, const slq_operator& op, int64_t P, int64_t
   SLQ_HIP(ctx, launch_adjoint_combine(s, st.Q, nullptr, ldc, nullptr, dr, nullptr, lam, nullptr,
                                       P, n, k, int(k), int(k), coef));
   // reverse scan (decomp.py:538, 575-599)
+  AdjointMatvec mv(op, P, mvs, mv_floats);
   for (int64_t idx = k - 1; idx >= 0; --idx) {
     const float* lin = lam;
     if (adj_reortho) {
@@ -661,20 +706,18 @@ int arnoldi_reverse(slq_context* ctx, const slq_operator& op, int64_t P, int64_t
       const int ncols = int(idx + 2 < k ? idx + 2 : k);
       SLQ_HIP(ctx, launch_dots(s, st.Q, ldc, lam, P, n, ncols, part1, pstride));
       SLQ_HIP(ctx, launch_project(s, st.Q, ldc, lam, lam2, P, n, ncols, part1, pstride, nullptr,
-                                  nullptr, 0, dH + idx * k, k * k));
+                                  nullptr, 0, dH + idx * k, k * k, mv.planes_out()));
       lin = lam2;
     }
-    // A^T lambda (decomp.py:587-588; A symmetric)
-    SLQ_HIP(ctx, launch_matvec(s, op, lin, P, vm, mvs, mv_floats));
-    // Q^T (A^T lambda) for Gamma[idx, :] (decomp.py:592-593)
-    SLQ_HIP(ctx, launch_dots(s, st.Q, ldc, vm, P, n, int(idx + 1), part2, pstride));
-    SLQ_HIP(ctx, launch_adjoint_coef(s, st.H, dH, Gam, part2, pstride, P, n, k, idx, coef, Pg,
-                                     gam));
+    // A^T lambda (decomp.py:587-588; A symmetric) and Q^T (A^T lambda) for
+    // Gamma[idx, :] (decomp.py:592-593)
+    SLQ_HIP(ctx, mv.run(s, lin, vm, st.Q, ldc, int(idx + 1), part2, pstride, adj_reortho));
     // Lambda[:, idx] = lambda and the next lambda, with Pi_xi[idx] = dQ_idx +
     // gamma_idx r (decomp.py:505, 596-599)
-    SLQ_HIP(ctx, launch_adjoint_combine(s, st.Q, Lam, ldc, st.R, lin, vm, adj_reortho ? lam : lam2,
-                                        Lam + idx * ldc, P, n, k, int(k), int(idx + 1), coef,
-                                        dQ ? dQ + idx * ldq : nullptr));
+    const AdjointStep step{st.H, dH, Gam, part2, pstride, idx, Pg, gam};
+    SLQ_HIP(ctx, launch_adjoint_step(s, st.Q, Lam, ldc, st.R, lin, vm, adj_reortho ? lam : lam2,
+                                     Lam + idx * ldc, P, n, k, step,
+                                     dQ ? dQ + idx * ldq : nullptr));
     if (!adj_reortho) std::swap(lam, lam2);
   }
   // dv = lambda c (decomp.py:602)
@@ -744,7 +787,8 @@ int lanczos_reverse(slq_context* ctx, const slq_operator& op, int64_t P, int64_t
     float* lam = Lam + i * ldc;
     SLQ_HIP(ctx, launch_lanczos_adj_lambda(s, xi, x, xplus, P, n, sc, lam));
     // A lambda (decomp.py:337; the operator is symmetric)
-    SLQ_HIP(ctx, launch_matvec(s, op, lam, P, W, mvs, mv_floats));
+    SLQ_HIP(ctx, launch_matvec(s, op, lam, P, W, mvs, mv_floats, nullptr, nullptr,
+                               last ? 0 : kMvPointsReady));
     // xi for step i - 1 (decomp.py:341) and that step's dots
     SLQ_HIP(ctx, launch_lanczos_adj_xi(s, W, lam, last ? nullptr : Lam + (i + 1) * ldc, xplus,
                                        last, i > 0 ? st.Q + (i - 1) * ldc : x, x, P, n, sc, xi,
@@ -842,7 +886,8 @@ int logdet_lanczos_reverse(slq_context* ctx, const slq_operator& op, int64_t P, 
                                            last ? nullptr : st.Q + (i + 1) * ldc, P, n, sc, lam));
     if (i == 0) break;
     // A lambda (decomp.py:337; the operator is symmetric)
-    SLQ_HIP(ctx, launch_matvec(s, op, lam, P, W, mvs, mv_floats));
+    SLQ_HIP(ctx, launch_matvec(s, op, lam, P, W, mvs, mv_floats, nullptr, nullptr,
+                               last ? 0 : kMvPointsReady));
     // xi for step i - 1 (decomp.py:341) and that step's dots
     SLQ_HIP(ctx, launch_lanczos_adj_xi(s, W, lam, last ? nullptr : Lam + (i + 1) * ldc,
                                        last ? st.R : st.Q + (i + 1) * ldc, last,

@@ -81,8 +81,10 @@ struct MvSplitSum {
 // Basis column c of probe p starts at Q + c * ldc + p * n (ldc >= P * n).
 // partial[p][b][c] = sum_{i in chunk b} Q[c][p][i] * x[p][i], c < ncols.
 // Q may be null with ncols = 1 to mean "sum of squares of x" (partial[p][b][0]).
+// rows: the same for that many blocks x + i * xrow, into partial + i * prow.
 hipError_t launch_dots(hipStream_t s, const float* Q, int64_t ldc, const float* x, int64_t P,
-                       int64_t n, int ncols, float* partial, int pstride);
+                       int64_t n, int ncols, float* partial, int pstride, int64_t rows = 1,
+                       int64_t xrow = 0, int64_t prow = 0);
 // launch_dots of x = the split-K sum `sum` (a deferred launch_matvec result),
 // which is also written to x (Q non-null), any ncols.
 hipError_t launch_dots_sum(hipStream_t s, const float* Q, int64_t ldc, const MvSplitSum& sum,
@@ -90,11 +92,13 @@ hipError_t launch_dots_sum(hipStream_t s, const float* Q, int64_t ldc, const MvS
 // y = x - sum_c Q[c] h[c] with h[c] = sum_b hpart[p][b][c] - hsub[p][c];
 // optional norm2part[p][b] = sum over chunk of y^2.  hout (if non-null)
 // receives sum_b hpart[p][b][c] at hout + p * hout_stride (written by chunk 0
-// only); hsub (if non-null) is read at hsub + p * hsub_stride.
+// only); hsub (if non-null) is read at hsub + p * hsub_stride; planes (if
+// non-null, n % 4 == 0 and 16-byte aligned operands) receives y's planes.
 hipError_t launch_project(hipStream_t s, const float* Q, int64_t ldc, const float* x, float* y,
                           int64_t P, int64_t n, int ncols, const float* hpart, int pstride,
                           float* norm2part, float* hout, int64_t hout_stride,
-                          const float* hsub = nullptr, int64_t hsub_stride = 0);
+                          const float* hsub = nullptr, int64_t hsub_stride = 0,
+                          const PlaneOut* planes = nullptr);
 // Fused: y = x - Q h1 (h1 reduced from h1part), then h2part = Q^T y per chunk.
 hipError_t launch_project_dots(hipStream_t s, const float* Q, int64_t ldc, const float* x,
                                float* y, int64_t P, int64_t n, int ncols, const float* h1part,
@@ -227,22 +231,28 @@ hipError_t launch_mean_and_sem(hipStream_t s, const double* v, int64_t P, double
                                double* sem);
 
 // ---- reverse pass (k_adjoint.hip) ------------------------------------------
-// One backward step idx: Gamma row idx and the combination coefficients
-// (coef, per probe 2 k + 4 floats) from the chunk partials of Q^T (A^T lambda).
-// Pg / gam (optional): Pi_gamma and gamma of general cotangents (see
-// launch_adjoint_pigamma_row / launch_adjoint_gamma_init); null: the SLQ
-// composition's dQ = dr = dc = 0 with a tridiagonal dH.
-hipError_t launch_adjoint_coef(hipStream_t s, const float* H, const float* dH, float* Gam,
-                               const float* part, int pstride, int64_t P, int64_t n, int64_t k,
-                               int64_t idx, float* coef, const float* Pg = nullptr,
-                               const float* gam = nullptr);
-// Row i of Pi_gamma = -dc c e_1 e_1^T + H dH^T - dQ^T Q per probe (P x k x k,
-// column-major) from the chunk partials of Q^T dQ_i (part, null: dQ = 0);
-// c, dc per probe (dc null: 0).
-hipError_t launch_adjoint_pigamma_row(hipStream_t s, const float* H, const float* dH,
-                                      const float* part, int pstride, const float* c,
-                                      const float* dc, int64_t P, int64_t n, int64_t k, int64_t i,
-                                      float* Pg);
+// One backward step idx: the combination coefficients and Gamma row idx from
+// the chunk partials of Q^T (A^T lambda).  Pg / gam (optional): Pi_gamma and
+// gamma of general cotangents (see launch_adjoint_pigamma /
+// launch_adjoint_gamma_init); null: the SLQ composition's dQ = dr = dc = 0
+// with a tridiagonal dH.
+struct AdjointStep {
+  const float *H, *dH;
+  float* Gam;
+  const float* part;
+  int pstride;
+  int64_t idx;
+  const float* Pg = nullptr;
+  const float* gam = nullptr;
+};
+// Rows i0 .. i0 + rows - 1 of Pi_gamma = -dc c e_1 e_1^T + H dH^T - dQ^T Q per
+// probe (P x k x k, column-major) from the chunk partials of Q^T dQ_i (part,
+// one row's prow floats after the other's; null: dQ = 0); c, dc per probe (dc
+// null: 0).
+hipError_t launch_adjoint_pigamma(hipStream_t s, const float* H, const float* dH,
+                                  const float* part, int64_t prow, int pstride, const float* c,
+                                  const float* dc, int64_t P, int64_t n, int64_t k, int64_t i0,
+                                  int64_t rows, float* Pg);
 // gamma = dH e_K - Q^T dr (part: chunk partials of Q^T dr, null: dr = 0) into
 // gam (P x k) and the coefficients of lambda = dr + Q gamma (x = dr).
 hipError_t launch_adjoint_gamma_init(hipStream_t s, const float* dH, const float* part, int pstride,
@@ -251,11 +261,18 @@ hipError_t launch_adjoint_gamma_init(hipStream_t s, const float* dH, const float
 hipError_t launch_adjoint_init_coef(hipStream_t s, const float* dH, int64_t P, int64_t k,
                                     float* coef);
 // y = scale (cr r + cl x + cv v + d + sum_{j < ncq} gq_j Q_j + sum_{jl0 <= j < k} gl_j Lam_j),
-// per probe (coef layout above); r, x, v, d may be null; save (if given) receives x.
+// per probe, gq = coef[0, k), gl = coef[k, 2k), (cr, cl, cv, scale) after them;
+// r, x, v, d may be null; save (if given) receives x.
 hipError_t launch_adjoint_combine(hipStream_t s, const float* Q, const float* Lam, int64_t ldc,
                                   const float* r, const float* x, const float* v, float* y,
                                   float* save, int64_t P, int64_t n, int64_t k, int ncq, int jl0,
                                   const float* coef, const float* d = nullptr);
+// The same with the coefficients of a backward step (x = lambda, v = A^T
+// lambda), ncq = k and jl0 = idx + 1; row idx of Gamma is written.
+hipError_t launch_adjoint_step(hipStream_t s, const float* Q, const float* Lam, int64_t ldc,
+                               const float* r, const float* x, const float* v, float* y,
+                               float* save, int64_t P, int64_t n, int64_t k,
+                               const AdjointStep& st, const float* d = nullptr);
 // out (n x n, row-major) = sum_{c < K} L_c R_c^T over columns c = (idx, p) at
 // base + idx * ldc + p * n (K = k P), FP32 MFMA.
 hipError_t launch_outer_sum(hipStream_t s, const float* L, const float* R, int64_t ldc, int64_t P,
