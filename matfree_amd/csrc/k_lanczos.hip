@@ -21,6 +21,7 @@
 //
 // Plain Lanczos (reortho="none", decomp.py:198-266) uses the single-column
 // dots, k_three_term and k_normalize: no basis is read.
+#include <algorithm>
 #include <initializer_list>
 #include <type_traits>
 
@@ -136,30 +137,46 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 // dots: partial[p][b][c] = sum over chunk b of Q[c][p][:] . x[p][:]
 // Columns in batches of NC (all held as per-lane partial sums).
 // ---------------------------------------------------------------------------
-// x of probe p, elements i .. i + V - 1: loaded, or (sm.partial) formed
-// from a deferred split-K sum exactly as the matvec's reduction does and
-// stored to x.
+// A deferred split-K sum at NE groups of V elements from off[e] (in range for
+// every lane), added in the order of the matvec's own reduction.  The planes'
+// loads are issued kSumBatch at a time for all groups: one plane at a time, the
+// sum over 8 slices took 3.7 us of the 10.5 us of the dots at n = 8192, 32
+// probes.
 // (The partial planes z >= 1 start at z P n floats, which need not keep the
 // 16-byte alignment of plane 0 when P n % 4 != 0: they are read by memcpy,
 // one global_load_dwordx4 at any dword alignment on gfx950.)
-template <int V>
-__device__ __forceinline__ void load_x(float* x, const MvSplitSum& sm, int64_t P, int64_t n,
-                                       int64_t p, int64_t i, float (&xv)[V]) {
-  const int64_t count = P * n, off = p * n + i;
-  __builtin_memcpy(xv, sm.partial + off, sizeof(xv));
-  for (int z = 1; z < sm.S; ++z) {
-    float pz[V];
-    __builtin_memcpy(pz, sm.partial + int64_t(z) * count + off, sizeof(pz));
+constexpr int kSumBatch = 4;
+
+template <int V, int NE>
+__device__ __forceinline__ void split_sum(const MvSplitSum& sm, int64_t count,
+                                          const int64_t (&off)[NE], float (&xv)[NE][V]) {
+  float vv[NE][V];
 #pragma unroll
-    for (int v = 0; v < V; ++v) xv[v] += pz[v];
+  for (int e = 0; e < NE; ++e) {
+    __builtin_memcpy(xv[e], sm.partial + off[e], sizeof(xv[e]));
+    if (sm.nugget) __builtin_memcpy(vv[e], sm.V + off[e], sizeof(vv[e]));
   }
-  if (sm.nugget) {
-    float vv[V];
-    __builtin_memcpy(vv, sm.V + off, sizeof(vv));
+  for (int z0 = 1; z0 < sm.S; z0 += kSumBatch) {
+    float pz[kSumBatch][NE][V];
 #pragma unroll
-    for (int v = 0; v < V; ++v) xv[v] = fmaf(sm.noise, vv[v], xv[v]);
+    for (int u = 0; u < kSumBatch; ++u) {
+      const float* plane = sm.partial + int64_t(z0 + u < sm.S ? z0 + u : sm.S - 1) * count;
+#pragma unroll
+      for (int e = 0; e < NE; ++e) __builtin_memcpy(pz[u][e], plane + off[e], sizeof(pz[u][e]));
+    }
+#pragma unroll
+    for (int u = 0; u < kSumBatch; ++u)
+      if (z0 + u < sm.S)
+#pragma unroll
+        for (int e = 0; e < NE; ++e)
+#pragma unroll
+          for (int v = 0; v < V; ++v) xv[e][v] += pz[u][e][v];
   }
-  VecIO<V>::store(x + p * n + i, xv);
+  if (sm.nugget)
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+#pragma unroll
+      for (int v = 0; v < V; ++v) xv[e][v] = fmaf(sm.noise, vv[e][v], xv[e][v]);
 }
 
 // Basis columns whose loads are issued together (one batch in flight per
@@ -170,66 +187,89 @@ __device__ __forceinline__ void load_x(float* x, const MvSplitSum& sm, int64_t P
 // not used), and element groups past n read the row's last group with x = 0.
 constexpr int kColBatch = 8;
 
+// Blocks (chunks times probes) from which the streaming kernels are bound by
+// the memory rather than by the latency of a block's own chain of loads.
+constexpr int64_t kManyBlocks = 1024;
+
+// Columns of a block of the dots kernels; the other columns of a chunk are
+// blocks of their own.  Few blocks: 8, so that no block waits for one batch of
+// loads after the other (n = 1001, 16 probes: 5% of a decomposition).  Many:
+// 16, which halves the reads of x (n = 32768, 128 probes, 64 columns: no
+// difference between 8 and 64, the memory bounds them all).
+inline int dots_columns(int64_t blocks, int ncols) {
+  return blocks < kManyBlocks || ncols <= 8 ? 8 : ncols <= 16 ? 16 : 32;
+}
+
+// SUM: x is the deferred split-K sum `sm`, stored to xw by the blocks of
+// column group 0.  blockIdx.z = row * column groups + column group; row i reads
+// x + i xrow and writes partial + i prow.
 template <int V, int NC, bool SUM>
 __global__ void __launch_bounds__(kStreamThreads)
     k_dots(const float* __restrict__ Q, int64_t ldc, const float* __restrict__ x, float* xw,
            int64_t n, int ncols, float* __restrict__ partial, int pstride, int64_t xrow,
            int64_t prow, MvSplitSum sm) {
   constexpr int NE = Layout<V>::NE;
-  constexpr int CB = NC < kColBatch ? NC : kColBatch;
+  constexpr int CB = kColBatch;
   __shared__ float red[kWaves * NC];
   const int64_t p = blockIdx.y;
   const int64_t b = blockIdx.x;
   const int64_t nb = gridDim.x;
   const int t = threadIdx.x;
   const int64_t base = b * kChunk;
-  x += blockIdx.z * xrow;
-  partial += blockIdx.z * prow;
+  const int groups = (ncols + NC - 1) / NC;
+  const int64_t row = blockIdx.z / groups;
+  const int c0 = int(blockIdx.z % groups) * NC;
 
-  float xv[NE][V];
   int64_t off[NE];
+  bool in[NE];
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
     const int64_t i = base + (int64_t(e) * kStreamThreads + t) * V;
-    off[e] = i < n ? i : n - V;  // V divides n
-    if (i < n) {
-      if constexpr (SUM)
-        load_x<V>(xw, sm, int64_t(gridDim.y), n, p, i, xv[e]);
-      else
-        VecIO<V>::load(x + p * n + i, xv[e]);
-    } else {
-#pragma unroll
-      for (int v = 0; v < V; ++v) xv[e][v] = 0.f;
-    }
+    in[e] = i < n;
+    off[e] = p * n + (in[e] ? i : n - V);  // V divides n
   }
-
-  const float* qp = Q + p * n;
-  for (int c0 = 0; c0 < ncols; c0 += NC) {
-    float acc[NC];
+  float qv[CB][NE][V];
+  auto load = [&](int g) {
 #pragma unroll
-    for (int c = 0; c < NC; ++c) acc[c] = 0.f;
+    for (int u = 0; u < CB; ++u) {
+      const int c = c0 + g + u;
+      const float* q = Q + int64_t(c < ncols ? c : ncols - 1) * ldc;
 #pragma unroll
-    for (int g = 0; g < NC; g += CB) {
-      if (c0 + g < ncols) {
-        float qv[CB][NE][V];
-#pragma unroll
-        for (int u = 0; u < CB; ++u) {
-          const int c = c0 + g + u < ncols ? c0 + g + u : ncols - 1;
-          const float* q = qp + int64_t(c) * ldc;
-#pragma unroll
-          for (int e = 0; e < NE; ++e) VecIO<V>::load(q + off[e], qv[u][e]);
-        }
-#pragma unroll
-        for (int u = 0; u < CB; ++u)
-#pragma unroll
-          for (int e = 0; e < NE; ++e)
-#pragma unroll
-            for (int v = 0; v < V; ++v) acc[g + u] = fmaf(qv[u][e][v], xv[e][v], acc[g + u]);
-      }
+      for (int e = 0; e < NE; ++e) VecIO<V>::load(q + off[e], qv[u][e]);
     }
-    const int live = ncols - c0 < NC ? ncols - c0 : NC;
-    block_column_sums<NC>(acc, live, red, partial + (p * nb + b) * pstride + c0);
+  };
+  load(0);
+  float xv[NE][V];
+  if constexpr (SUM) {
+    split_sum<V, NE>(sm, int64_t(gridDim.y) * n, off, xv);
+  } else {
+#pragma unroll
+    for (int e = 0; e < NE; ++e) VecIO<V>::load(x + row * xrow + off[e], xv[e]);
   }
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    if (SUM && in[e] && c0 == 0) VecIO<V>::store(xw + off[e], xv[e]);
+#pragma unroll
+    for (int v = 0; v < V; ++v) xv[e][v] = in[e] ? xv[e][v] : 0.f;
+  }
+  float acc[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) acc[c] = 0.f;
+#pragma unroll
+  for (int g = 0; g < NC; g += CB) {
+    if (g > 0) {
+      if (c0 + g >= ncols) break;
+      load(g);
+    }
+#pragma unroll
+    for (int u = 0; u < CB; ++u)
+#pragma unroll
+      for (int e = 0; e < NE; ++e)
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[g + u] = fmaf(qv[u][e][v], xv[e][v], acc[g + u]);
+  }
+  const int live = ncols - c0 < NC ? ncols - c0 : NC;
+  block_column_sums<NC>(acc, live, red, partial + row * prow + (p * nb + b) * pstride + c0);
 }
 
 // Rows whose length n is not a multiple of 4 start at every alignment (probe
@@ -262,80 +302,84 @@ struct ShiftedRow {
   }
 };
 
-// SUM: x is the deferred split-K sum `sm` (formed as the matvec's reduction
-// does it and written to xw), as in k_dots.
+// k_dots for such rows.
 template <int NC, bool SUM>
 __global__ void __launch_bounds__(kStreamThreads)
     k_dots_shifted(const float* __restrict__ Q, int64_t ldc, const float* __restrict__ x,
                    float* xw, int64_t n, int ncols, float* __restrict__ partial, int pstride,
                    int64_t xrow, int64_t prow, MvSplitSum sm) {
   constexpr int NE = Layout<4>::NE;
-  constexpr int CB = NC < kColBatch ? NC : kColBatch;
+  constexpr int CB = kColBatch;
   __shared__ float red[kWaves * NC];
   const int64_t p = blockIdx.y, b = blockIdx.x, nb = gridDim.x;
   const int t = threadIdx.x;
+  const int groups = (ncols + NC - 1) / NC;
+  const int64_t drow = blockIdx.z / groups;
+  const int c0 = int(blockIdx.z % groups) * NC;
   const ShiftedRow row(p, n, b, t);
-  const float* xr = x + blockIdx.z * xrow + p * n;
-  partial += blockIdx.z * prow;
-  float xv[NE][4];
   int64_t off[NE];
+  bool in[NE];
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
     const int64_t i = ShiftedRow::group(p, n, b, e, t);
-    const bool full = i < row.gend;
-    off[e] = full ? i : row.gend - 4;
-    if (full) {
-      if constexpr (SUM)
-        load_x<4>(xw, sm, int64_t(gridDim.y), n, p, i, xv[e]);
-      else
-        VecIO<4>::load(xr + i, xv[e]);
-    } else {
+    in[e] = i < row.gend;
+    off[e] = p * n + (in[e] ? i : row.gend - 4);
+  }
+  const bool single = row.ix >= 0;
+  const int64_t ixo[1] = {p * n + (single ? row.ix : 0)};
+  float qv[CB][NE][4], qh[CB];
+  auto load = [&](int g) {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) xv[e][v] = 0.f;
+    for (int u = 0; u < CB; ++u) {
+      const int c = c0 + g + u;
+      const float* q = Q + int64_t(c < ncols ? c : ncols - 1) * ldc;
+#pragma unroll
+      for (int e = 0; e < NE; ++e) VecIO<4>::load(q + off[e], qv[u][e]);
+      qh[u] = q[ixo[0]];
+    }
+  };
+  load(0);
+  float xv[NE][4], xh[1][1];
+  if constexpr (SUM) {
+    split_sum<4, NE>(sm, int64_t(gridDim.y) * n, off, xv);
+    split_sum<1, 1>(sm, int64_t(gridDim.y) * n, ixo, xh);
+  } else {
+    const float* xr = x + drow * xrow;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) VecIO<4>::load(xr + off[e], xv[e]);
+    xh[0][0] = xr[ixo[0]];
+  }
+  if (SUM && c0 == 0) {
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+      if (in[e]) VecIO<4>::store(xw + off[e], xv[e]);
+    if (single) xw[ixo[0]] = xh[0][0];
+  }
+#pragma unroll
+  for (int e = 0; e < NE; ++e)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) xv[e][v] = in[e] ? xv[e][v] : 0.f;
+  const float x1 = single ? xh[0][0] : 0.f;
+  float acc[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) acc[c] = 0.f;
+#pragma unroll
+  for (int g = 0; g < NC; g += CB) {
+    if (g > 0) {
+      if (c0 + g >= ncols) break;
+      load(g);
+    }
+#pragma unroll
+    for (int u = 0; u < CB; ++u) {
+#pragma unroll
+      for (int e = 0; e < NE; ++e)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[g + u] = fmaf(qv[u][e][v], xv[e][v], acc[g + u]);
+      acc[g + u] = fmaf(qh[u], x1, acc[g + u]);
     }
   }
-  const int64_t ixo = row.ix >= 0 ? row.ix : 0;
-  float xh = 0.f;
-  if (row.ix >= 0) {
-    if constexpr (SUM) {
-      float one[1];
-      load_x<1>(xw, sm, int64_t(gridDim.y), n, p, ixo, one);
-      xh = one[0];
-    } else {
-      xh = xr[ixo];
-    }
-  }
-
-  const float* qp = Q + p * n;
-  for (int c0 = 0; c0 < ncols; c0 += NC) {
-    float acc[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) acc[c] = 0.f;
-#pragma unroll
-    for (int g = 0; g < NC; g += CB) {
-      if (c0 + g < ncols) {
-        float qv[CB][NE][4], qh[CB];
-#pragma unroll
-        for (int u = 0; u < CB; ++u) {
-          const int c = c0 + g + u < ncols ? c0 + g + u : ncols - 1;
-          const float* q = qp + int64_t(c) * ldc;
-#pragma unroll
-          for (int e = 0; e < NE; ++e) VecIO<4>::load(q + off[e], qv[u][e]);
-          qh[u] = q[ixo];
-        }
-#pragma unroll
-        for (int u = 0; u < CB; ++u) {
-#pragma unroll
-          for (int e = 0; e < NE; ++e)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[g + u] = fmaf(qv[u][e][v], xv[e][v], acc[g + u]);
-          acc[g + u] = fmaf(qh[u], xh, acc[g + u]);
-        }
-      }
-    }
-    const int live = ncols - c0 < NC ? ncols - c0 : NC;
-    block_column_sums<NC>(acc, live, red, partial + (p * nb + b) * pstride + c0);
-  }
+  const int live = ncols - c0 < NC ? ncols - c0 : NC;
+  block_column_sums<NC>(acc, live, red, partial + drow * prow + (p * nb + b) * pstride + c0);
 }
 
 // sum of squares: partial[p][b] = sum over chunk b of x[p][:]^2
@@ -438,12 +482,13 @@ __device__ __forceinline__ void store_planes(const PlaneOut& pl, int64_t p, int6
 
 // ---------------------------------------------------------------------------
 // project: y = x - Q h (h from partials); optional norm^2 partials of y.
-// Columns in batches of kColBatch loaded together, the last ncols % kColBatch
-// in batches of 4, 2 and 1 (no column is read twice).  pl (V = 4): the planes
+// Columns in batches of kColBatch loaded together, one batch ahead of the one
+// being added (the first before the coefficients are summed); the last batch
+// repeats the last column (from the L1).  pl (V = 4): the planes
 // of y for the matvec that follows, which saves its split launch (3.3 us at
 // n = 8192, 32 probes).
 // ---------------------------------------------------------------------------
-template <int V>
+template <int V, bool AHEAD, bool PLANES>
 __global__ void __launch_bounds__(kStreamThreads)
     k_project(const float* __restrict__ Q, int64_t ldc, const float* __restrict__ x,
               float* __restrict__ y, int64_t n, int ncols, const float* __restrict__ hpart,
@@ -451,13 +496,12 @@ __global__ void __launch_bounds__(kStreamThreads)
               int64_t hout_stride, const float* __restrict__ hsub, int64_t hsub_stride,
               PlaneOut pl) {
   constexpr int NE = Layout<V>::NE;
+  constexpr int CB = kColBatch;
   extern __shared__ float hs[];
   __shared__ float red[kWaves];
   const int64_t p = blockIdx.y, b = blockIdx.x, nb = gridDim.x;
   const int t = threadIdx.x;
   const int64_t base = b * kChunk;
-  load_coeffs(hpart, p, nb, ncols, pstride, hs, hout, hout_stride, b == 0, hsub, hsub_stride);
-
   float s[NE][V];
   int64_t off[NE];
 #pragma unroll
@@ -469,18 +513,20 @@ __global__ void __launch_bounds__(kStreamThreads)
   }
 
   const float* qp = Q + p * n;
-  // columns [c0, c0 + B), loaded together, added in column order
-  auto batch = [&](auto bsz, int c0) {
-    constexpr int B = decltype(bsz)::value;
-    float qv[B][NE][V];
+  using Batch = float[CB][NE][V];
+  // columns [c0, c0 + CB), loaded together, added in column order
+  auto load = [&](int c0, Batch& qv) {
 #pragma unroll
-    for (int u = 0; u < B; ++u) {
-      const float* q = qp + int64_t(c0 + u) * ldc;
+    for (int u = 0; u < CB; ++u) {
+      const float* q = qp + int64_t(c0 + u < ncols ? c0 + u : ncols - 1) * ldc;
 #pragma unroll
       for (int e = 0; e < NE; ++e) VecIO<V>::load(q + off[e], qv[u][e]);
     }
+  };
+  auto add = [&](int c0, const Batch& qv) {
 #pragma unroll
-    for (int u = 0; u < B; ++u) {
+    for (int u = 0; u < CB; ++u) {
+      if (c0 + u >= ncols) break;
       const float hc = hs[c0 + u];
 #pragma unroll
       for (int e = 0; e < NE; ++e)
@@ -488,11 +534,44 @@ __global__ void __launch_bounds__(kStreamThreads)
         for (int v = 0; v < V; ++v) s[e][v] = fmaf(qv[u][e][v], hc, s[e][v]);
     }
   };
-  int c0 = 0;
-  for (; c0 + kColBatch <= ncols; c0 += kColBatch) batch(std::integral_constant<int, kColBatch>{}, c0);
-  if (c0 + 4 <= ncols) { batch(std::integral_constant<int, 4>{}, c0); c0 += 4; }
-  if (c0 + 2 <= ncols) { batch(std::integral_constant<int, 2>{}, c0); c0 += 2; }
-  if (c0 < ncols) batch(std::integral_constant<int, 1>{}, c0);
+  Batch qa;
+  if constexpr (AHEAD) {
+    Batch qb;
+    if (ncols > 0) load(0, qa);
+    load_coeffs(hpart, p, nb, ncols, pstride, hs, hout, hout_stride, b == 0, hsub, hsub_stride);
+    for (int c0 = 0; c0 < ncols; c0 += 2 * CB) {
+      if (c0 + CB < ncols) load(c0 + CB, qb);
+      add(c0, qa);
+      if (c0 + CB >= ncols) break;
+      if (c0 + 2 * CB < ncols) load(c0 + 2 * CB, qa);
+      add(c0 + CB, qb);
+    }
+  } else {
+    load_coeffs(hpart, p, nb, ncols, pstride, hs, hout, hout_stride, b == 0, hsub, hsub_stride);
+    auto batch = [&](auto bsz, int c0) {
+      constexpr int B = decltype(bsz)::value;
+      float qv[B][NE][V];
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        const float* q = qp + int64_t(c0 + u) * ldc;
+#pragma unroll
+        for (int e = 0; e < NE; ++e) VecIO<V>::load(q + off[e], qv[u][e]);
+      }
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        const float hc = hs[c0 + u];
+#pragma unroll
+        for (int e = 0; e < NE; ++e)
+#pragma unroll
+          for (int v = 0; v < V; ++v) s[e][v] = fmaf(qv[u][e][v], hc, s[e][v]);
+      }
+    };
+    int c0 = 0;
+    for (; c0 + CB <= ncols; c0 += CB) batch(std::integral_constant<int, CB>{}, c0);
+    if (c0 + 4 <= ncols) { batch(std::integral_constant<int, 4>{}, c0); c0 += 4; }
+    if (c0 + 2 <= ncols) { batch(std::integral_constant<int, 2>{}, c0); c0 += 2; }
+    if (c0 < ncols) batch(std::integral_constant<int, 1>{}, c0);
+  }
 
   float acc = 0.f;
 #pragma unroll
@@ -507,8 +586,7 @@ __global__ void __launch_bounds__(kStreamThreads)
         acc = fmaf(xv[v], xv[v], acc);
       }
       VecIO<V>::store(y + p * n + i, xv);
-      if constexpr (V == 4)
-        if (pl.hi) store_planes<V>(pl, p, i, xv);
+      if constexpr (PLANES) store_planes<V>(pl, p, i, xv);
     }
   }
   if (norm2part) {
@@ -518,6 +596,7 @@ __global__ void __launch_bounds__(kStreamThreads)
 }
 
 // k_project for rows that start at every alignment (see k_dots_shifted).
+template <bool AHEAD>
 __global__ void __launch_bounds__(kStreamThreads)
     k_project_shifted(const float* __restrict__ Q, int64_t ldc, const float* __restrict__ x,
                       float* __restrict__ y, int64_t n, int ncols,
@@ -525,13 +604,12 @@ __global__ void __launch_bounds__(kStreamThreads)
                       float* __restrict__ norm2part, float* __restrict__ hout,
                       int64_t hout_stride, const float* __restrict__ hsub, int64_t hsub_stride) {
   constexpr int NE = Layout<4>::NE;
+  constexpr int CB = kColBatch;
   extern __shared__ float hs[];
   __shared__ float red[kWaves];
   const int64_t p = blockIdx.y, b = blockIdx.x, nb = gridDim.x;
   const int t = threadIdx.x;
   const ShiftedRow row(p, n, b, t);
-  load_coeffs(hpart, p, nb, ncols, pstride, hs, hout, hout_stride, b == 0, hsub, hsub_stride);
-
   float s[NE][4];
   int64_t off[NE];
 #pragma unroll
@@ -545,31 +623,70 @@ __global__ void __launch_bounds__(kStreamThreads)
   float sx = 0.f;
 
   const float* qp = Q + p * n;
-  auto batch = [&](auto bsz, int c0) {
-    constexpr int B = decltype(bsz)::value;
-    float qv[B][NE][4], qh[B];
+  struct Batch {
+    float v[CB][NE][4], h[CB];
+  };
+  auto load = [&](int c0, Batch& qv) {
 #pragma unroll
-    for (int u = 0; u < B; ++u) {
-      const float* q = qp + int64_t(c0 + u) * ldc;
+    for (int u = 0; u < CB; ++u) {
+      const float* q = qp + int64_t(c0 + u < ncols ? c0 + u : ncols - 1) * ldc;
 #pragma unroll
-      for (int e = 0; e < NE; ++e) VecIO<4>::load(q + off[e], qv[u][e]);
-      qh[u] = q[ixo];
+      for (int e = 0; e < NE; ++e) VecIO<4>::load(q + off[e], qv.v[u][e]);
+      qv.h[u] = q[ixo];
     }
+  };
+  auto add = [&](int c0, const Batch& qv) {
 #pragma unroll
-    for (int u = 0; u < B; ++u) {
+    for (int u = 0; u < CB; ++u) {
+      if (c0 + u >= ncols) break;
       const float hc = hs[c0 + u];
 #pragma unroll
       for (int e = 0; e < NE; ++e)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) s[e][v] = fmaf(qv[u][e][v], hc, s[e][v]);
-      sx = fmaf(qh[u], hc, sx);
+        for (int v = 0; v < 4; ++v) s[e][v] = fmaf(qv.v[u][e][v], hc, s[e][v]);
+      sx = fmaf(qv.h[u], hc, sx);
     }
   };
-  int c0 = 0;
-  for (; c0 + kColBatch <= ncols; c0 += kColBatch) batch(std::integral_constant<int, kColBatch>{}, c0);
-  if (c0 + 4 <= ncols) { batch(std::integral_constant<int, 4>{}, c0); c0 += 4; }
-  if (c0 + 2 <= ncols) { batch(std::integral_constant<int, 2>{}, c0); c0 += 2; }
-  if (c0 < ncols) batch(std::integral_constant<int, 1>{}, c0);
+  Batch qa;
+  if constexpr (AHEAD) {
+    Batch qb;
+    if (ncols > 0) load(0, qa);
+    load_coeffs(hpart, p, nb, ncols, pstride, hs, hout, hout_stride, b == 0, hsub, hsub_stride);
+    for (int c0 = 0; c0 < ncols; c0 += 2 * CB) {
+      if (c0 + CB < ncols) load(c0 + CB, qb);
+      add(c0, qa);
+      if (c0 + CB >= ncols) break;
+      if (c0 + 2 * CB < ncols) load(c0 + 2 * CB, qa);
+      add(c0 + CB, qb);
+    }
+  } else {
+    load_coeffs(hpart, p, nb, ncols, pstride, hs, hout, hout_stride, b == 0, hsub, hsub_stride);
+    auto batch = [&](auto bsz, int c0) {
+      constexpr int B = decltype(bsz)::value;
+      float qv[B][NE][4], qh[B];
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        const float* q = qp + int64_t(c0 + u) * ldc;
+#pragma unroll
+        for (int e = 0; e < NE; ++e) VecIO<4>::load(q + off[e], qv[u][e]);
+        qh[u] = q[ixo];
+      }
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        const float hc = hs[c0 + u];
+#pragma unroll
+        for (int e = 0; e < NE; ++e)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) s[e][v] = fmaf(qv[u][e][v], hc, s[e][v]);
+        sx = fmaf(qh[u], hc, sx);
+      }
+    };
+    int c0 = 0;
+    for (; c0 + CB <= ncols; c0 += CB) batch(std::integral_constant<int, CB>{}, c0);
+    if (c0 + 4 <= ncols) { batch(std::integral_constant<int, 4>{}, c0); c0 += 4; }
+    if (c0 + 2 <= ncols) { batch(std::integral_constant<int, 2>{}, c0); c0 += 2; }
+    if (c0 < ncols) batch(std::integral_constant<int, 1>{}, c0);
+  }
 
   float acc = 0.f;
   const float* xr = x + p * n;
@@ -808,36 +925,53 @@ inline int stream_width(int64_t n, int64_t ld, std::initializer_list<const void*
   return 1;
 }
 
-template <int V>
-hipError_t launch_dots_v(hipStream_t s, const float* Q, int64_t ldc, const float* x, int64_t P,
-                         int64_t n, int ncols, float* partial, int pstride, int64_t rows,
-                         int64_t xrow, int64_t prow) {
-  const dim3 grid(unsigned(num_chunks(n)), unsigned(P), unsigned(rows));
+// k_dots / k_dots_shifted; SUM: x is the split-K sum, written to xw
+template <bool SUM>
+hipError_t launch_dots_any(hipStream_t s, const float* Q, int64_t ldc, const float* x, float* xw,
+                           const MvSplitSum& sum, int64_t P, int64_t n, int ncols, float* partial,
+                           int pstride, int64_t rows, int64_t xrow, int64_t prow,
+                           std::initializer_list<const void*> ptrs) {
+  const int V = stream_width(n, ldc, ptrs);
+  const bool shifted = shifted_ok(n, ldc, ptrs);  // faster than the float2 kernels for even n
+  const int64_t nb = num_chunks(n);
+  const int nc = V == 4 || shifted ? dots_columns(nb * P * rows, ncols) : 8;
+  const dim3 grid(unsigned(nb), unsigned(P), unsigned(rows * ((ncols + nc - 1) / nc)));
   const dim3 block(kStreamThreads);
-  const MvSplitSum sm;
-  if (ncols <= 8)
-    hipLaunchKernelGGL((k_dots<V, 8, false>), grid, block, 0, s, Q, ldc, x, nullptr, n, ncols,
-                       partial, pstride, xrow, prow, sm);
-  else if (ncols <= 16)
-    hipLaunchKernelGGL((k_dots<V, 16, false>), grid, block, 0, s, Q, ldc, x, nullptr, n, ncols,
-                       partial, pstride, xrow, prow, sm);
-  else if (ncols <= 32)
-    hipLaunchKernelGGL((k_dots<V, 32, false>), grid, block, 0, s, Q, ldc, x, nullptr, n, ncols,
-                       partial, pstride, xrow, prow, sm);
-  else
-    hipLaunchKernelGGL((k_dots<V, 64, false>), grid, block, 0, s, Q, ldc, x, nullptr, n, ncols,
-                       partial, pstride, xrow, prow, sm);
+  auto wide = [&](auto columns) {
+    constexpr int NC = decltype(columns)::value;
+    if (V == 4)
+      hipLaunchKernelGGL((k_dots<4, NC, SUM>), grid, block, 0, s, Q, ldc, x, xw, n, ncols, partial,
+                         pstride, xrow, prow, sum);
+    else
+      hipLaunchKernelGGL((k_dots_shifted<NC, SUM>), grid, block, 0, s, Q, ldc, x, xw, n, ncols,
+                         partial, pstride, xrow, prow, sum);
+  };
+  if (V == 4 || shifted) {
+    if (nc == 8)
+      wide(std::integral_constant<int, 8>{});
+    else if (nc == 16)
+      wide(std::integral_constant<int, 16>{});
+    else
+      wide(std::integral_constant<int, 32>{});
+  } else if (V == 2) {
+    hipLaunchKernelGGL((k_dots<2, 8, SUM>), grid, block, 0, s, Q, ldc, x, xw, n, ncols, partial,
+                       pstride, xrow, prow, sum);
+  } else {
+    hipLaunchKernelGGL((k_dots<1, 8, SUM>), grid, block, 0, s, Q, ldc, x, xw, n, ncols, partial,
+                       pstride, xrow, prow, sum);
+  }
   return hipGetLastError();
 }
 
 }  // namespace
 
+int64_t max_dot_rows(int64_t ncols) { return std::max<int64_t>(1, 65535 / ((ncols + 7) / 8)); }
+
 hipError_t launch_dots(hipStream_t s, const float* Q, int64_t ldc, const float* x, int64_t P,
                        int64_t n, int ncols, float* partial, int pstride, int64_t rows,
                        int64_t xrow, int64_t prow) {
-  if (rows > 1 && xrow % 4 != 0) return hipErrorInvalidValue;  // one alignment for all rows
-  const int V = Q ? stream_width(n, ldc, {x, Q}) : stream_width(n, n, {x});
   if (Q == nullptr) {
+    const int V = stream_width(n, n, {x});
     const dim3 grid(unsigned(num_chunks(n)), unsigned(P));
     if (V == 4)
       hipLaunchKernelGGL(k_sumsq<4>, grid, dim3(kStreamThreads), 0, s, x, n, partial);
@@ -847,89 +981,50 @@ hipError_t launch_dots(hipStream_t s, const float* Q, int64_t ldc, const float* 
       hipLaunchKernelGGL(k_sumsq<1>, grid, dim3(kStreamThreads), 0, s, x, n, partial);
     return hipGetLastError();
   }
-  if (V == 4)
-    return launch_dots_v<4>(s, Q, ldc, x, P, n, ncols, partial, pstride, rows, xrow, prow);
-  if (shifted_ok(n, ldc, {x, Q})) {  // measured faster than the float2 kernels for even n
-    const dim3 grid(unsigned(num_chunks(n)), unsigned(P), unsigned(rows));
-    const dim3 block(kStreamThreads);
-    if (ncols <= 8)
-      hipLaunchKernelGGL((k_dots_shifted<8, false>), grid, block, 0, s, Q, ldc, x, nullptr, n,
-                         ncols, partial, pstride, xrow, prow, MvSplitSum{});
-    else if (ncols <= 16)
-      hipLaunchKernelGGL((k_dots_shifted<16, false>), grid, block, 0, s, Q, ldc, x, nullptr, n,
-                         ncols, partial, pstride, xrow, prow, MvSplitSum{});
-    else if (ncols <= 32)
-      hipLaunchKernelGGL((k_dots_shifted<32, false>), grid, block, 0, s, Q, ldc, x, nullptr, n,
-                         ncols, partial, pstride, xrow, prow, MvSplitSum{});
-    else
-      hipLaunchKernelGGL((k_dots_shifted<64, false>), grid, block, 0, s, Q, ldc, x, nullptr, n,
-                         ncols, partial, pstride, xrow, prow, MvSplitSum{});
-    return hipGetLastError();
-  }
-  if (V == 2)
-    return launch_dots_v<2>(s, Q, ldc, x, P, n, ncols, partial, pstride, rows, xrow, prow);
-  return launch_dots_v<1>(s, Q, ldc, x, P, n, ncols, partial, pstride, rows, xrow, prow);
+  if (rows > 1 && xrow % 4 != 0) return hipErrorInvalidValue;  // one alignment for all rows
+  return launch_dots_any<false>(s, Q, ldc, x, nullptr, MvSplitSum{}, P, n, ncols, partial, pstride,
+                                rows, xrow, prow, {x, Q});
 }
 
 hipError_t launch_dots_sum(hipStream_t s, const float* Q, int64_t ldc, const MvSplitSum& sum,
                            float* x, int64_t P, int64_t n, int ncols, float* partial, int pstride) {
-  const dim3 grid(unsigned(num_chunks(n)), unsigned(P));
-  const dim3 block(kStreamThreads);
-  const std::initializer_list<const void*> ptrs = {x, Q, sum.partial, sum.nugget ? sum.V : x};
-  const int V = stream_width(n, ldc, ptrs);
-#define SLQ_DS(VV, NC)                                                                          \
-  hipLaunchKernelGGL((k_dots<VV, NC, true>), grid, block, 0, s, Q, ldc, nullptr, x, n, ncols, \
-                     partial, pstride, 0, 0, sum)
-#define SLQ_DSH(NC)                                                                          \
-  hipLaunchKernelGGL((k_dots_shifted<NC, true>), grid, block, 0, s, Q, ldc, nullptr, x, n, \
-                     ncols, partial, pstride, 0, 0, sum)
-#define SLQ_DS_NC(M)         \
-  if (ncols <= 8) M(8);      \
-  else if (ncols <= 16) M(16); \
-  else if (ncols <= 32) M(32); \
-  else M(64)
-  if (V == 4) {
-#define SLQ_DS4(NC) SLQ_DS(4, NC)
-    SLQ_DS_NC(SLQ_DS4);
-#undef SLQ_DS4
-  } else if (shifted_ok(n, ldc, ptrs)) {
-    SLQ_DS_NC(SLQ_DSH);
-  } else if (V == 2) {
-#define SLQ_DS2(NC) SLQ_DS(2, NC)
-    SLQ_DS_NC(SLQ_DS2);
-#undef SLQ_DS2
-  } else {
-#define SLQ_DS1(NC) SLQ_DS(1, NC)
-    SLQ_DS_NC(SLQ_DS1);
-#undef SLQ_DS1
-  }
-#undef SLQ_DS_NC
-#undef SLQ_DSH
-#undef SLQ_DS
-  return hipGetLastError();
+  return launch_dots_any<true>(s, Q, ldc, nullptr, x, sum, P, n, ncols, partial, pstride, 1, 0, 0,
+                               {x, Q, sum.partial, sum.nugget ? sum.V : x});
 }
 
 hipError_t launch_project(hipStream_t s, const float* Q, int64_t ldc, const float* x, float* y,
                           int64_t P, int64_t n, int ncols, const float* hpart, int pstride,
                           float* norm2part, float* hout, int64_t hout_stride, const float* hsub,
                           int64_t hsub_stride, const PlaneOut* planes) {
-  const dim3 grid(unsigned(num_chunks(n)), unsigned(P));
+  const int64_t nb = num_chunks(n);
+  const dim3 grid{unsigned(nb), unsigned(P)};
   const size_t shmem = size_t(ncols > 0 ? ncols : 1) * sizeof(float);
   const int V = stream_width(n, ldc, {x, y, Q});
   if (planes && V != 4) return hipErrorInvalidValue;
-  const PlaneOut pl = planes ? *planes : PlaneOut{};
-  if (V == 4)
-    hipLaunchKernelGGL(k_project<4>, grid, dim3(kStreamThreads), shmem, s, Q, ldc, x, y, n, ncols,
-                       hpart, pstride, norm2part, hout, hout_stride, hsub, hsub_stride, pl);
-  else if (shifted_ok(n, ldc, {x, y, Q}))  // measured faster than the float2 kernel for even n
-    hipLaunchKernelGGL(k_project_shifted, grid, dim3(kStreamThreads), shmem, s, Q, ldc, x, y, n,
-                       ncols, hpart, pstride, norm2part, hout, hout_stride, hsub, hsub_stride);
-  else if (V == 2)
-    hipLaunchKernelGGL(k_project<2>, grid, dim3(kStreamThreads), shmem, s, Q, ldc, x, y, n, ncols,
-                       hpart, pstride, norm2part, hout, hout_stride, hsub, hsub_stride, pl);
-  else
-    hipLaunchKernelGGL(k_project<1>, grid, dim3(kStreamThreads), shmem, s, Q, ldc, x, y, n, ncols,
-                       hpart, pstride, norm2part, hout, hout_stride, hsub, hsub_stride, pl);
+  const bool ahead = nb * P < kManyBlocks;
+#define SLQ_PROJECT(K, ...)                                                                     \
+  hipLaunchKernelGGL(K, grid, dim3(kStreamThreads), shmem, s, Q, ldc, x, y, n, ncols, hpart,    \
+                     pstride, norm2part, hout, hout_stride, hsub, hsub_stride, ##__VA_ARGS__)
+  if (V == 4) {
+    if (planes && ahead)
+      SLQ_PROJECT((k_project<4, true, true>), *planes);
+    else if (planes)
+      SLQ_PROJECT((k_project<4, false, true>), *planes);
+    else if (ahead)
+      SLQ_PROJECT((k_project<4, true, false>), PlaneOut{});
+    else
+      SLQ_PROJECT((k_project<4, false, false>), PlaneOut{});
+  } else if (shifted_ok(n, ldc, {x, y, Q})) {  // measured faster than the float2 kernel for even n
+    if (ahead)
+      SLQ_PROJECT((k_project_shifted<true>));
+    else
+      SLQ_PROJECT((k_project_shifted<false>));
+  } else if (V == 2) {
+    SLQ_PROJECT((k_project<2, false, false>), PlaneOut{});
+  } else {
+    SLQ_PROJECT((k_project<1, false, false>), PlaneOut{});
+  }
+#undef SLQ_PROJECT
   return hipGetLastError();
 }
 

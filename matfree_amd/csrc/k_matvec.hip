@@ -1274,6 +1274,109 @@ __global__ void __launch_bounds__(64 * kStreamWaves, 3)
               [](float (&)[4]) {});
 }
 
+// FP32-unit form, for the forward pass that a reverse pass is taken at
+// (kPrecFp32Units): products and sums on the FP32 matrix cores, 128 rows per
+// workgroup, 32 per wave, the rows' fragments loaded a tile ahead by each
+// wave, the probe tiles staged in LDS.  A general cotangent's reverse scan
+// multiplies the rounding of the basis it is taken at by a hundred to a
+// thousand (n = 1500, 32 steps: T good to 8e-8, the start vectors' cotangent
+// to 2e-6 .. 1e-4 from one matrix to the next), so any other order of these
+// sums gives another cotangent, no nearer and no further on average; the
+// scan's own products do not matter in that way.  n = 4096, 32 probes: 19 us,
+// as the stream form.
+constexpr int LDU = BK + 4;  // padded LDS row of floats
+
+template <int NACC>
+__global__ void __launch_bounds__(kThreads)
+    k_matvec_f32_units(const float* __restrict__ A, const float* __restrict__ V, int64_t P,
+                       int64_t n, float* __restrict__ W) {
+  constexpr int BPW = 32 * NACC;  // probes per workgroup
+  __shared__ __attribute__((aligned(16))) float Vs[2][BPW * LDU];
+  const int t = threadIdx.x;
+  const int lane = t & 63, wave = t >> 6, r = lane & 31, h = lane >> 5;
+  const int64_t i0w = int64_t(blockIdx.x) * BI + 32 * wave;
+  const int64_t row = i0w + r;
+  const int64_t p0 = int64_t(blockIdx.y) * BPW;
+  const int64_t all_tiles = (n + BK - 1) / BK;
+  const int64_t kt_begin = all_tiles * blockIdx.z / gridDim.z;
+  const int64_t ntiles = all_tiles * (blockIdx.z + 1) / gridDim.z - kt_begin;
+  const int64_t mbase = kt_begin * BK;
+  float* Wout = W + int64_t(blockIdx.z) * P * n;
+
+  // four values from column m of a row of n (zeros past it)
+  auto load4 = [&](const float* base, int64_t m) {
+    if (m + 4 <= n) return load4u(base + m);
+    return make_float4(m + 0 < n ? base[m + 0] : 0.f, m + 1 < n ? base[m + 1] : 0.f,
+                       m + 2 < n ? base[m + 2] : 0.f, 0.f);
+  };
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  // probe tile: thread t moves float4 t & 7 of probes t / 8 + 32 u
+  float4 vreg[NACC], an[4], ac[4];
+  auto load_v = [&](int64_t m0) {
+#pragma unroll
+    for (int u = 0; u < NACC; ++u) {
+      const int64_t p = p0 + (t >> 3) + 32 * u;
+      vreg[u] = p < P ? load4(V + p * n, m0 + 4 * (t & 7)) : zero;
+    }
+  };
+  auto store_v = [&](int buf) {
+#pragma unroll
+    for (int u = 0; u < NACC; ++u)
+      *reinterpret_cast<float4*>(&Vs[buf][((t >> 3) + 32 * u) * LDU + 4 * (t & 7)]) = vreg[u];
+  };
+  // the lane's 16 values A[row][m0 + 16 h + 0 .. 15]
+  auto load_a = [&](int64_t m0) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) an[g] = row < n ? load4(A + row * n, m0 + 16 * h + 4 * g) : zero;
+  };
+
+  floatx16 acc[NACC];
+#pragma unroll
+  for (int c = 0; c < NACC; ++c)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[c][e] = 0.f;
+  load_v(mbase);
+  store_v(0);
+  load_a(mbase);
+  __syncthreads();
+  for (int64_t kt = 0; kt < ntiles; ++kt) {
+    const int buf = int(kt & 1);
+    const int64_t m0 = mbase + kt * BK;
+    const bool more = kt + 1 < ntiles;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) ac[g] = an[g];
+    if (more) {
+      load_v(m0 + BK);
+      load_a(m0 + BK);
+    }
+    floatx16 tmp[NACC];
+#pragma unroll
+    for (int c = 0; c < NACC; ++c)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) tmp[c][e] = 0.f;
+    const float* vb = Vs[buf] + r * LDU + 16 * h;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float a[4] = {ac[g].x, ac[g].y, ac[g].z, ac[g].w};
+#pragma unroll
+      for (int c = 0; c < NACC; ++c) {
+        const float4 v4 = *reinterpret_cast<const float4*>(vb + 32 * c * LDU + 4 * g);
+        const float b[4] = {v4.x, v4.y, v4.z, v4.w};
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          tmp[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u], b[u], tmp[c], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < NACC; ++c)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[c][e] += tmp[c][e];
+    if (more) store_v(buf ^ 1);
+    __syncthreads();
+  }
+  store_out<NACC, false, false>(Wout, V, P, n, i0w, p0, acc, 0.f);
+}
+
 // RBF exponents for the BF16 kernels.  The base-2 exponent of a 32 x 32 tile,
 //   arg[m][i] = c |x_m|^2 + c |x_i|^2 + sum_d x_m,d (-2c x_i,d),
 // is a short sum of products of FP32 numbers.  Each factor f is split into
@@ -2683,6 +2786,7 @@ bool packed_op(const slq_operator& op) {
   return op.kind == SLQ_OP_DENSE && op.storage != SLQ_STORE_FP32;
 }
 bool fp32_op(const slq_operator& op) { return op.precision == SLQ_PREC_FP32 && !packed_op(op); }
+bool fp32_units_op(const slq_operator& op) { return op.precision == kPrecFp32Units; }
 
 // Floats of the FP32 matvec's three BF16 planes of `probes` (padded) probes.
 int64_t f32_plane_floats(int64_t npad, int64_t probes) { return 3 * npad * probes / 2; }
@@ -2706,7 +2810,7 @@ int64_t matvec_scratch_floats(const slq_operator& op, int64_t P, bool lean) {
   // the FP32 matvec takes a third plane (for up to 32 probes it fits the
   // records' place)
   int64_t planes = z.Ppad * z.npad + 16 * z.npad;
-  if (!lean && fp32_op(op) && !rows_kernel(op, P)) {
+  if (!lean && (fp32_op(op) || fp32_units_op(op)) && !rows_kernel(op, P)) {
     const int64_t three = f32_plane_floats(z.npad, z.Ppad);
     if (three > planes) planes = three;
   }
@@ -2715,7 +2819,7 @@ int64_t matvec_scratch_floats(const slq_operator& op, int64_t P, bool lean) {
 
 PlaneOut matvec_planes(const slq_operator& op, int64_t P, float* scratch, int64_t scratch_floats) {
   PlaneOut out;
-  if (rows_kernel(op, P) || !scratch) return out;
+  if (rows_kernel(op, P) || fp32_units_op(op) || !scratch) return out;
   const PlaneSizes z(op.n, P);
   if (fp32_op(op)) {
     // with less scratch the launch splits groups of probes by itself
@@ -2824,7 +2928,22 @@ hipError_t launch_matvec(hipStream_t s, const slq_operator& op, const float* V, 
   }
   float* partial = nullptr;
   int S = 1;
-  if (fp32) {
+  if (fp32_units_op(op)) {
+    partial = scratch;
+    S = choose_splitk(n, P, scratch_floats, true);
+    const int nacc = nacc_for(P);
+    const dim3 grid(unsigned((n + BI - 1) / BI), unsigned((P + 32 * nacc - 1) / (32 * nacc)),
+                    unsigned(S));
+    float* out = S > 1 ? partial : W;
+    if (ev0) (void)hipEventRecord(ev0, s);
+    if (nacc == 1)
+      hipLaunchKernelGGL(k_matvec_f32_units<1>, grid, dim3(kThreads), 0, s, op.matrix, V, P, n, out);
+    else if (nacc == 2)
+      hipLaunchKernelGGL(k_matvec_f32_units<2>, grid, dim3(kThreads), 0, s, op.matrix, V, P, n, out);
+    else
+      hipLaunchKernelGGL(k_matvec_f32_units<4>, grid, dim3(kThreads), 0, s, op.matrix, V, P, n, out);
+    err = hipGetLastError();
+  } else if (fp32) {
     // scratch layout: [three BF16 planes of a group of probes][split-K
     // partial sums].  The group is every probe unless the scratch is the lean
     // size, where the planes of a part of them fit at a time; a probe's

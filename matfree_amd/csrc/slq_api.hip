@@ -681,7 +681,7 @@ int arnoldi_reverse(slq_context* ctx, const slq_operator& op, int64_t P, int64_t
   // at a time as the partial dots dQ_i^T Q fit in Lambda's place (not yet in
   // use) and a grid takes; one if the rows of dQ differ in alignment
   const int64_t prow = P * nb * pstride;
-  const int64_t fit = std::min<int64_t>(std::min<int64_t>(k * ldc / prow, k), 65535);
+  const int64_t fit = std::min<int64_t>(std::min<int64_t>(k * ldc / prow, k), max_dot_rows(k));
   const int64_t group = ldq % 4 == 0 || !dQ ? fit : 1;
   for (int64_t i = 0; i < k; i += group) {
     const int64_t rows = std::min(group, k - i);
@@ -1058,7 +1058,11 @@ int slq_arnoldi_vjp(slq_context* ctx, const slq_operator* op, const float* V0, i
   SLQ_TRY(ensure_t(ctx, ctx->hmat, size_t(P * k * k), &st.H));
   SLQ_TRY(ensure_t(ctx, ctx->resid, size_t(P * n), &st.R));
   SLQ_TRY(ensure_t(ctx, ctx->scal1, size_t(P), &st.c));
-  SLQ_TRY(hessenberg_core(ctx, *op, V0, P, k, st.Q, st.ldc, st.H, st.R, st.c, reortho != 0));
+  // the cotangents move with the basis's rounding: see k_matvec_f32_units
+  slq_operator fwd = *op;
+  if (op->kind == SLQ_OP_DENSE && op->storage == SLQ_STORE_FP32 && op->precision == SLQ_PREC_FP32)
+    fwd.precision = kPrecFp32Units;
+  SLQ_TRY(hessenberg_core(ctx, fwd, V0, P, k, st.Q, st.ldc, st.H, st.R, st.c, reortho != 0));
   Timed tm(ctx, SLQ_KC_ADJOINT);
   return arnoldi_reverse(ctx, *op, P, k, st, reortho_adjoint != 0, dQ, dH, dr, dc, dv, dparams,
                          dmatrix);

@@ -81,7 +81,9 @@ struct MvSplitSum {
 // Basis column c of probe p starts at Q + c * ldc + p * n (ldc >= P * n).
 // partial[p][b][c] = sum_{i in chunk b} Q[c][p][i] * x[p][i], c < ncols.
 // Q may be null with ncols = 1 to mean "sum of squares of x" (partial[p][b][0]).
-// rows: the same for that many blocks x + i * xrow, into partial + i * prow.
+// rows (up to max_dot_rows): the same for that many blocks x + i * xrow, into
+// partial + i * prow.
+int64_t max_dot_rows(int64_t ncols);
 hipError_t launch_dots(hipStream_t s, const float* Q, int64_t ldc, const float* x, int64_t P,
                        int64_t n, int ncols, float* partial, int pstride, int64_t rows = 1,
                        int64_t xrow = 0, int64_t prow = 0);
@@ -186,6 +188,10 @@ int64_t matvec_scratch_floats(const slq_operator& op, int64_t P, bool lean = fal
 // PlaneOut producer after a call that split them, so the padding is zero);
 // kMvPointsReady -- the RBF point records in the scratch are those of op
 // (a previous call with the same operator and scratch).
+// An internal precision of a stored FP32 matrix: the products on the FP32
+// matrix cores (k_matvec_f32_units), for the forward pass a reverse pass is
+// taken at.
+constexpr int32_t kPrecFp32Units = -1;
 constexpr int kMvPlanesReady = 1;
 constexpr int kMvPointsReady = 2;
 // With defer non-null a split-K result is not reduced into W; *defer
