@@ -903,6 +903,172 @@ __global__ void __launch_bounds__(kStreamThreads)
   }
 }
 
+// ---------------------------------------------------------------------------
+// A whole Gram-Schmidt step of one probe in one workgroup, for rows of one
+// chunk (n <= kChunk): the dots, the projection, the second pass, the norm and
+// the normalisation, with the vector and the coefficients in LDS.  Such steps
+// are bound by the latency of each kernel's load - reduce - store chain and by
+// the launches around it, not by bytes.  The waves are four sets of 256
+// threads; a column's dot is one set's (as a k_dots / k_project_dots block: the
+// same elements per thread, the same tree, so rows of whole float4 groups give
+// the same bits), the projection gives each thread two elements.  Decomposition
+// of a stored matrix, with a launch per pass before: n = 1001, 16 probes, 20
+// steps 487 -> 385 us, n = 2048, 256 probes, 40 steps 2730 -> 2400.  (512
+// threads with the next pass's columns loaded a barrier ahead: within 3%
+// either way.)
+// ---------------------------------------------------------------------------
+constexpr int kRowThreads = 1024;
+constexpr int kRowSets = kRowThreads / kStreamThreads;
+static_assert(kChunk == 2 * kRowThreads, "two elements of the projection per thread");
+
+// LDS floats of a step with ncols columns: the vector, the coefficients and
+// the dots' sums per wave of a set.
+inline int64_t row_step_floats(int64_t ncols) { return kChunk + (kWaves + 1) * ncols; }
+
+// red[wave of the set][c] = that wave's part of sum_i Q[c][i] ys[i].  V = 4:
+// the elements of k_dots, V = 2: those of k_project_dots.  The last group of a
+// row whose length is no multiple of V is read from n - V on, the elements that
+// another thread has masked.
+template <int V>
+__device__ __forceinline__ void row_dots(const float* __restrict__ qp, int64_t ldc, int n,
+                                         int ncols, const float* ys, float* red) {
+  constexpr int NE = Layout<V>::NE;
+  constexpr int CB = kColBatch;
+  const int t = threadIdx.x, lane = t & 63, set = t / kStreamThreads;
+  const int st = t % kStreamThreads, swave = st >> 6;
+  int off[NE];
+  float xv[NE][V];
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const int i = (e * kStreamThreads + st) * V;
+    off[e] = i < n - V ? i : n - V;
+#pragma unroll
+    for (int v = 0; v < V; ++v) xv[e][v] = i < n && off[e] + v >= i ? ys[off[e] + v] : 0.f;
+  }
+  for (int c0 = CB * set; c0 < ncols; c0 += CB * kRowSets) {
+    float qv[CB][NE][V];
+#pragma unroll
+    for (int u = 0; u < CB; ++u) {
+      const float* q = qp + int64_t(c0 + u < ncols ? c0 + u : ncols - 1) * ldc;
+#pragma unroll
+      for (int e = 0; e < NE; ++e) __builtin_memcpy(qv[u][e], q + off[e], sizeof(qv[u][e]));
+    }
+    float acc[CB];
+#pragma unroll
+    for (int u = 0; u < CB; ++u) {
+      acc[u] = 0.f;
+#pragma unroll
+      for (int e = 0; e < NE; ++e)
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[u] = fmaf(qv[u][e][v], xv[e][v], acc[u]);
+    }
+    ReduceScatter<CB, 32>::run(acc, lane);
+    constexpr int shift = 6 - log2i(CB);
+    const int c = c0 + (lane >> shift);
+    if ((lane & ((1 << shift) - 1)) == 0 && c < ncols) red[swave * ncols + c] = acc[0];
+  }
+}
+
+// ys -= sum_c Q[c] hs[c], the columns added in order.
+__device__ __forceinline__ void row_project(const float* __restrict__ qp, int64_t ldc, int n,
+                                            int ncols, const float* hs, float* ys) {
+  constexpr int CB = 2 * kColBatch;
+  const int i = 2 * threadIdx.x;
+  if (i >= n) return;
+  const int off = i < n - 2 ? i : n - 2;
+  float s[2] = {0.f, 0.f};
+  for (int c0 = 0; c0 < ncols; c0 += CB) {
+    float qv[CB][2];
+#pragma unroll
+    for (int u = 0; u < CB; ++u)
+      __builtin_memcpy(qv[u], qp + int64_t(c0 + u < ncols ? c0 + u : ncols - 1) * ldc + off,
+                       sizeof(qv[u]));
+#pragma unroll
+    for (int u = 0; u < CB; ++u) {
+      if (c0 + u >= ncols) break;
+      const float hc = hs[c0 + u];
+#pragma unroll
+      for (int v = 0; v < 2; ++v) s[v] = fmaf(qv[u][v], hc, s[v]);
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < 2; ++v)
+    if (off + v >= i) ys[off + v] -= s[v];
+}
+
+__global__ void __launch_bounds__(kRowThreads)
+    k_row_step(const float* __restrict__ Q, int64_t ldc, int n, int ncols, RowStep st) {
+  extern __shared__ float lds[];
+  float* ys = lds;
+  float* hs = lds + kChunk;
+  float* red = hs + ncols;
+  const int64_t p = blockIdx.x;
+  const int t = threadIdx.x, lane = t & 63;
+  const float* qp = Q + p * n;
+
+  // the input, a deferred split-K sum where the product left one
+  for (int i = t; i < n; i += kRowThreads) {
+    if (st.sum.partial) {
+      const int64_t off[1] = {p * n + i};
+      float v[1][1];
+      split_sum<1, 1>(st.sum, int64_t(gridDim.x) * n, off, v);
+      ys[i] = v[0][0];
+    } else {
+      ys[i] = st.x[p * n + i];
+    }
+  }
+  __syncthreads();
+  auto coefficients = [&](float* hout, const float* hsub) {
+    __syncthreads();
+    for (int c = t; c < ncols; c += kRowThreads) {
+      float s = 0.f;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) s += red[w * ncols + c];
+      if (hout) hout[c] = s;
+      if (hsub) s -= hsub[c];
+      hs[c] = s;
+    }
+    __syncthreads();
+  };
+  row_dots<4>(qp, ldc, n, ncols, ys, red);
+  coefficients(st.hout ? st.hout + p * st.hout_stride : nullptr,
+               st.hsub ? st.hsub + p * st.hsub_stride : nullptr);
+  row_project(qp, ldc, n, ncols, hs, ys);
+  __syncthreads();
+  if (st.second) {
+    row_dots<2>(qp, ldc, n, ncols, ys, red);
+    coefficients(nullptr, nullptr);
+    row_project(qp, ldc, n, ncols, hs, ys);
+    __syncthreads();
+  }
+  float len = 1.f;
+  if (st.normalize) {
+    if (t < kStreamThreads) {
+      float acc = 0.f;
+#pragma unroll
+      for (int e = 0; e < Layout<4>::NE; ++e)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int i = (e * kStreamThreads + t) * 4 + v;
+          if (i < n) acc = fmaf(ys[i], ys[i], acc);
+        }
+      acc = wave_sum(acc);
+      if (lane == 0) red[t >> 6] = acc;
+    }
+    __syncthreads();
+    float s = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) s += red[w];
+    len = sqrtf(s);
+    if (t == 0 && st.hslot) st.hslot[p * st.hout_stride] = len;
+  }
+  for (int i = t; i < n; i += kRowThreads) {
+    const float v[1] = {st.normalize ? ys[i] / len : ys[i]};
+    st.out[p * n + i] = v[0];
+    if (st.planes.hi) store_planes<1>(st.planes, p, i, v);
+  }
+}
+
 inline bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 
 // Vector width of the streaming kernels for rows of n floats at these
@@ -990,6 +1156,19 @@ hipError_t launch_dots_sum(hipStream_t s, const float* Q, int64_t ldc, const MvS
                            float* x, int64_t P, int64_t n, int ncols, float* partial, int pstride) {
   return launch_dots_any<true>(s, Q, ldc, nullptr, x, sum, P, n, ncols, partial, pstride, 1, 0, 0,
                                {x, Q, sum.partial, sum.nugget ? sum.V : x});
+}
+
+bool row_step_ok(int64_t P, int64_t n, int64_t ncols) {
+  return n >= 4 && n <= kChunk && ncols >= 1 && row_step_floats(ncols) * 4 <= 64 * 1024;
+}
+
+hipError_t launch_row_step(hipStream_t s, const float* Q, int64_t ldc, int64_t P, int64_t n,
+                           int ncols, const RowStep& step) {
+  if (!row_step_ok(P, n, ncols)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_row_step, dim3(unsigned(P)), dim3(kRowThreads),
+                     size_t(row_step_floats(ncols)) * sizeof(float), s, Q, ldc, int(n), ncols,
+                     step);
+  return hipGetLastError();
 }
 
 hipError_t launch_project(hipStream_t s, const float* Q, int64_t ldc, const float* x, float* y,

@@ -294,6 +294,24 @@ int hessenberg_core(slq_context* ctx, const slq_operator& op, const float* V0, i
       SLQ_HIP(ctx, launch_matvec(s, op, qj, P, w, mvs, mv_floats, ev.first, ev.second, flags,
                                  &pend));
     }
+    const bool last = (j + 1 == k);
+    float* dst = last ? R : w;
+    if (row_step_ok(P, n, ncols)) {
+      // all of decomp.py:463-475 (and the next step's :456-457) in one launch
+      Timed tm(ctx, SLQ_KC_PROJECT_DOTS);
+      RowStep st;
+      st.x = w;
+      st.sum = pend;
+      st.hout = hcol;
+      st.hout_stride = k * k;
+      st.second = reortho;
+      st.normalize = !last;
+      st.hslot = last ? nullptr : hcol + j + 1;
+      st.out = last ? R : Q + (j + 1) * ldc;
+      if (!last) st.planes = planes;
+      SLQ_HIP(ctx, launch_row_step(s, Q, ldc, P, n, ncols, st));
+      continue;
+    }
     // h = Q^T w (decomp.py:463)
     {
       Timed tm(ctx, SLQ_KC_DOTS);
@@ -302,8 +320,6 @@ int hessenberg_core(slq_context* ctx, const slq_operator& op, const float* V0, i
       else
         SLQ_HIP(ctx, launch_dots(s, Q, ldc, w, P, n, ncols, part1, pstride));
     }
-    const bool last = (j + 1 == k);
-    float* dst = last ? R : w;
     if (!reortho) {
       // w = w - Q h and <w, w> (decomp.py:464, 471), h into H[:, j]
       {
@@ -562,6 +578,25 @@ struct AdjointMatvec {
   }
 };
 
+// lam2 = lam - Q (Q^T lam - hsub) (decomp.py:576-584) and its planes.
+hipError_t adjoint_reortho(hipStream_t s, const float* Q, int64_t ldc, const float* lam,
+                           float* lam2, int64_t P, int64_t n, int ncols, float* part, int pstride,
+                           const float* hsub, int64_t hsub_stride, const PlaneOut* planes) {
+  if (row_step_ok(P, n, ncols)) {
+    RowStep st;
+    st.x = lam;
+    st.hsub = hsub;
+    st.hsub_stride = hsub_stride;
+    st.out = lam2;
+    if (planes) st.planes = *planes;
+    return launch_row_step(s, Q, ldc, P, n, ncols, st);
+  }
+  const hipError_t e = launch_dots(s, Q, ldc, lam, P, n, ncols, part, pstride);
+  if (e != hipSuccess) return e;
+  return launch_project(s, Q, ldc, lam, lam2, P, n, ncols, part, pstride, nullptr, nullptr, 0,
+                        hsub, hsub_stride, planes);
+}
+
 // The reverse pass: cotangent of the probe mean w.r.t. H (eigh VJP), the
 // Arnoldi adjoint recursion (decomp.py:480-600, reortho="full"), and the
 // operator parameters' cotangents (the matvec VJPs of decomp.py:587-589).
@@ -601,9 +636,8 @@ int logdet_reverse(slq_context* ctx, const slq_operator& op, int64_t P, int64_t 
   for (int64_t idx = k - 1; idx >= 0; --idx) {
     // lambda -= Q_m (Q_m^T lambda - dH[:, idx]_m), columns j <= idx + 1 (decomp.py:576-584)
     const int ncols = int(idx + 2 < k ? idx + 2 : k);
-    SLQ_HIP(ctx, launch_dots(s, st.Q, ldc, lam, P, n, ncols, part1, pstride));
-    SLQ_HIP(ctx, launch_project(s, st.Q, ldc, lam, lam2, P, n, ncols, part1, pstride, nullptr,
-                                nullptr, 0, dH + idx * k, k * k, mv.planes_out()));
+    SLQ_HIP(ctx, adjoint_reortho(s, st.Q, ldc, lam, lam2, P, n, ncols, part1, pstride,
+                                 dH + idx * k, k * k, mv.planes_out()));
     // A^T lambda (decomp.py:587-588; A symmetric) and Q^T (A^T lambda) for
     // Gamma[idx, :] (decomp.py:592-593)
     SLQ_HIP(ctx, mv.run(s, lam2, vm, st.Q, ldc, int(idx + 1), part2, pstride, true));
@@ -704,9 +738,8 @@ int arnoldi_reverse(slq_context* ctx, const slq_operator& op, int64_t P, int64_t
     if (adj_reortho) {
       // lambda -= Q_m (Q_m^T lambda - dH[:, idx]_m), columns j <= idx + 1
       const int ncols = int(idx + 2 < k ? idx + 2 : k);
-      SLQ_HIP(ctx, launch_dots(s, st.Q, ldc, lam, P, n, ncols, part1, pstride));
-      SLQ_HIP(ctx, launch_project(s, st.Q, ldc, lam, lam2, P, n, ncols, part1, pstride, nullptr,
-                                  nullptr, 0, dH + idx * k, k * k, mv.planes_out()));
+      SLQ_HIP(ctx, adjoint_reortho(s, st.Q, ldc, lam, lam2, P, n, ncols, part1, pstride,
+                                   dH + idx * k, k * k, mv.planes_out()));
       lin = lam2;
     }
     // A^T lambda (decomp.py:587-588; A symmetric) and Q^T (A^T lambda) for

@@ -105,6 +105,27 @@ hipError_t launch_project(hipStream_t s, const float* Q, int64_t ldc, const floa
 hipError_t launch_project_dots(hipStream_t s, const float* Q, int64_t ldc, const float* x,
                                float* y, int64_t P, int64_t n, int ncols, const float* h1part,
                                float* h2part, int pstride, float* hout, int64_t hout_stride);
+// A Gram-Schmidt step of rows of one chunk in one launch: y = x - Q h with
+// h = Q^T x - hsub, and with `second` y -= Q (Q^T y); out = y, or y / |y| with
+// `normalize`.  x is the deferred split-K sum where sum.partial is non-null.
+// hout[p * hout_stride + c] (optional) receives Q^T x, hslot[p * hout_stride]
+// (optional) |y|, planes the planes of out.
+struct RowStep {
+  const float* x = nullptr;
+  MvSplitSum sum;
+  float* hout = nullptr;
+  int64_t hout_stride = 0;
+  const float* hsub = nullptr;
+  int64_t hsub_stride = 0;
+  int second = 0;
+  int normalize = 0;
+  float* hslot = nullptr;
+  float* out = nullptr;
+  PlaneOut planes;
+};
+bool row_step_ok(int64_t P, int64_t n, int64_t ncols);
+hipError_t launch_row_step(hipStream_t s, const float* Q, int64_t ldc, int64_t P, int64_t n,
+                           int ncols, const RowStep& step);
 // out[p][i] = x[p][i] / sqrt(sum_b norm2part[p][b]); optionally writes the
 // norm to norm_out[p] (float), to hslot[p * hslot_stride] and
 // hslot2[p * hslot_stride], and its reciprocal to inv_out[p].
