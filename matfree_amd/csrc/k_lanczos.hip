@@ -435,6 +435,13 @@ __device__ __forceinline__ int plane_group(int c4, int perm) {
 template <int V>
 __device__ __forceinline__ void store_planes(const PlaneOut& pl, int64_t p, int64_t i,
                                              const float (&v)[V]) {
+  if (pl.three == 2) {
+    // the stream form's tiles (k_tile_probes); i % V == 0, one group of four
+    float* dst = reinterpret_cast<float*>(pl.hi) +
+                 (((i / 32) * 4 + ((i >> 2) & 3)) * 64 + p + 32 * ((i >> 4) & 1)) * 4 + (i & 3);
+    VecIO<V>::store(dst, v);
+    return;
+  }
   if (pl.three) {
     // the FP32 matvec's planes: 8 columns of a probe per 16-byte word
     // (k_split3_probes); i % V == 0, so a group lies in one word

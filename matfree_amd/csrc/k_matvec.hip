@@ -1104,6 +1104,22 @@ __global__ void __launch_bounds__(kThreads, 3)
   });
 }
 
+// The probes (up to 32) in the order of the stream form's B fragments, zero past
+// n and P: tile kt, group g, lane (r, h) holds columns 32 kt + 16 h + 4 g .. + 3
+// of probe r.  One thread per group of four.
+__global__ void __launch_bounds__(256)
+    k_tile_probes(const float* __restrict__ V, int64_t P, int64_t n, int64_t npad,
+                  float4* __restrict__ tiles) {
+  const int64_t w = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (w >= npad * 8) return;
+  const int64_t r = w & 31;
+  const int64_t m = (w >> 8) * 32 + 16 * ((w >> 5) & 1) + 4 * ((w >> 6) & 3);
+  float v[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) v[u] = r < P && m + u < n ? V[r * n + m + u] : 0.f;
+  tiles[w] = make_float4(v[0], v[1], v[2], v[3]);
+}
+
 // Stream form, for a stored matrix and up to 32 probes: the matrix's bytes are
 // the bound, and with one probe block per entry the FP32 matrix cores (1024
 // cycles a tile) keep up with HBM while splitting the entries for the BF16
@@ -1115,13 +1131,20 @@ __global__ void __launch_bounds__(kThreads, 3)
 // loader keeps up to 64 KB per workgroup in flight (two workgroups fill the
 // CU's LDS).  A row's piece of a block is 512 contiguous bytes: unaligned rows
 // read in the 128-byte rows of a tile reach 4.2 TB/s, in these pieces 4.9.
+// TILED: the vectors in the order of the fragments (k_tile_probes).  A lane's own
+// row in 16-byte pieces touches 32 rows an instruction, which the L1 takes one
+// at a time.  Decomposition of depth 8 with 32 probes, without: n = 10413 1108 ->
+// 1060 us, 15001 1927 -> 1766, 16384 2024 -> 1941; a single product 222 -> 212 us
+// at 15001.
 // Whole calls with 32 probes, each wave loading its own rows before: n = 10413
 // 149 -> 117 us, 15001 271 -> 216, 4096 23.6 -> 19.7, 16384 225 -> 232 us.
 constexpr int kStreamWaves = 5;
 constexpr int kStreamStages = 5;
+template <bool TILED>
 __global__ void __launch_bounds__(64 * kStreamWaves, 3)
-    k_matvec_f32_stream(const float* __restrict__ A, const float* __restrict__ V, int64_t P,
-                        int64_t n, float* __restrict__ W, int64_t wstride) {
+    k_matvec_f32_stream(const float* __restrict__ A, const float4* __restrict__ tiles,
+                        const float* __restrict__ V, int64_t P, int64_t n, float* __restrict__ W,
+                        int64_t wstride) {
   constexpr int kBlockTiles = 4;
   __shared__ __attribute__((aligned(16))) float4 as[kStreamStages * 1024];
   const int t = threadIdx.x;
@@ -1194,7 +1217,8 @@ __global__ void __launch_bounds__(64 * kStreamWaves, 3)
     const float* vrow = V + (r < P ? r : P - 1) * n + kt_begin * BK + 16 * h;
     auto load_v = [&](int64_t kt, float4 (&v)[4]) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) v[g] = load4u(vrow + kt * BK + 4 * g);
+      for (int g = 0; g < 4; ++g)
+        v[g] = TILED ? tiles[((kt_begin + kt) * 4 + g) * 64 + lane] : load4u(vrow + kt * BK + 4 * g);
     };
     auto tile_products = [&](const float4 (&a)[4], const float4 (&v)[4]) {
       floatx16 tmp;
@@ -2535,6 +2559,15 @@ bool f32_planes(int64_t n, int64_t P, bool rbf) {
   return nacc_for(P) > 1 || (rbf && n >= 4096);
 }
 
+// Whether the stream form takes the probes in the order of its fragments
+// (k_tile_probes; written by the producer of the input where there is one, in a
+// launch of about 3.5 us otherwise).  With up to 16 probes most of a tile is
+// padding, and its lines cost more than the rows' (15001, 16 probes: 199 -> 208
+// us); up to n = 8400 the launch costs what the tiles save.
+bool stream_tiles(int64_t n, int64_t P, bool rbf) {
+  return !rbf && nacc_for(P) == 1 && n > 8960 && P > 24;
+}
+
 // The FP32 matvec of P vectors (a group of the launch's probes) from planes
 // of npb blocks of 32 probes; out: W, or the first of S partial planes of
 // wstride floats.
@@ -2547,9 +2580,15 @@ hipError_t launch_f32(hipStream_t s, const float* A, const RBFParams& prm, const
                   unsigned(S));
   if (nacc == 1) {
     const dim3 wgrid(unsigned((n + 31) / 32), 1, unsigned(S));
-    if constexpr (!RBF)
-      hipLaunchKernelGGL(k_matvec_f32_stream, wgrid, dim3(64 * kStreamWaves), 0, s, A, V, P, n,
-                         out, wstride);
+    if constexpr (!RBF) {
+      const float4* tiles = reinterpret_cast<const float4*>(planes);
+      if (stream_tiles(n, P, false))
+        hipLaunchKernelGGL(k_matvec_f32_stream<true>, wgrid, dim3(64 * kStreamWaves), 0, s, A,
+                           tiles, V, P, n, out, wstride);
+      else
+        hipLaunchKernelGGL(k_matvec_f32_stream<false>, wgrid, dim3(64 * kStreamWaves), 0, s, A,
+                           tiles, V, P, n, out, wstride);
+    }
     else if (f32_planes(n, P, true))
       hipLaunchKernelGGL((k_matvec_f32_wave<DIM, true>), wgrid, dim3(kThreads), 0, s, prm, planes,
                          plane_words, V, P, n, out, wstride);
@@ -2823,13 +2862,14 @@ PlaneOut matvec_planes(const slq_operator& op, int64_t P, float* scratch, int64_
   const PlaneSizes z(op.n, P);
   if (fp32_op(op)) {
     // with less scratch the launch splits groups of probes by itself
-    if (!f32_planes(op.n, P, op.kind == SLQ_OP_RBF)) return out;
+    const bool rbf = op.kind == SLQ_OP_RBF, tiled = stream_tiles(op.n, P, rbf);
+    if (!f32_planes(op.n, P, rbf) && !tiled) return out;
     const int64_t S = choose_splitk_f32(op.n, P, op.kind == SLQ_OP_RBF);
     if (f32_plane_floats(z.npad, z.Ppad) + S * P * op.n > scratch_floats) return out;
     out.Ppad = z.Ppad;
     out.hi = reinterpret_cast<__bf16*>(scratch);
     out.plane = z.Ppad * z.npad;
-    out.three = 1;
+    out.three = tiled ? 2 : 1;
     return out;
   }
   out.Ppad = z.Ppad;
@@ -2958,7 +2998,9 @@ hipError_t launch_matvec(hipStream_t s, const slq_operator& op, const float* V, 
     }
     u32x4* planes = reinterpret_cast<u32x4*>(scratch);
     partial = scratch + f32_plane_floats(npad, group);
-    const bool ready = !f32_planes(n, P, op.kind == SLQ_OP_RBF) || ((flags & kMvPlanesReady) && group == Ppad);
+    const bool rbf = op.kind == SLQ_OP_RBF, tiled = stream_tiles(n, P, rbf);
+    const bool ready =
+        !(f32_planes(n, P, rbf) || tiled) || ((flags & kMvPlanesReady) && group == Ppad);
     if (ready && ev0) (void)hipEventRecord(ev0, s);
     for (int64_t p0 = 0; p0 < P && err == hipSuccess; p0 += group) {
       const int64_t Pg = P - p0 < group ? P - p0 : group;
@@ -2967,8 +3009,12 @@ hipError_t launch_matvec(hipStream_t s, const slq_operator& op, const float* V, 
       if (!ready) {
         int64_t blocks = (words + 255) / 256;
         if (blocks > 8192) blocks = 8192;
-        hipLaunchKernelGGL(k_split3_probes, dim3(unsigned(blocks)), dim3(256), 0, s, V + p0 * n,
-                           Pg, n, zg.Ppad / 32, words, planes);
+        if (tiled)
+          hipLaunchKernelGGL(k_tile_probes, dim3(unsigned((npad * 8 + 255) / 256)), dim3(256), 0, s,
+                             V, P, n, npad, reinterpret_cast<float4*>(planes));
+        else
+          hipLaunchKernelGGL(k_split3_probes, dim3(unsigned(blocks)), dim3(256), 0, s, V + p0 * n,
+                             Pg, n, zg.Ppad / 32, words, planes);
         if ((err = hipGetLastError()) != hipSuccess) break;
         if (p0 == 0 && ev0) (void)hipEventRecord(ev0, s);
       }

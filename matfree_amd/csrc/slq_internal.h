@@ -61,7 +61,8 @@ struct PlaneOut {
   int64_t Ppad = 0;
   int perm = 0;  // RBF fragment order of the columns within a tile
   // three: the FP32 matvec's planes instead (x = hi + mid + lo, `plane`
-  // elements apart, in the fragment order of k_split3_probes)
+  // elements apart, in the fragment order of k_split3_probes); 2: FP32 values
+  // in the order of k_tile_probes
   int three = 0;
   int64_t plane = 0;
 };

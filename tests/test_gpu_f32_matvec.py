@@ -110,3 +110,25 @@ def test_least_scratch_gives_the_same_results(cuda):
         out.append(per.cpu().numpy())
     del keep
     np.testing.assert_array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("n,P", [(8961, 25), (8963, 32), (9024, 31), (10413, 32)])
+def test_probe_tiles_of_the_stream_form(cuda, n, P):
+    # vectors read in the order of the fragments: the first row that takes it, no whole last
+    # tile, and the tiles written by the normalisation (the three vectors' relation
+    # A q_j = Q h_j, whose last columns have few terms: 2e-6 as for the product)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    A = torch.randn((n, n), generator=gen, device="cuda")
+    A = (A + A.T) / (2 * n) ** 0.5
+    V = torch.randn((P, n), generator=gen, device="cuda")
+    A64 = A.double()
+    W = operators.dense_matvec(V, A)
+    assert rel(W, (V.double() @ A64).cpu().numpy()) < 2e-6
+    out = decomp.hessenberg(3, reortho="full").batched(operators.dense_matvec, V, A)
+    Q, H = out.Q_tall.double(), out.J_small.double()
+    if Q.shape[1] != 3:
+        Q = Q.transpose(1, 2)
+    image = H.transpose(1, 2) @ Q
+    image[:, -1] += out.residual.double()
+    for j in range(3):
+        assert rel(image[:, j], (Q[:, j] @ A64).cpu().numpy()) < 2e-6
