@@ -200,25 +200,30 @@ inline int dots_columns(int64_t blocks, int ncols) {
   return blocks < kManyBlocks || ncols <= 8 ? 8 : ncols <= 16 ? 16 : 32;
 }
 
+// Probe of a block: in order, or back (see launch_dots).
+__device__ __forceinline__ int64_t probe_of(unsigned i, unsigned count, int back) {
+  return back ? count - 1 - i : i;
+}
+
 // SUM: x is the deferred split-K sum `sm`, stored to xw by the blocks of
-// column group 0.  blockIdx.z = row * column groups + column group; row i reads
+// column group 0.  blockIdx.y = row * column groups + column group; row i reads
 // x + i xrow and writes partial + i prow.
 template <int V, int NC, bool SUM>
 __global__ void __launch_bounds__(kStreamThreads)
     k_dots(const float* __restrict__ Q, int64_t ldc, const float* __restrict__ x, float* xw,
            int64_t n, int ncols, float* __restrict__ partial, int pstride, int64_t xrow,
-           int64_t prow, MvSplitSum sm) {
+           int64_t prow, MvSplitSum sm, int back) {
   constexpr int NE = Layout<V>::NE;
   constexpr int CB = kColBatch;
   __shared__ float red[kWaves * NC];
-  const int64_t p = blockIdx.y;
+  const int64_t p = probe_of(blockIdx.z, gridDim.z, back);
   const int64_t b = blockIdx.x;
   const int64_t nb = gridDim.x;
   const int t = threadIdx.x;
   const int64_t base = b * kChunk;
   const int groups = (ncols + NC - 1) / NC;
-  const int64_t row = blockIdx.z / groups;
-  const int c0 = int(blockIdx.z % groups) * NC;
+  const int64_t row = blockIdx.y / groups;
+  const int c0 = int(blockIdx.y % groups) * NC;
 
   int64_t off[NE];
   bool in[NE];
@@ -241,7 +246,7 @@ __global__ void __launch_bounds__(kStreamThreads)
   load(0);
   float xv[NE][V];
   if constexpr (SUM) {
-    split_sum<V, NE>(sm, int64_t(gridDim.y) * n, off, xv);
+    split_sum<V, NE>(sm, int64_t(gridDim.z) * n, off, xv);
   } else {
 #pragma unroll
     for (int e = 0; e < NE; ++e) VecIO<V>::load(x + row * xrow + off[e], xv[e]);
@@ -307,15 +312,15 @@ template <int NC, bool SUM>
 __global__ void __launch_bounds__(kStreamThreads)
     k_dots_shifted(const float* __restrict__ Q, int64_t ldc, const float* __restrict__ x,
                    float* xw, int64_t n, int ncols, float* __restrict__ partial, int pstride,
-                   int64_t xrow, int64_t prow, MvSplitSum sm) {
+                   int64_t xrow, int64_t prow, MvSplitSum sm, int back) {
   constexpr int NE = Layout<4>::NE;
   constexpr int CB = kColBatch;
   __shared__ float red[kWaves * NC];
-  const int64_t p = blockIdx.y, b = blockIdx.x, nb = gridDim.x;
+  const int64_t p = probe_of(blockIdx.z, gridDim.z, back), b = blockIdx.x, nb = gridDim.x;
   const int t = threadIdx.x;
   const int groups = (ncols + NC - 1) / NC;
-  const int64_t drow = blockIdx.z / groups;
-  const int c0 = int(blockIdx.z % groups) * NC;
+  const int64_t drow = blockIdx.y / groups;
+  const int c0 = int(blockIdx.y % groups) * NC;
   const ShiftedRow row(p, n, b, t);
   int64_t off[NE];
   bool in[NE];
@@ -341,8 +346,8 @@ __global__ void __launch_bounds__(kStreamThreads)
   load(0);
   float xv[NE][4], xh[1][1];
   if constexpr (SUM) {
-    split_sum<4, NE>(sm, int64_t(gridDim.y) * n, off, xv);
-    split_sum<1, 1>(sm, int64_t(gridDim.y) * n, ixo, xh);
+    split_sum<4, NE>(sm, int64_t(gridDim.z) * n, off, xv);
+    split_sum<1, 1>(sm, int64_t(gridDim.z) * n, ixo, xh);
   } else {
     const float* xr = x + drow * xrow;
 #pragma unroll
@@ -501,12 +506,12 @@ __global__ void __launch_bounds__(kStreamThreads)
               float* __restrict__ y, int64_t n, int ncols, const float* __restrict__ hpart,
               int pstride, float* __restrict__ norm2part, float* __restrict__ hout,
               int64_t hout_stride, const float* __restrict__ hsub, int64_t hsub_stride,
-              PlaneOut pl) {
+              int back, PlaneOut pl) {
   constexpr int NE = Layout<V>::NE;
   constexpr int CB = kColBatch;
   extern __shared__ float hs[];
   __shared__ float red[kWaves];
-  const int64_t p = blockIdx.y, b = blockIdx.x, nb = gridDim.x;
+  const int64_t p = probe_of(blockIdx.y, gridDim.y, back), b = blockIdx.x, nb = gridDim.x;
   const int t = threadIdx.x;
   const int64_t base = b * kChunk;
   float s[NE][V];
@@ -609,12 +614,13 @@ __global__ void __launch_bounds__(kStreamThreads)
                       float* __restrict__ y, int64_t n, int ncols,
                       const float* __restrict__ hpart, int pstride,
                       float* __restrict__ norm2part, float* __restrict__ hout,
-                      int64_t hout_stride, const float* __restrict__ hsub, int64_t hsub_stride) {
+                      int64_t hout_stride, const float* __restrict__ hsub, int64_t hsub_stride,
+                      int back) {
   constexpr int NE = Layout<4>::NE;
   constexpr int CB = kColBatch;
   extern __shared__ float hs[];
   __shared__ float red[kWaves];
-  const int64_t p = blockIdx.y, b = blockIdx.x, nb = gridDim.x;
+  const int64_t p = probe_of(blockIdx.y, gridDim.y, back), b = blockIdx.x, nb = gridDim.x;
   const int t = threadIdx.x;
   const ShiftedRow row(p, n, b, t);
   float s[NE][4];
@@ -760,11 +766,11 @@ __global__ void __launch_bounds__(kStreamThreads)
     k_project_dots(const float* __restrict__ Q, int64_t ldc, const float* __restrict__ x,
                    float* __restrict__ y, int64_t n, int ncols,
                    const float* __restrict__ h1part, float* __restrict__ h2part, int pstride,
-                   float* __restrict__ hout, int64_t hout_stride) {
+                   float* __restrict__ hout, int64_t hout_stride, int back) {
   using VT = typename VecE<E>::T;
   __shared__ __attribute__((aligned(16))) float hs[NC];
   __shared__ float red[kWaves * NC];
-  const int64_t p = blockIdx.y, b = blockIdx.x, nb = gridDim.x;
+  const int64_t p = probe_of(blockIdx.y, gridDim.y, back), b = blockIdx.x, nb = gridDim.x;
   const int t = threadIdx.x;
   const int64_t base = b * kChunk;
   if (t < NC) hs[t] = 0.f;
@@ -1103,21 +1109,21 @@ template <bool SUM>
 hipError_t launch_dots_any(hipStream_t s, const float* Q, int64_t ldc, const float* x, float* xw,
                            const MvSplitSum& sum, int64_t P, int64_t n, int ncols, float* partial,
                            int pstride, int64_t rows, int64_t xrow, int64_t prow,
-                           std::initializer_list<const void*> ptrs) {
+                           int back, std::initializer_list<const void*> ptrs) {
   const int V = stream_width(n, ldc, ptrs);
   const bool shifted = shifted_ok(n, ldc, ptrs);  // faster than the float2 kernels for even n
   const int64_t nb = num_chunks(n);
   const int nc = V == 4 || shifted ? dots_columns(nb * P * rows, ncols) : 8;
-  const dim3 grid(unsigned(nb), unsigned(P), unsigned(rows * ((ncols + nc - 1) / nc)));
+  const dim3 grid(unsigned(nb), unsigned(rows * ((ncols + nc - 1) / nc)), unsigned(P));
   const dim3 block(kStreamThreads);
   auto wide = [&](auto columns) {
     constexpr int NC = decltype(columns)::value;
     if (V == 4)
       hipLaunchKernelGGL((k_dots<4, NC, SUM>), grid, block, 0, s, Q, ldc, x, xw, n, ncols, partial,
-                         pstride, xrow, prow, sum);
+                         pstride, xrow, prow, sum, back);
     else
       hipLaunchKernelGGL((k_dots_shifted<NC, SUM>), grid, block, 0, s, Q, ldc, x, xw, n, ncols,
-                         partial, pstride, xrow, prow, sum);
+                         partial, pstride, xrow, prow, sum, back);
   };
   if (V == 4 || shifted) {
     if (nc == 8)
@@ -1128,10 +1134,10 @@ hipError_t launch_dots_any(hipStream_t s, const float* Q, int64_t ldc, const flo
       wide(std::integral_constant<int, 32>{});
   } else if (V == 2) {
     hipLaunchKernelGGL((k_dots<2, 8, SUM>), grid, block, 0, s, Q, ldc, x, xw, n, ncols, partial,
-                       pstride, xrow, prow, sum);
+                       pstride, xrow, prow, sum, back);
   } else {
     hipLaunchKernelGGL((k_dots<1, 8, SUM>), grid, block, 0, s, Q, ldc, x, xw, n, ncols, partial,
-                       pstride, xrow, prow, sum);
+                       pstride, xrow, prow, sum, back);
   }
   return hipGetLastError();
 }
@@ -1142,7 +1148,7 @@ int64_t max_dot_rows(int64_t ncols) { return std::max<int64_t>(1, 65535 / ((ncol
 
 hipError_t launch_dots(hipStream_t s, const float* Q, int64_t ldc, const float* x, int64_t P,
                        int64_t n, int ncols, float* partial, int pstride, int64_t rows,
-                       int64_t xrow, int64_t prow) {
+                       int64_t xrow, int64_t prow, int back) {
   if (Q == nullptr) {
     const int V = stream_width(n, n, {x});
     const dim3 grid(unsigned(num_chunks(n)), unsigned(P));
@@ -1156,13 +1162,14 @@ hipError_t launch_dots(hipStream_t s, const float* Q, int64_t ldc, const float* 
   }
   if (rows > 1 && xrow % 4 != 0) return hipErrorInvalidValue;  // one alignment for all rows
   return launch_dots_any<false>(s, Q, ldc, x, nullptr, MvSplitSum{}, P, n, ncols, partial, pstride,
-                                rows, xrow, prow, {x, Q});
+                                rows, xrow, prow, back, {x, Q});
 }
 
 hipError_t launch_dots_sum(hipStream_t s, const float* Q, int64_t ldc, const MvSplitSum& sum,
-                           float* x, int64_t P, int64_t n, int ncols, float* partial, int pstride) {
+                           float* x, int64_t P, int64_t n, int ncols, float* partial, int pstride,
+                           int back) {
   return launch_dots_any<true>(s, Q, ldc, nullptr, x, sum, P, n, ncols, partial, pstride, 1, 0, 0,
-                               {x, Q, sum.partial, sum.nugget ? sum.V : x});
+                               back, {x, Q, sum.partial, sum.nugget ? sum.V : x});
 }
 
 bool row_step_ok(int64_t P, int64_t n, int64_t ncols) {
@@ -1181,7 +1188,7 @@ hipError_t launch_row_step(hipStream_t s, const float* Q, int64_t ldc, int64_t P
 hipError_t launch_project(hipStream_t s, const float* Q, int64_t ldc, const float* x, float* y,
                           int64_t P, int64_t n, int ncols, const float* hpart, int pstride,
                           float* norm2part, float* hout, int64_t hout_stride, const float* hsub,
-                          int64_t hsub_stride, const PlaneOut* planes) {
+                          int64_t hsub_stride, const PlaneOut* planes, int back) {
   const int64_t nb = num_chunks(n);
   const dim3 grid{unsigned(nb), unsigned(P)};
   const size_t shmem = size_t(ncols > 0 ? ncols : 1) * sizeof(float);
@@ -1190,7 +1197,7 @@ hipError_t launch_project(hipStream_t s, const float* Q, int64_t ldc, const floa
   const bool ahead = nb * P < kManyBlocks;
 #define SLQ_PROJECT(K, ...)                                                                     \
   hipLaunchKernelGGL(K, grid, dim3(kStreamThreads), shmem, s, Q, ldc, x, y, n, ncols, hpart,    \
-                     pstride, norm2part, hout, hout_stride, hsub, hsub_stride, ##__VA_ARGS__)
+                     pstride, norm2part, hout, hout_stride, hsub, hsub_stride, back, ##__VA_ARGS__)
   if (V == 4) {
     if (planes && ahead)
       SLQ_PROJECT((k_project<4, true, true>), *planes);
@@ -1216,14 +1223,15 @@ hipError_t launch_project(hipStream_t s, const float* Q, int64_t ldc, const floa
 
 hipError_t launch_project_dots(hipStream_t s, const float* Q, int64_t ldc, const float* x,
                                float* y, int64_t P, int64_t n, int ncols, const float* h1part,
-                               float* h2part, int pstride, float* hout, int64_t hout_stride) {
+                               float* h2part, int pstride, float* hout, int64_t hout_stride,
+                               int back) {
   const dim3 grid(unsigned(num_chunks(n)), unsigned(P));
   const dim3 block(kStreamThreads);
   const bool v2 = (n % 2 == 0) && ldc % 2 == 0 && ((reinterpret_cast<uintptr_t>(Q) |
                    reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 7) == 0;
 #define SLQ_PD(NC, E)                                                                        \
   hipLaunchKernelGGL((k_project_dots<NC, E>), grid, block, 0, s, Q, ldc, x, y, n, ncols, h1part, \
-                     h2part, pstride, hout, hout_stride)
+                     h2part, pstride, hout, hout_stride, back)
   if (ncols <= 8) {
     if (v2) SLQ_PD(8, 2); else SLQ_PD(8, 1);
   } else if (ncols <= 16) {

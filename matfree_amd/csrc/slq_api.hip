@@ -312,13 +312,14 @@ int hessenberg_core(slq_context* ctx, const slq_operator& op, const float* V0, i
       SLQ_HIP(ctx, launch_row_step(s, Q, ldc, P, n, ncols, st));
       continue;
     }
+    const int back = j & 1;
     // h = Q^T w (decomp.py:463)
     {
       Timed tm(ctx, SLQ_KC_DOTS);
       if (pend.partial)
-        SLQ_HIP(ctx, launch_dots_sum(s, Q, ldc, pend, w, P, n, ncols, part1, pstride));
+        SLQ_HIP(ctx, launch_dots_sum(s, Q, ldc, pend, w, P, n, ncols, part1, pstride, back));
       else
-        SLQ_HIP(ctx, launch_dots(s, Q, ldc, w, P, n, ncols, part1, pstride));
+        SLQ_HIP(ctx, launch_dots(s, Q, ldc, w, P, n, ncols, part1, pstride, 1, 0, 0, back));
     }
     if (!reortho) {
       // w = w - Q h and <w, w> (decomp.py:464, 471), h into H[:, j]
@@ -338,7 +339,7 @@ int hessenberg_core(slq_context* ctx, const slq_operator& op, const float* V0, i
     if (ncols <= kFusedMaxCols) {
       Timed tm(ctx, SLQ_KC_PROJECT_DOTS);
       SLQ_HIP(ctx, launch_project_dots(s, Q, ldc, w, w2, P, n, ncols, part1, part2, pstride, hcol,
-                                        k * k));
+                                        k * k, !back));
     } else {
       SLQ_HIP(ctx, launch_project(s, Q, ldc, w, w2, P, n, ncols, part1, pstride, nullptr, hcol, k * k));
       SLQ_HIP(ctx, launch_dots(s, Q, ldc, w2, P, n, ncols, part2, pstride));
@@ -346,7 +347,8 @@ int hessenberg_core(slq_context* ctx, const slq_operator& op, const float* V0, i
     // w = w - Q (Q^T w) and <w, w> (decomp.py:468, 471)
     {
       Timed tm(ctx, SLQ_KC_PROJECT);
-      SLQ_HIP(ctx, launch_project(s, Q, ldc, w2, dst, P, n, ncols, part2, pstride, norm2, nullptr, 0));
+      SLQ_HIP(ctx, launch_project(s, Q, ldc, w2, dst, P, n, ncols, part2, pstride, norm2, nullptr, 0,
+                                  nullptr, 0, nullptr, back));
     }
     if (!last) {
       // length = sqrt(<w, w>); h[j+1] = length (decomp.py:471-475); next
