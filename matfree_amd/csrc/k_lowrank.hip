@@ -393,7 +393,7 @@ __global__ void __launch_bounds__(kT)
 // matvec of d added in the order of launch_matvec's own reduction (so q is
 // the same, bit for bit), written to q, and the per-column partial dots d . q
 // over the same chunks as k_cg_dot; the partials' loads are issued 16 at a
-// time.
+// time for all of a thread's elements.
 __global__ void __launch_bounds__(kTq)
     k_cg_dot_q(const float* __restrict__ d, MvSplitSum qsum, int64_t n, float* __restrict__ q,
                float* __restrict__ part) {
@@ -401,26 +401,37 @@ __global__ void __launch_bounds__(kTq)
   const int64_t p = blockIdx.y, c = blockIdx.x, nb = gridDim.x;
   const int64_t count = int64_t(gridDim.y) * n;
   const int64_t base = c * kCgChunk;
-  float acc = 0.f;
+  // all of a thread's elements are loaded together (indices past n are the
+  // row's last one, not used)
+  int64_t at[kQPer];
+  float v[kQPer], dv[kQPer];
 #pragma unroll
   for (int e = 0; e < kQPer; ++e) {
     const int64_t i = base + int64_t(e) * kTq + threadIdx.x;
-    if (i < n) {
-      const int64_t at = p * n + i;
-      float v = qsum.partial[at];
-      for (int z0 = 1; z0 < qsum.S; z0 += 16) {
-        float pz[16];
+    at[e] = p * n + (i < n ? i : n - 1);
+    v[e] = qsum.partial[at[e]];
+    dv[e] = d[at[e]];
+  }
+  for (int z0 = 1; z0 < qsum.S; z0 += 16) {
+    float pz[kQPer][16];
 #pragma unroll
-        for (int z = 0; z < 16; ++z)
-          pz[z] = z0 + z < qsum.S ? qsum.partial[int64_t(z0 + z) * count + at] : 0.f;
+    for (int z = 0; z < 16; ++z)
 #pragma unroll
-        for (int z = 0; z < 16; ++z)
-          if (z0 + z < qsum.S) v += pz[z];
-      }
-      const float dv = d[at];
-      if (qsum.nugget) v = fmaf(qsum.noise, dv, v);
-      q[at] = v;
-      acc = fmaf(dv, v, acc);
+      for (int e = 0; e < kQPer; ++e)
+        pz[e][z] = z0 + z < qsum.S ? qsum.partial[int64_t(z0 + z) * count + at[e]] : 0.f;
+#pragma unroll
+    for (int z = 0; z < 16; ++z)
+      if (z0 + z < qsum.S)
+#pragma unroll
+        for (int e = 0; e < kQPer; ++e) v[e] += pz[e][z];
+  }
+  float acc = 0.f;
+#pragma unroll
+  for (int e = 0; e < kQPer; ++e) {
+    if (base + int64_t(e) * kTq + threadIdx.x < n) {
+      if (qsum.nugget) v[e] = fmaf(qsum.noise, dv[e], v[e]);
+      q[at[e]] = v[e];
+      acc = fmaf(dv[e], v[e], acc);
     }
   }
   const float s = block_sum_f<kTq>(acc, red);
@@ -428,9 +439,7 @@ __global__ void __launch_bounds__(kTq)
 }
 
 __device__ __forceinline__ float sum_parts(const float* part, int64_t p, int64_t nb) {
-  float s = 0.f;
-  for (int64_t c = 0; c < nb; ++c) s += part[p * nb + c];
-  return s;
+  return ordered_sum(part + p * nb, nb, 1);
 }
 
 // generation 0: gamma = r . z, atol2 = max(tol^2 b.b, atol^2), active
@@ -466,20 +475,30 @@ __global__ void __launch_bounds__(kTq)
   __shared__ float red[kTq / 64];
   const int64_t p = blockIdx.y, c = blockIdx.x, nb = gridDim.x, P = gridDim.y;
   const int64_t base = c * kCgChunk;
+  // the vectors are on their way while the scalars are read and divided
+  int64_t at[kQPer];
+  float xv[kQPer], rv[kQPer], dv[kQPer], qv[kQPer];
+#pragma unroll
+  for (int e = 0; e < kQPer; ++e) {
+    const int64_t i = base + int64_t(e) * kTq + threadIdx.x;
+    at[e] = p * n + (i < n ? i : n - 1);
+    xv[e] = x[at[e]];
+    rv[e] = r[at[e]];
+    dv[e] = d[at[e]];
+    qv[e] = q[at[e]];
+  }
   const bool act = sc.active[gen * P + p] != 0;
   const float al = act ? sc.gamma[gen * P + p] / sum_parts(pq, p, nb) : 0.f;
   float acc = 0.f;
 #pragma unroll
   for (int e = 0; e < kQPer; ++e) {
-    const int64_t i = base + int64_t(e) * kTq + threadIdx.x;
-    if (i < n) {
-      float rv = r[p * n + i];
+    if (base + int64_t(e) * kTq + threadIdx.x < n) {
       if (act) {
-        x[p * n + i] = fmaf(al, d[p * n + i], x[p * n + i]);
-        rv = fmaf(-al, q[p * n + i], rv);
-        r[p * n + i] = rv;
+        x[at[e]] = fmaf(al, dv[e], xv[e]);
+        rv[e] = fmaf(-al, qv[e], rv[e]);
+        r[at[e]] = rv[e];
       }
-      acc = fmaf(rv, rv, acc);
+      acc = fmaf(rv[e], rv[e], acc);
     }
   }
   const float s = block_sum_f<kTq>(acc, red);
@@ -496,6 +515,16 @@ __global__ void __launch_bounds__(kTq)
                         int64_t maxiter, CgScalars sc, int gen) {
   const int64_t p = blockIdx.y, c = blockIdx.x, nb = gridDim.x, P = gridDim.y;
   const int64_t cur = gen * P + p, nxt = (gen ^ 1) * P + p;
+  const int64_t base = c * kCgChunk;
+  int64_t at[kQPer];
+  float dv[kQPer], zv[kQPer];
+#pragma unroll
+  for (int e = 0; e < kQPer; ++e) {
+    const int64_t i = base + int64_t(e) * kTq + threadIdx.x;
+    at[e] = p * n + (i < n ? i : n - 1);
+    dv[e] = d[at[e]];
+    zv[e] = z[at[e]];
+  }
   const int act = sc.active[cur];
   const float g = act ? sum_parts(precond ? rz : rr, p, nb) : 0.f;
   if (c == 0 && threadIdx.x == 0) {
@@ -511,12 +540,9 @@ __global__ void __launch_bounds__(kTq)
   }
   if (!act) return;
   const float be = g / sc.gamma[cur];
-  const int64_t base = c * kCgChunk;
 #pragma unroll
-  for (int e = 0; e < kQPer; ++e) {
-    const int64_t i = base + int64_t(e) * kTq + threadIdx.x;
-    if (i < n) d[p * n + i] = fmaf(be, d[p * n + i], z[p * n + i]);
-  }
+  for (int e = 0; e < kQPer; ++e)
+    if (base + int64_t(e) * kTq + threadIdx.x < n) d[at[e]] = fmaf(be, dv[e], zv[e]);
 }
 
 // *nactive = number of columns active in generation gen
