@@ -36,6 +36,8 @@
 // update, and beta with the new direction.  The host reads the number of
 // active columns after batches of 1, 2, 4, 8, 8, ... iterations (an iteration
 // with no active column changes nothing).
+#include <type_traits>
+
 #include <cfloat>
 
 #include "slq_internal.h"
@@ -51,6 +53,10 @@ constexpr int kCgChunk = kT * kCgPer;
 // chunks, so more threads per chunk shorten these latency-bound launches.
 constexpr int kTq = 1024;
 constexpr int kQPer = kCgChunk / kTq;
+// Columns of up to this many chunks (n <= 8192) finish an iteration in one
+// workgroup, of up to this many (n <= 4096) with the split-K sum as well.
+constexpr int kCgColumnChunks = 4;
+constexpr int kCgColumnSumChunks = 2;
 
 __device__ __forceinline__ float wsum_f(float v) {
 #pragma unroll
@@ -545,6 +551,107 @@ __global__ void __launch_bounds__(kTq)
     if (base + int64_t(e) * kTq + threadIdx.x < n) d[at[e]] = fmaf(be, dv[e], zv[e]);
 }
 
+// k_cg_update and k_cg_beta_direction of a column of NB chunks (no
+// preconditioner) in one workgroup, with SUM also the k_cg_dot_q before them:
+// the chunk sums meet in LDS, the vectors stay in registers in between.  The
+// same sums in the same order.  60 iterations of the RBF operator, a launch
+// each before: n = 1024 1516 -> 1026 us, 4500 1719 -> 1553, 8192
+// 2046 -> 1945; 16 columns of 2048 1571 -> 962.
+template <int NB, bool SUM>
+__global__ void __launch_bounds__(kTq)
+    k_cg_column(float* __restrict__ x, float* __restrict__ r, float* __restrict__ d,
+                const float* __restrict__ q, MvSplitSum qsum, int64_t n,
+                const float* __restrict__ pq, int64_t maxiter, CgScalars sc, int gen) {
+  constexpr int NE = NB * kQPer, NW = kTq / 64;
+  __shared__ float red[2][NB][NW];
+  const int64_t p = blockIdx.x, P = gridDim.x;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int64_t cur = gen * P + p, nxt = (gen ^ 1) * P + p;
+  // every load is issued first (indices past n are the row's last, not used)
+  int64_t at[NE];
+  float xv[NE], rv[NE], dv[NE], qv[NE];
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const int64_t i = int64_t(e) * kTq + t;
+    at[e] = p * n + (i < n ? i : n - 1);
+    qv[e] = SUM ? qsum.partial[at[e]] : q[at[e]];
+    dv[e] = d[at[e]];
+    xv[e] = x[at[e]];
+    rv[e] = r[at[e]];
+  }
+  const float gamma = sc.gamma[cur];
+  if (sc.active[cur] == 0) {
+    if (t == 0) {
+      sc.gamma[nxt] = gamma;
+      sc.active[nxt] = 0;
+    }
+    return;
+  }
+  auto live = [&](int e) { return int64_t(e) * kTq + t < n; };
+  // sum over the column's chunks of the chunk sums of term(e) = fma(u, v, acc)
+  auto column_sum = [&](float (&part)[NB][NW], auto term) {
+#pragma unroll
+    for (int c = 0; c < NB; ++c) {
+      float acc = 0.f;
+#pragma unroll
+      for (int u = 0; u < kQPer; ++u)
+        if (live(c * kQPer + u)) acc = term(c * kQPer + u, acc);
+      acc = wsum_f(acc);
+      if (lane == 0) part[c][wave] = acc;
+    }
+    __syncthreads();
+    float g = 0.f;
+#pragma unroll
+    for (int c = 0; c < NB; ++c) {
+      float s = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) s += part[c][w];
+      g += s;
+    }
+    return g;
+  };
+  float pap;
+  if constexpr (SUM) {
+    const int64_t count = P * n;
+    for (int z0 = 1; z0 < qsum.S; z0 += 8) {
+      float pz[8][NE];
+#pragma unroll
+      for (int z = 0; z < 8; ++z)
+#pragma unroll
+        for (int e = 0; e < NE; ++e)
+          pz[z][e] = z0 + z < qsum.S ? qsum.partial[int64_t(z0 + z) * count + at[e]] : 0.f;
+#pragma unroll
+      for (int z = 0; z < 8; ++z)
+        if (z0 + z < qsum.S)
+#pragma unroll
+          for (int e = 0; e < NE; ++e) qv[e] += pz[z][e];
+    }
+    if (qsum.nugget)
+#pragma unroll
+      for (int e = 0; e < NE; ++e) qv[e] = fmaf(qsum.noise, dv[e], qv[e]);
+    pap = column_sum(red[0], [&](int e, float acc) { return fmaf(dv[e], qv[e], acc); });
+  } else {
+    pap = sum_parts(pq, p, NB);
+  }
+  const float al = gamma / pap;
+  const float g = column_sum(red[1], [&](int e, float acc) {
+    x[at[e]] = fmaf(al, dv[e], xv[e]);
+    rv[e] = fmaf(-al, qv[e], rv[e]);
+    r[at[e]] = rv[e];
+    return fmaf(rv[e], rv[e], acc);
+  });
+  if (t == 0) {
+    const int64_t k = sc.iters[p] + 1;
+    sc.iters[p] = k;
+    sc.gamma[nxt] = g;
+    sc.active[nxt] = (g > sc.atol2[p]) && (k < maxiter);
+  }
+  const float be = g / gamma;
+#pragma unroll
+  for (int e = 0; e < NE; ++e)
+    if (live(e)) d[at[e]] = fmaf(be, dv[e], rv[e]);
+}
+
 // *nactive = number of columns active in generation gen
 __global__ void __launch_bounds__(kT)
     k_cg_count(CgScalars sc, int gen, int64_t P, int* __restrict__ nactive) {
@@ -642,10 +749,34 @@ hipError_t launch_cg_step(hipStream_t s, float* x, float* r, float* d, float* q,
                           float* rz, const CgPrecond* M) {
   const int64_t nb = cg_chunks(n);
   const dim3 grid{unsigned(nb), unsigned(P)};
-  if (qsum.partial)
+  const bool columns = !precond && nb <= kCgColumnChunks;
+  const bool column_sums = columns && qsum.partial && nb <= kCgColumnSumChunks;
+  if (qsum.partial && !column_sums)
     hipLaunchKernelGGL(k_cg_dot_q, grid, dim3(kTq), 0, s, d, qsum, n, q, pq);
-  else
+  else if (!qsum.partial)
     hipLaunchKernelGGL(k_cg_dot, grid, dim3(kT), 0, s, d, q, n, pq);
+  if (columns) {
+    auto column = [&](auto chunks, auto sums) {
+      constexpr int NB = decltype(chunks)::value;
+      constexpr bool SUM = decltype(sums)::value;
+      hipLaunchKernelGGL((k_cg_column<NB, SUM>), dim3(unsigned(P)), dim3(kTq), 0, s, x, r, d, q,
+                         qsum, n, pq, maxiter, sc, gen);
+    };
+    using std::integral_constant;
+    if (nb == 1 && column_sums)
+      column(integral_constant<int, 1>{}, std::true_type{});
+    else if (nb == 1)
+      column(integral_constant<int, 1>{}, std::false_type{});
+    else if (nb == 2 && column_sums)
+      column(integral_constant<int, 2>{}, std::true_type{});
+    else if (nb == 2)
+      column(integral_constant<int, 2>{}, std::false_type{});
+    else if (nb == 3)
+      column(integral_constant<int, 3>{}, std::false_type{});
+    else
+      column(integral_constant<int, 4>{}, std::false_type{});
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(k_cg_update, grid, dim3(kTq), 0, s, x, r, d, q, n, pq, sc, gen, rr);
   if (precond) {
     hipError_t e = launch_woodbury_apply(s, M->L, n, M->rank, M->shift, M->C, r, P, M->Wp, M->Z, z);

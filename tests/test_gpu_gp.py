@@ -302,3 +302,25 @@ def test_gaussian_logpdf_with_only_the_lengthscale_learned(cuda):
     alpha = np.linalg.solve(A, y.astype(np.float64))
     exact = 0.5 * (alpha @ dA @ alpha - np.trace(np.linalg.solve(A, dA)))
     assert abs(float(ell.grad) - exact) <= 0.1 * abs(exact) + 0.05, (float(ell.grad), exact)
+
+
+@pytest.mark.parametrize("n", [5, 700, 1024, 2047, 2048, 2049, 4096, 4097, 6145, 8192, 8193])
+def test_cg_column_kernels(cuda, n):
+    # an iteration of a column in one workgroup (n <= 8192), with the split-K sum (n <= 4096)
+    # and without, at the chunk edges; a zero right-hand side beside the others stays at zero.
+    # A stored matrix with eigenvalues in [1, 5]: the recurrence stops at 1e-6 |b|, and its
+    # residual and the true one part by sum_t |alpha_t A d_t| times the products' 2e-6, at most
+    # 2e-6 |A| 2 |x| = 2e-5 |b|.  Together with the sums' own rounding 3e-5.
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    G = torch.randn((n, n), generator=gen, device="cuda")
+    A = G @ G.T / n
+    A = 0.5 * (A + A.T)
+    A.diagonal().add_(1.0)
+    B = torch.randn((3, n), generator=gen, device="cuda")
+    B[1] = 0.0
+    x, iters = linalg.cg_batched(operators.dense_matvec, B, (A,), tol=1e-6)
+    residual = (B.double() - x.double() @ A.double()).norm(dim=1)
+    assert float(x[1].abs().max()) == 0.0 and int(iters[1]) == 0
+    assert int(iters[0]) > 0 and int(iters[2]) > 0
+    for p in (0, 2):
+        assert float(residual[p] / B[p].double().norm()) < 3e-5
