@@ -200,30 +200,38 @@ inline int dots_columns(int64_t blocks, int ncols) {
   return blocks < kManyBlocks || ncols <= 8 ? 8 : ncols <= 16 ? 16 : 32;
 }
 
-// Probe of a block: in order, or back (see launch_dots).
+// Order of a pass over the basis: of a dots pass column group by column group,
+// or probe by probe, in ascending or descending order (see launch_dots).  Few
+// blocks keep the first: a chunk of a probe then has the same place in the
+// grid, so the same XCD, in every pass of a step, and its columns are found in
+// that XCD's L2 (n = 8192, 32 probes, depth 32 with gradient: 3740 us, 3900
+// with alternating probes).  From kManyBlocks on a few columns fill the L2s.
+enum ProbeOrder { kColumnGroups = 0, kProbes = 1, kProbesBack = 2 };
+
 __device__ __forceinline__ int64_t probe_of(unsigned i, unsigned count, int back) {
   return back ? count - 1 - i : i;
 }
 
 // SUM: x is the deferred split-K sum `sm`, stored to xw by the blocks of
-// column group 0.  blockIdx.y = row * column groups + column group; row i reads
+// column group 0.  zi = row * column groups + column group; row i reads
 // x + i xrow and writes partial + i prow.
 template <int V, int NC, bool SUM>
 __global__ void __launch_bounds__(kStreamThreads)
     k_dots(const float* __restrict__ Q, int64_t ldc, const float* __restrict__ x, float* xw,
            int64_t n, int ncols, float* __restrict__ partial, int pstride, int64_t xrow,
-           int64_t prow, MvSplitSum sm, int back) {
+           int64_t prow, MvSplitSum sm, ProbeOrder order) {
   constexpr int NE = Layout<V>::NE;
   constexpr int CB = kColBatch;
   __shared__ float red[kWaves * NC];
-  const int64_t p = probe_of(blockIdx.z, gridDim.z, back);
+  const int64_t P = order ? gridDim.z : gridDim.y, zi = order ? blockIdx.y : blockIdx.z;
+  const int64_t p = order ? probe_of(blockIdx.z, gridDim.z, order == kProbesBack) : blockIdx.y;
   const int64_t b = blockIdx.x;
   const int64_t nb = gridDim.x;
   const int t = threadIdx.x;
   const int64_t base = b * kChunk;
   const int groups = (ncols + NC - 1) / NC;
-  const int64_t row = blockIdx.y / groups;
-  const int c0 = int(blockIdx.y % groups) * NC;
+  const int64_t row = zi / groups;
+  const int c0 = int(zi % groups) * NC;
 
   int64_t off[NE];
   bool in[NE];
@@ -246,7 +254,7 @@ __global__ void __launch_bounds__(kStreamThreads)
   load(0);
   float xv[NE][V];
   if constexpr (SUM) {
-    split_sum<V, NE>(sm, int64_t(gridDim.z) * n, off, xv);
+    split_sum<V, NE>(sm, P * n, off, xv);
   } else {
 #pragma unroll
     for (int e = 0; e < NE; ++e) VecIO<V>::load(x + row * xrow + off[e], xv[e]);
@@ -312,15 +320,17 @@ template <int NC, bool SUM>
 __global__ void __launch_bounds__(kStreamThreads)
     k_dots_shifted(const float* __restrict__ Q, int64_t ldc, const float* __restrict__ x,
                    float* xw, int64_t n, int ncols, float* __restrict__ partial, int pstride,
-                   int64_t xrow, int64_t prow, MvSplitSum sm, int back) {
+                   int64_t xrow, int64_t prow, MvSplitSum sm, ProbeOrder order) {
   constexpr int NE = Layout<4>::NE;
   constexpr int CB = kColBatch;
   __shared__ float red[kWaves * NC];
-  const int64_t p = probe_of(blockIdx.z, gridDim.z, back), b = blockIdx.x, nb = gridDim.x;
+  const int64_t P = order ? gridDim.z : gridDim.y, zi = order ? blockIdx.y : blockIdx.z;
+  const int64_t p = order ? probe_of(blockIdx.z, gridDim.z, order == kProbesBack) : blockIdx.y;
+  const int64_t b = blockIdx.x, nb = gridDim.x;
   const int t = threadIdx.x;
   const int groups = (ncols + NC - 1) / NC;
-  const int64_t drow = blockIdx.y / groups;
-  const int c0 = int(blockIdx.y % groups) * NC;
+  const int64_t drow = zi / groups;
+  const int c0 = int(zi % groups) * NC;
   const ShiftedRow row(p, n, b, t);
   int64_t off[NE];
   bool in[NE];
@@ -346,8 +356,8 @@ __global__ void __launch_bounds__(kStreamThreads)
   load(0);
   float xv[NE][4], xh[1][1];
   if constexpr (SUM) {
-    split_sum<4, NE>(sm, int64_t(gridDim.z) * n, off, xv);
-    split_sum<1, 1>(sm, int64_t(gridDim.z) * n, ixo, xh);
+    split_sum<4, NE>(sm, P * n, off, xv);
+    split_sum<1, 1>(sm, P * n, ixo, xh);
   } else {
     const float* xr = x + drow * xrow;
 #pragma unroll
@@ -1114,16 +1124,19 @@ hipError_t launch_dots_any(hipStream_t s, const float* Q, int64_t ldc, const flo
   const bool shifted = shifted_ok(n, ldc, ptrs);  // faster than the float2 kernels for even n
   const int64_t nb = num_chunks(n);
   const int nc = V == 4 || shifted ? dots_columns(nb * P * rows, ncols) : 8;
-  const dim3 grid(unsigned(nb), unsigned(rows * ((ncols + nc - 1) / nc)), unsigned(P));
+  const unsigned groups = unsigned(rows * ((ncols + nc - 1) / nc));
+  const ProbeOrder order = nb * P < kManyBlocks ? kColumnGroups : back ? kProbesBack : kProbes;
+  const dim3 grid = order ? dim3(unsigned(nb), groups, unsigned(P))
+                          : dim3(unsigned(nb), unsigned(P), groups);
   const dim3 block(kStreamThreads);
   auto wide = [&](auto columns) {
     constexpr int NC = decltype(columns)::value;
     if (V == 4)
       hipLaunchKernelGGL((k_dots<4, NC, SUM>), grid, block, 0, s, Q, ldc, x, xw, n, ncols, partial,
-                         pstride, xrow, prow, sum, back);
+                         pstride, xrow, prow, sum, order);
     else
       hipLaunchKernelGGL((k_dots_shifted<NC, SUM>), grid, block, 0, s, Q, ldc, x, xw, n, ncols,
-                         partial, pstride, xrow, prow, sum, back);
+                         partial, pstride, xrow, prow, sum, order);
   };
   if (V == 4 || shifted) {
     if (nc == 8)
@@ -1134,10 +1147,10 @@ hipError_t launch_dots_any(hipStream_t s, const float* Q, int64_t ldc, const flo
       wide(std::integral_constant<int, 32>{});
   } else if (V == 2) {
     hipLaunchKernelGGL((k_dots<2, 8, SUM>), grid, block, 0, s, Q, ldc, x, xw, n, ncols, partial,
-                       pstride, xrow, prow, sum, back);
+                       pstride, xrow, prow, sum, order);
   } else {
     hipLaunchKernelGGL((k_dots<1, 8, SUM>), grid, block, 0, s, Q, ldc, x, xw, n, ncols, partial,
-                       pstride, xrow, prow, sum, back);
+                       pstride, xrow, prow, sum, order);
   }
   return hipGetLastError();
 }
@@ -1195,6 +1208,7 @@ hipError_t launch_project(hipStream_t s, const float* Q, int64_t ldc, const floa
   const int V = stream_width(n, ldc, {x, y, Q});
   if (planes && V != 4) return hipErrorInvalidValue;
   const bool ahead = nb * P < kManyBlocks;
+  if (ahead) back = 0;
 #define SLQ_PROJECT(K, ...)                                                                     \
   hipLaunchKernelGGL(K, grid, dim3(kStreamThreads), shmem, s, Q, ldc, x, y, n, ncols, hpart,    \
                      pstride, norm2part, hout, hout_stride, hsub, hsub_stride, back, ##__VA_ARGS__)
@@ -1227,6 +1241,7 @@ hipError_t launch_project_dots(hipStream_t s, const float* Q, int64_t ldc, const
                                int back) {
   const dim3 grid(unsigned(num_chunks(n)), unsigned(P));
   const dim3 block(kStreamThreads);
+  if (num_chunks(n) * P < kManyBlocks) back = 0;
   const bool v2 = (n % 2 == 0) && ldc % 2 == 0 && ((reinterpret_cast<uintptr_t>(Q) |
                    reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 7) == 0;
 #define SLQ_PD(NC, E)                                                                        \

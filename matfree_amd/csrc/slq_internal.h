@@ -84,7 +84,7 @@ struct MvSplitSum {
 // Q may be null with ncols = 1 to mean "sum of squares of x" (partial[p][b][0]).
 // rows (up to max_dot_rows): the same for that many blocks x + i * xrow, into
 // partial + i * prow.
-// back: the probes in descending order.  The passes over the basis of a step
+// back: from 1024 blocks on, the probes in descending order.  The passes over the basis of a step
 // alternate, so that each begins with what the one before read last (256 MB
 // stay in the Infinity Cache).  Depth 40 at n = 16384, 256 probes: the projection
 // with dots 3.38 -> 2.74 ms of a decomposition, the other passes as before; a
