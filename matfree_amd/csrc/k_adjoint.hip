@@ -99,17 +99,29 @@ __global__ void __launch_bounds__(kStreamThreads)
                       int64_t n, int64_t k, int ncq, int jl0, const float* __restrict__ coef,
                       const float* __restrict__ d, AdjointStep st, int64_t nb) {
   extern __shared__ float cs[];
-  const int64_t p = blockIdx.y;
+  // kSub blocks a chunk, at that chunk's place modulo the XCDs in the dots' and
+  // the projections' grids (chunk b of probe p is block p nb + b there): the
+  // columns are found in the XCD's L2 (n = 8192, 32 probes, depth 32: 13.0 ->
+  // 11.6 us a step; with blocks in the order of the row they were not).
+  constexpr int kSub = int(kChunk / (kStreamThreads * V));
+  constexpr int kXcds = 8;
+  const int64_t id = blockIdx.x, set = int64_t(kXcds) * kSub;
+  const bool whole = id / set * set + set <= gridDim.x;
+  const int64_t c = whole ? id / set * kXcds + id % kXcds : id / kSub;
+  const int sub = int(whole ? id % set / kXcds : id % kSub);
+  const int64_t p = c / nb;
+  const int64_t first = c % nb * kChunk + int64_t(sub) * kStreamThreads * V;
+  if (first >= n) return;
   const int t = threadIdx.x;
   if constexpr (STEP) {
-    step_coefficients(st, p, nb, k, blockIdx.x == 0, cs);
+    step_coefficients(st, p, nb, k, first == 0, cs);
   } else {
     const float* cp = coef + p * (2 * k + 4);
     for (int64_t j = t; j < 2 * k + 4; j += blockDim.x) cs[j] = cp[j];
     __syncthreads();
   }
   const float cr = cs[2 * k], cl = cs[2 * k + 1], cv = cs[2 * k + 2], sc = cs[2 * k + 3];
-  const int64_t i = (int64_t(blockIdx.x) * kStreamThreads + t) * V;
+  const int64_t i = first + int64_t(t) * V;
   if (i >= n) return;
   // W elements from offset off (W = 4: one 16-byte access per operand)
   auto combine = [&](auto width, int64_t off) {
@@ -535,8 +547,8 @@ hipError_t launch_combine(hipStream_t s, const float* Q, const float* Lam, int64
                           int64_t P, int64_t n, int64_t k, int ncq, int jl0, const float* coef,
                           const float* d, const AdjointStep& st) {
   const bool vec = P * n >= (int64_t(1) << 20);
-  const int64_t per_block = int64_t(kStreamThreads) * (vec ? 4 : 1);
-  const dim3 grid(unsigned((n + per_block - 1) / per_block), unsigned(P));
+  const int64_t sub = kChunk / (kStreamThreads * (vec ? 4 : 1));
+  const dim3 grid(unsigned(P * num_chunks(n) * sub));
   const size_t shmem = size_t(2 * k + 4) * sizeof(float);
   if (vec)
     hipLaunchKernelGGL((k_adjoint_combine<4, STEP>), grid, dim3(kStreamThreads), shmem, s, Q, Lam,
