@@ -192,12 +192,17 @@ constexpr int kColBatch = 8;
 constexpr int64_t kManyBlocks = 1024;
 
 // Columns of a block of the dots kernels; the other columns of a chunk are
-// blocks of their own.  Few blocks: 8, so that no block waits for one batch of
-// loads after the other (n = 1001, 16 probes: 5% of a decomposition).  Many:
-// 16, which halves the reads of x (n = 32768, 128 probes, 64 columns: no
-// difference between 8 and 64, the memory bounds them all).
+// blocks of their own.  As many as leave two blocks a CU: with fewer no block
+// should wait for one batch of loads after the other (n = 1001, 16 probes, 8
+// columns: 5% of a decomposition), with more every block of a chunk reads its
+// x, or adds up its split-K slices, again (log-determinant of depth 48 with 128
+// probes, 8 columns up to 1024 blocks: n = 6144 4.71 ms, this rule 4.15; 12288
+// 8.88 and 8.05; one block a CU: 64 probes of 9984 4.03 -> 4.13).
+constexpr int64_t kDotsBlocks = 512;
 inline int dots_columns(int64_t blocks, int ncols) {
-  return blocks < kManyBlocks || ncols <= 8 ? 8 : ncols <= 16 ? 16 : 32;
+  for (int nc = 64; nc > 8; nc /= 2)
+    if (ncols > nc / 2 && blocks * ((ncols + nc - 1) / nc) >= kDotsBlocks) return nc;
+  return 8;
 }
 
 // Order of a pass over the basis: of a dots pass column group by column group,
@@ -1143,8 +1148,10 @@ hipError_t launch_dots_any(hipStream_t s, const float* Q, int64_t ldc, const flo
       wide(std::integral_constant<int, 8>{});
     else if (nc == 16)
       wide(std::integral_constant<int, 16>{});
-    else
+    else if (nc == 32)
       wide(std::integral_constant<int, 32>{});
+    else
+      wide(std::integral_constant<int, 64>{});
   } else if (V == 2) {
     hipLaunchKernelGGL((k_dots<2, 8, SUM>), grid, block, 0, s, Q, ldc, x, xw, n, ncols, partial,
                        pstride, xrow, prow, sum, order);
