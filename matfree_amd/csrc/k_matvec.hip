@@ -26,8 +26,8 @@ namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
-constexpr int BI = 128;      // output elements per workgroup
-constexpr int BK = 32;       // contraction tile
+constexpr int BI = kMvRows;
+constexpr int BK = kMvTile;
 constexpr int kThreads = 256;
 
 struct RBFParams {
@@ -380,16 +380,16 @@ __device__ __forceinline__ float tile_sign(int64_t kt) {
 // ((kt * Ppad / 32 + p / 32) * 2 + kb) * 64 + (p % 32) + 32 h of a plane holds
 // columns 32 kt + 16 kb + 8 h .. + 7 of probe p, so that a workgroup's probe
 // tile is contiguous and a wave's fragment is 64 consecutive words (no bank
-// conflicts without padding).  One word per thread.
+// conflicts without padding).  One word per thread, from tile kt0 on.
 __global__ void __launch_bounds__(256)
-    k_split3_probes(const float* __restrict__ V, int64_t P, int64_t n, int64_t npb, int64_t words,
-                    u32x4* __restrict__ planes) {
+    k_split3_probes(const float* __restrict__ V, int64_t P, int64_t n, int64_t npb, int64_t kt0,
+                    int64_t words, u32x4* __restrict__ planes) {
   const int64_t stride = int64_t(gridDim.x) * blockDim.x;
   for (int64_t w = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; w < words; w += stride) {
     const int lane = int(w & 63), kb = int(w >> 6) & 1;
     const int64_t blk = w >> 7;
-    const int64_t kt = blk / npb, p = (blk - kt * npb) * 32 + (lane & 31);
-    const int64_t m = kt * BK + 16 * kb + 8 * (lane >> 5);
+    const int64_t row = blk / npb, p = (blk - row * npb) * 32 + (lane & 31);
+    const int64_t kt = kt0 + row, m = kt * BK + 16 * kb + 8 * (lane >> 5);
     float x[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) x[e] = 0.f;
@@ -513,7 +513,7 @@ template <int NACC, bool RBF, int DIM>
 __global__ void __launch_bounds__(kThreads, 2)
     k_matvec_f32(const float* __restrict__ A, RBFParams prm, const u32x4* __restrict__ planes,
                  int64_t plane_words, int64_t npb, const float* __restrict__ V, int64_t P,
-                 int64_t n, float* __restrict__ W, int64_t wstride) {
+                 int64_t n, float* __restrict__ W, int64_t wstride, int S, int z0) {
   constexpr int TW = 128 * NACC;  // words of one plane's tile
   constexpr int kPieces = 3 * TW;
   constexpr int PT = kPieces / kThreads;
@@ -531,16 +531,17 @@ __global__ void __launch_bounds__(kThreads, 2)
   const int64_t i0w = int64_t(blockIdx.x) * BI + 32 * wave;
   const int64_t row = i0w + r;
   const int64_t p0 = int64_t(blockIdx.y) * 32 * NACC;
-  // split-K: slice z of gridDim.z covers tiles [kt_begin, kt_end), whole runs of
-  // one plane sign
+  // split-K: slice z of S covers tiles [kt_begin, kt_end), whole runs of one
+  // plane sign (`planes` points where tile 0 would be)
+  const int64_t z = z0 + int64_t(blockIdx.z);
   const int64_t all_tiles = (n + BK - 1) / BK;
   const int64_t runs = (all_tiles + kSignRun - 1) / kSignRun;
-  const int64_t kt_begin = runs * blockIdx.z / gridDim.z * kSignRun;
-  int64_t kt_end = runs * (blockIdx.z + 1) / gridDim.z * kSignRun;
+  const int64_t kt_begin = runs * z / S * kSignRun;
+  int64_t kt_end = runs * (z + 1) / S * kSignRun;
   if (kt_end > all_tiles) kt_end = all_tiles;
   const int64_t ntiles = kt_end - kt_begin;
-  const bool split = gridDim.z > 1;
-  float* Wout = W + int64_t(blockIdx.z) * wstride;
+  const bool split = S > 1;
+  float* Wout = W + z * wstride;
 
   floatx16 acc[NACC], sum[NACC];
 #pragma unroll
@@ -2549,82 +2550,56 @@ hipError_t launch_tpl_bf16(hipStream_t s, const float* A, const u32x4* rec, cons
   return launch_tpl_bf16_n<NACC, RBF, 1>(s, A, rec, prm, Vhi, Vlo, Ppad, V, P, n, W, vec, S);
 }
 
-int nacc_for(int64_t P) { return P <= 32 ? 1 : (P <= 64 ? 2 : 4); }
-
-// Whether the FP32 matvec of P vectors reads planes: not the stream form of a
-// stored matrix (up to 32 probes), and not the wave form at small n, where the
-// waves split the vectors themselves (the launch that writes the planes costs
-// about 3.5 us, splitting in the waves 0.2 us per 1000 columns).
-bool f32_planes(int64_t n, int64_t P, bool rbf) {
-  return nacc_for(P) > 1 || (rbf && n >= 4096);
-}
-
-// Whether the stream form takes the probes in the order of its fragments
-// (k_tile_probes; written by the producer of the input where there is one, in a
-// launch of about 3.5 us otherwise).  With up to 16 probes most of a tile is
-// padding, and its lines cost more than the rows' (15001, 16 probes: 199 -> 208
-// us); up to n = 8400 the launch costs what the tiles save.
-bool stream_tiles(int64_t n, int64_t P, bool rbf) {
-  return !rbf && nacc_for(P) == 1 && n > 8960 && P > 24;
-}
-
-// The FP32 matvec of P vectors (a group of the launch's probes) from planes
-// of npb blocks of 32 probes; out: W, or the first of S partial planes of
-// wstride floats.
+// Slices [z0, z1) of the FP32 matvec of a plan; input: planes (tile 0's
+// place) or tiles; out: W, or the first of S partial planes of P n floats.
 template <bool RBF, int DIM>
-hipError_t launch_f32(hipStream_t s, const float* A, const RBFParams& prm, const u32x4* planes,
-                      int64_t plane_words, int64_t npb, const float* V, int64_t P, int64_t n,
-                      float* out, int64_t wstride, int S) {
-  const int nacc = nacc_for(P);
-  const dim3 grid(unsigned((n + BI - 1) / BI), unsigned((P + 32 * nacc - 1) / (32 * nacc)),
-                  unsigned(S));
-  if (nacc == 1) {
-    const dim3 wgrid(unsigned((n + 31) / 32), 1, unsigned(S));
-    if constexpr (!RBF) {
-      const float4* tiles = reinterpret_cast<const float4*>(planes);
-      if (stream_tiles(n, P, false))
-        hipLaunchKernelGGL(k_matvec_f32_stream<true>, wgrid, dim3(64 * kStreamWaves), 0, s, A,
-                           tiles, V, P, n, out, wstride);
-      else
-        hipLaunchKernelGGL(k_matvec_f32_stream<false>, wgrid, dim3(64 * kStreamWaves), 0, s, A,
-                           tiles, V, P, n, out, wstride);
-    }
-    else if (f32_planes(n, P, true))
-      hipLaunchKernelGGL((k_matvec_f32_wave<DIM, true>), wgrid, dim3(kThreads), 0, s, prm, planes,
+hipError_t launch_f32(hipStream_t s, const F32Plan& pl, const float* A, const RBFParams& prm,
+                      const u32x4* input, int64_t plane_words, const float* V, float* out, int z0,
+                      int z1) {
+  const int64_t n = pl.n, P = pl.P, wstride = P * n;
+  const dim3 rows(unsigned((n + 31) / 32), 1, unsigned(pl.S));
+  if (pl.form == F32Plan::kWorkgroup) {
+    const dim3 grid(unsigned((n + BI - 1) / BI), unsigned(pl.z.Ppad / (32 * pl.nacc)),
+                    unsigned(z1 - z0));
+    if (pl.nacc == 2)
+      hipLaunchKernelGGL((k_matvec_f32<2, RBF, DIM>), grid, dim3(kThreads), 0, s, A, prm, input,
+                         plane_words, pl.z.Ppad / 32, V, P, n, out, wstride, pl.S, z0);
+    else
+      hipLaunchKernelGGL((k_matvec_f32<4, RBF, DIM>), grid, dim3(kThreads), 0, s, A, prm, input,
+                         plane_words, pl.z.Ppad / 32, V, P, n, out, wstride, pl.S, z0);
+  } else if constexpr (RBF) {
+    if (pl.input == F32Plan::kPlanes)
+      hipLaunchKernelGGL((k_matvec_f32_wave<DIM, true>), rows, dim3(kThreads), 0, s, prm, input,
                          plane_words, V, P, n, out, wstride);
     else
-      hipLaunchKernelGGL((k_matvec_f32_wave<DIM, false>), wgrid, dim3(kThreads), 0, s, prm,
-                         planes, plane_words, V, P, n, out, wstride);
-  } else if (nacc == 2) {
-    hipLaunchKernelGGL((k_matvec_f32<2, RBF, DIM>), grid, dim3(kThreads), 0, s, A, prm, planes,
-                       plane_words, npb, V, P, n, out, wstride);
+      hipLaunchKernelGGL((k_matvec_f32_wave<DIM, false>), rows, dim3(kThreads), 0, s, prm, input,
+                         plane_words, V, P, n, out, wstride);
   } else {
-    hipLaunchKernelGGL((k_matvec_f32<4, RBF, DIM>), grid, dim3(kThreads), 0, s, A, prm, planes,
-                       plane_words, npb, V, P, n, out, wstride);
+    const float4* tiles = reinterpret_cast<const float4*>(input);
+    if (pl.input == F32Plan::kTiles)
+      hipLaunchKernelGGL(k_matvec_f32_stream<true>, rows, dim3(64 * kStreamWaves), 0, s, A, tiles,
+                         V, P, n, out, wstride);
+    else
+      hipLaunchKernelGGL(k_matvec_f32_stream<false>, rows, dim3(64 * kStreamWaves), 0, s, A, tiles,
+                         V, P, n, out, wstride);
   }
   return hipGetLastError();
 }
 
-hipError_t launch_f32_any(hipStream_t s, const slq_operator& op, const RBFParams& prm,
-                          const u32x4* planes, int64_t plane_words, int64_t npb, const float* V,
-                          int64_t P, float* out, int64_t wstride, int S) {
-  const int64_t n = op.n;
+hipError_t launch_f32_any(hipStream_t s, const slq_operator& op, const F32Plan& pl,
+                          const RBFParams& prm, const u32x4* input, int64_t plane_words,
+                          const float* V, float* out, int z0, int z1) {
   if (op.kind == SLQ_OP_DENSE)
-    return launch_f32<false, 1>(s, op.matrix, prm, planes, plane_words, npb, V, P, n, out, wstride,
-                                S);
+    return launch_f32<false, 1>(s, pl, op.matrix, prm, input, plane_words, V, out, z0, z1);
   switch (op.dim) {
     case 1:
-      return launch_f32<true, 1>(s, nullptr, prm, planes, plane_words, npb, V, P, n, out, wstride,
-                                 S);
+      return launch_f32<true, 1>(s, pl, nullptr, prm, input, plane_words, V, out, z0, z1);
     case 2:
-      return launch_f32<true, 2>(s, nullptr, prm, planes, plane_words, npb, V, P, n, out, wstride,
-                                 S);
+      return launch_f32<true, 2>(s, pl, nullptr, prm, input, plane_words, V, out, z0, z1);
     case 3:
-      return launch_f32<true, 3>(s, nullptr, prm, planes, plane_words, npb, V, P, n, out, wstride,
-                                 S);
+      return launch_f32<true, 3>(s, pl, nullptr, prm, input, plane_words, V, out, z0, z1);
     default:
-      return launch_f32<true, 4>(s, nullptr, prm, planes, plane_words, npb, V, P, n, out, wstride,
-                                 S);
+      return launch_f32<true, 4>(s, pl, nullptr, prm, input, plane_words, V, out, z0, z1);
   }
 }
 
@@ -2687,50 +2662,6 @@ hipError_t launch_bf16(hipStream_t s, const float* A, const u32x4* rec, const RB
     default:
       return launch_tpl_bf16<4, RBF>(s, A, rec, prm, Vhi, Vlo, Ppad, V, P, n, W, vec, nprod, S);
   }
-}
-
-// Split-K factor: enough workgroups for two per CU (256 CUs), as long as
-// every slice keeps at least 8 tiles and the partial sums fit the scratch.
-// The FP32 kernels for up to 32 probes use under 128 registers and hold four
-// waves per SIMD, so they get twice the workgroups (more waves to hide the
-// latency of their short per-tile chains).
-int choose_splitk(int64_t n, int64_t P, int64_t avail_floats, bool fp32) {
-  const int64_t nacc = nacc_for(P);
-  const int64_t wgs = ((n + BI - 1) / BI) * ((P + 32 * nacc - 1) / (32 * nacc));
-  const int64_t tiles = (n + BK - 1) / BK;
-  const int64_t target = (fp32 && nacc == 1) ? 1024 : 512;
-  int S = 1;
-  while (S < kMaxSplitK && wgs * S < target && tiles / (2 * S) >= 8 &&
-         int64_t(2 * S) * P * n <= avail_floats)
-    S *= 2;
-  return S;
-}
-
-// Column slices of the FP32 matvec, up to the factor above (which sizes the
-// scratch).  Workgroup form: the last round of resident workgroups (two per
-// CU) filled best.  Wave form: three per CU.  Stream form: one per CU runs
-// faster than two that share the CU's part of the bandwidth (n = 4096, 32
-// probes: 20 us in 256 workgroups, 27 in 512), so rounds of 256, by up to
-// three slices (10413: 1, 2, 3 slices take 143, 121, 117 us).
-int choose_splitk_f32(int64_t n, int64_t P, bool rbf) {
-  const int most = choose_splitk(n, P, int64_t(1) << 60, true);
-  const int64_t nacc = nacc_for(P);
-  const bool stream = nacc == 1 && !rbf;
-  const int64_t wgs = nacc == 1 ? (n + 31) / 32
-                                : (n + BI - 1) / BI * ((P + 32 * nacc - 1) / (32 * nacc));
-  const int64_t resident = stream ? 256 : (nacc == 1 ? 768 : 512);
-  if (stream && wgs <= resident) return int(std::min<int64_t>(most, resident / wgs));
-  int best = 1;
-  double fill = 0.0;
-  for (int S = 1; S <= (stream ? std::min(most, 3) : most); ++S) {
-    const double rounds = double(wgs * S) / double(resident);
-    const double f = rounds / std::ceil(rounds);
-    if (f > fill + 0.02) {
-      fill = f;
-      best = S;
-    }
-  }
-  return best;
 }
 
 // Derivative-kernel contraction: columns in launches of G column blocks of
@@ -2808,16 +2739,6 @@ hipError_t launch_pack_matrix(hipStream_t s, const float* A, int64_t n, int stor
 
 namespace {
 
-// Padded sizes of the planes of P probes.
-struct PlaneSizes {
-  int64_t npad, Ppad;
-  PlaneSizes(int64_t n, int64_t P) {
-    const int64_t bpw = 32 * nacc_for(P);
-    npad = (n + BK - 1) / BK * BK;
-    Ppad = (P + bpw - 1) / bpw * bpw;
-  }
-};
-
 bool rows_kernel(const slq_operator& op, int64_t P) {
   return op.kind == SLQ_OP_RBF && P <= kRowsMaxP && op.dim >= 1 && op.dim <= 4;
 }
@@ -2826,9 +2747,6 @@ bool packed_op(const slq_operator& op) {
 }
 bool fp32_op(const slq_operator& op) { return op.precision == SLQ_PREC_FP32 && !packed_op(op); }
 bool fp32_units_op(const slq_operator& op) { return op.precision == kPrecFp32Units; }
-
-// Floats of the FP32 matvec's three BF16 planes of `probes` (padded) probes.
-int64_t f32_plane_floats(int64_t npad, int64_t probes) { return 3 * npad * probes / 2; }
 
 }  // namespace
 
@@ -2861,15 +2779,13 @@ PlaneOut matvec_planes(const slq_operator& op, int64_t P, float* scratch, int64_
   if (rows_kernel(op, P) || fp32_units_op(op) || !scratch) return out;
   const PlaneSizes z(op.n, P);
   if (fp32_op(op)) {
-    // with less scratch the launch splits groups of probes by itself
-    const bool rbf = op.kind == SLQ_OP_RBF, tiled = stream_tiles(op.n, P, rbf);
-    if (!f32_planes(op.n, P, rbf) && !tiled) return out;
-    const int64_t S = choose_splitk_f32(op.n, P, op.kind == SLQ_OP_RBF);
-    if (f32_plane_floats(z.npad, z.Ppad) + S * P * op.n > scratch_floats) return out;
+    // with less scratch the launch splits the vectors pass by pass
+    const F32Plan pl(op.n, P, op.kind == SLQ_OP_RBF);
+    if (pl.input == F32Plan::kRows || !pl.whole(scratch_floats)) return out;
     out.Ppad = z.Ppad;
     out.hi = reinterpret_cast<__bf16*>(scratch);
     out.plane = z.Ppad * z.npad;
-    out.three = tiled ? 2 : 1;
+    out.three = pl.input == F32Plan::kTiles ? 2 : 1;
     return out;
   }
   out.Ppad = z.Ppad;
@@ -2984,42 +2900,34 @@ hipError_t launch_matvec(hipStream_t s, const slq_operator& op, const float* V, 
       hipLaunchKernelGGL(k_matvec_f32_units<4>, grid, dim3(kThreads), 0, s, op.matrix, V, P, n, out);
     err = hipGetLastError();
   } else if (fp32) {
-    // scratch layout: [three BF16 planes of a group of probes][split-K
-    // partial sums].  The group is every probe unless the scratch is the lean
-    // size, where the planes of a part of them fit at a time; a probe's
-    // result does not depend on the grouping.
-    S = choose_splitk_f32(n, P, op.kind == SLQ_OP_RBF);
-    const int64_t sums = S > 1 ? int64_t(S) * P * n : 0;
-    int64_t group = Ppad;
-    if (f32_plane_floats(npad, Ppad) + sums > scratch_floats) {
-      group = (scratch_floats - sums) / f32_plane_floats(npad, 1);
-      group = group >= 128 ? group / 128 * 128 : (group >= 64 ? 64 : group / 32 * 32);
-      if (group <= 0) return hipErrorInvalidValue;
-    }
-    u32x4* planes = reinterpret_cast<u32x4*>(scratch);
-    partial = scratch + f32_plane_floats(npad, group);
-    const bool rbf = op.kind == SLQ_OP_RBF, tiled = stream_tiles(n, P, rbf);
-    const bool ready =
-        !(f32_planes(n, P, rbf) || tiled) || ((flags & kMvPlanesReady) && group == Ppad);
+    // scratch layout: [the input's planes or tiles][split-K partial sums]; one
+    // pass over the slices unless the scratch is the least size
+    const F32Plan pl(n, P, op.kind == SLQ_OP_RBF);
+    S = pl.S;
+    partial = scratch + (scratch_floats - pl.sum_floats()) / 4 * 4;
+    u32x4* input = reinterpret_cast<u32x4*>(scratch);
+    const bool ready = pl.input == F32Plan::kRows ||
+                       ((flags & kMvPlanesReady) && pl.whole(scratch_floats));
     if (ready && ev0) (void)hipEventRecord(ev0, s);
-    for (int64_t p0 = 0; p0 < P && err == hipSuccess; p0 += group) {
-      const int64_t Pg = P - p0 < group ? P - p0 : group;
-      const PlaneSizes zg(n, Pg);
-      const int64_t words = zg.Ppad * npad / 8;
+    for (int z0 = 0, z1; z0 < S && err == hipSuccess; z0 = z1) {
+      z1 = pl.pass_end(z0, scratch_floats);
+      if (z1 == z0) return hipErrorInvalidValue;
+      const int64_t t0 = z1 - z0 < S ? pl.slice_tile(z0) : 0;
+      const int64_t t1 = z1 - z0 < S ? pl.slice_tile(z1) : npad / BK;
+      const int64_t words = (t1 - t0) * BK * Ppad / 8;  // of one plane
       if (!ready) {
-        int64_t blocks = (words + 255) / 256;
-        if (blocks > 8192) blocks = 8192;
-        if (tiled)
+        if (pl.input == F32Plan::kTiles)
           hipLaunchKernelGGL(k_tile_probes, dim3(unsigned((npad * 8 + 255) / 256)), dim3(256), 0, s,
-                             V, P, n, npad, reinterpret_cast<float4*>(planes));
-        else
-          hipLaunchKernelGGL(k_split3_probes, dim3(unsigned(blocks)), dim3(256), 0, s, V + p0 * n,
-                             Pg, n, zg.Ppad / 32, words, planes);
+                             V, P, n, npad, reinterpret_cast<float4*>(input));
+        else if (words > 0)
+          hipLaunchKernelGGL(k_split3_probes,
+                             dim3(unsigned(std::min<int64_t>((words + 255) / 256, 8192))),
+                             dim3(256), 0, s, V, P, n, Ppad / 32, t0, words, input);
         if ((err = hipGetLastError()) != hipSuccess) break;
-        if (p0 == 0 && ev0) (void)hipEventRecord(ev0, s);
+        if (z0 == 0 && ev0) (void)hipEventRecord(ev0, s);
       }
-      err = launch_f32_any(s, op, prm, planes, words, zg.Ppad / 32, V + p0 * n, Pg,
-                           (S > 1 ? partial : W) + p0 * n, P * n, S);
+      err = launch_f32_any(s, op, pl, prm, input - t0 * (Ppad / 32) * 128, words, V,
+                           S > 1 ? partial : W, z0, z1);
     }
   } else {
     // scratch layout: [BF16 planes, RBF point records][split-K partial sums]

@@ -1185,7 +1185,7 @@ int slq_logdet_noalloc(slq_context* ctx, const slq_operator* op, const float* Z,
   ForwardState st;
   int rc = logdet_forward(&sizing, *op, Z, P, k, per_probe, mean, alpha, beta, st);
   if (rc == SLQ_OK && sizing.arena_off > size_t(SLQ_NOALLOC_SCRATCH_BYTES)) {
-    // the least scratch: the same results
+    // the least scratch: the products in passes over their slices, the same bits
     slq_context least;
     least.device = ctx->device;
     least.stream = ctx->stream;

@@ -8,6 +8,7 @@
 #include <string>
 
 #include "../../include/slq.h"
+#include "matvec_plan.h"
 #include "slq_check.h"
 
 namespace slq {
@@ -47,9 +48,6 @@ __device__ __forceinline__ float ordered_sum(const float* __restrict__ v, int64_
 
 // ---- probes (k_probes.hip) -------------------------------------------------
 hipError_t launch_rademacher(hipStream_t s, uint32_t k0, uint32_t k1, int64_t count, float* out);
-
-// The FP32 matvec's planes hold V and -V in turns of this many 32-column tiles.
-constexpr int kPlaneSignRun = 2;
 
 // BF16 planes of the block matvec's input (tile-major, zero-padded; see
 // k_matvec.hip), written by the kernel that produces the input so that the
@@ -202,14 +200,10 @@ hipError_t launch_lanczos_adj_xi(hipStream_t s, const float* W, const float* lam
                                  const LanczosAdjStep& st, float* xi, float* part_out);
 
 // ---- block matvec (k_matvec.hip) -------------------------------------------
-// Largest split-K factor of the block matvec; its partial sums need up to
-// kMaxSplitK * P * n floats of scratch (matvec_scratch_floats sizes it for
-// the factor the launch will take).
-constexpr int kMaxSplitK = 16;
 // Scratch (in floats) the block matvec of op can use for P vectors: the
 // split-K partial sums and the BF16 planes of the vectors.  lean: the least
-// it works with (the FP32 matvec then splits its probes in groups, with the
-// same results).
+// it works with (the FP32 matvec may then go over its column slices in several
+// passes: the same kernels and sums, so the same bits).
 int64_t matvec_scratch_floats(const slq_operator& op, int64_t P, bool lean = false);
 // ev0 / ev1 (optional) are recorded on s right before and after the block
 // matvec kernel (the launches around it excluded).
