@@ -211,10 +211,11 @@ int slq_logdet(slq_context* ctx, const slq_operator* op, const float* Z, int64_t
  * from a static device array of SLQ_NOALLOC_SCRATCH_BYTES bytes per GPU (held
  * by each GPU the library runs on until the process ends) instead of the
  * context's pool; the call makes no hipMalloc/hipFree.  A call needing more
- * scratch than that (roughly 4 (k + 6) P n bytes) fails with SLQ_EINVAL
- * before anything is queued.  The array is located when the first context on
- * a device is created.  All calls on one GPU share its array: two calls whose work overlaps on the device
- * (different streams, or different contexts) race on it; serialise them. */
+ * scratch than that (roughly 4 (k + 6) P n bytes) fails with SLQ_EINVAL before
+ * anything is queued.  The array is located when the first context on
+ * a device is created.  All calls on one GPU share its array: two calls whose
+ * work overlaps on the device (different streams, or different contexts) race
+ * on it; serialise them. */
 #define SLQ_NOALLOC_SCRATCH_BYTES (256ull << 20)
 int slq_logdet_noalloc(slq_context* ctx, const slq_operator* op, const float* Z, int64_t P,
                        int64_t k, double* per_probe, double* mean, float* alpha, float* beta);

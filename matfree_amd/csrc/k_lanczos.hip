@@ -474,7 +474,7 @@ __device__ __forceinline__ void store_planes(const PlaneOut& pl, int64_t p, int6
 #pragma unroll
     for (int u = 0; u < V; ++u) {
       // every second run of tiles holds -V (k_matvec_f32)
-      const float x = (i / (32 * kPlaneSignRun)) & 1 ? -v[u] : v[u];
+      const float x = v[u] * ((i / (32 * kPlaneSignRun)) & 1 ? -kPlaneScale : kPlaneScale);
       q[0].b[u] = __bf16(x);
       const float r = x - float(q[0].b[u]);
       q[1].b[u] = __bf16(r);

@@ -6,7 +6,7 @@
 // probes), in three forms (which one: launch_f32):
 //
 //  * workgroup form (more than 32 probes): 128 rows x 64 or 128 probes, six
-//    products of three BF16 parts per factor; the probes' parts and the
+//    products of three BF16 parts per factor (k_matvec_f32); the probes' parts and the
 //    matrix tiles (or the tile's points) pass through LDS, an entry is formed
 //    once and used for every probe;
 //  * wave form (RBF, up to 32 probes): the same products, four waves sharing
@@ -371,6 +371,28 @@ __device__ __forceinline__ void wait_loads() {
 
 // Tiles of one plane sign (see k_matvec_f32).
 constexpr int kSignRun = kPlaneSignRun;
+
+// Both factors are split times this power of two, and the sums of products
+// taken back by its square: every FP32 number is a multiple of 2^-149, so the
+// scaled one is a multiple of BF16's least, 2^-133, and its three parts are
+// exact however small it is (without it the low parts of operands below 2^-110
+// were lost: 1e-36 came with a relative error of 1e-4).  Sums beyond 2^96 overflow
+// and take f32_block.
+constexpr float kSplitScale = kPlaneScale;
+constexpr float kSplitUnscale = 1.f / (kSplitScale * kSplitScale);
+
+// split_part of x kSplitScale for RBF entries (0 <= x <= 1), one integer add
+// for the pair's exponents instead of a product each (wave form, n = 32768, 32
+// probes, against the unscaled split: 1-D 7.2% longer with products, 4.6% so;
+// 3-D 2.9% and 1.9%).  An entry of 0 gets the high part 2^-111 and its negative as the
+// rest: far below what an entry under 2^-126, flushed to 0, leaves out.
+__device__ __forceinline__ float split_entries(float x0, float x1, uint32_t& word, float& r1) {
+  static_assert(kSplitScale == 65536.f, "16 in both exponent fields");
+  const uint32_t w = pack_bf16(x0, x1) + (uint32_t(16) << 23 | uint32_t(16) << 7);
+  word = w;
+  r1 = fmaf(x1, kSplitScale, -__builtin_bit_cast(float, w & 0xffff0000u));
+  return fmaf(x0, kSplitScale, -__builtin_bit_cast(float, w << 16));
+}
 __device__ __forceinline__ float tile_sign(int64_t kt) {
   return (kt / kSignRun) & 1 ? -1.f : 1.f;
 }
@@ -405,7 +427,7 @@ __global__ void __launch_bounds__(256)
           if (m + e < n) x[e] = src[e];
       }
     }
-    const float sgn = tile_sign(kt);
+    const float sgn = tile_sign(kt) * kSplitScale;
     u32x4 q[3];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -483,8 +505,7 @@ __device__ floatx16 f32_block(const float* __restrict__ A, const RBFParams& prm,
 // W = A V in FP32 from six BF16 products.  With a = a_h + a_m + a_l and
 // v = v_h + v_m + v_l (exact), a v = a_h v_h + (a_h v_m + a_m v_h) + (a_m v_m
 // + a_h v_l + a_l v_h) + dropped parts of at most 2^-26 |a v|, below the
-// rounding of one FP32 product; BF16 products are exact in FP32.  (Operands
-// below 2^-110 lose the parts that fall under BF16's subnormals.)  v_mfma
+// rounding of one FP32 product; BF16 products are exact in FP32.  v_mfma
 // 32x32x16 BF16 runs 16 times the FP32 matrix rate, so six products take 3/8
 // of the FP32 form's matrix cycles.  The stored row (or the generated RBF
 // entries) is split in registers, once per wave and tile; the probes' planes
@@ -659,14 +680,15 @@ __global__ void __launch_bounds__(kThreads, 2)
         if (DIM > 3) xm.w = comp(ga[DIM > 3 ? 3 : 0], m);
         ev[m] = rbf_entry<DIM>(xr, xm);
       } else {
-        ev[m] = comp(ga[0], m);
+        ev[m] = comp(ga[0], m) * kSplitScale;
       }
       return;
     }
     const int e = 2 * ((m - 4) >> 1);  // pair of the group
     const int kb = g >> 1, word = 2 * (g & 1) + e / 2;
     uint32_t w;
-    ev[e] = split_part(ev[e], ev[e + 1], w, ev[e + 1]);
+    ev[e] = RBF && (m & 1) == 0 ? split_entries(ev[e], ev[e + 1], w, ev[e + 1])
+                                : split_part(ev[e], ev[e + 1], w, ev[e + 1]);
     if ((m & 1) == 0) {
       nxt[0][kb][word] = w;
     } else {
@@ -720,7 +742,7 @@ __global__ void __launch_bounds__(kThreads, 2)
       }
       if (!RBF) {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[c][e] = fmaf(sgn, tmp[e], acc[c][e]);
+        for (int e = 0; e < 16; ++e) acc[c][e] = fmaf(sgn * kSplitUnscale, tmp[e], acc[c][e]);
       }
     }
   };
@@ -793,11 +815,11 @@ __global__ void __launch_bounds__(kThreads, 2)
     for (; kt + 1 < nwhole; kt += 2) {
       step(kt, 0, fA, fB);
       step(kt + 1, 1, fB, fA);
-      flush(tile_sign(kt_begin + kt));
+      flush(tile_sign(kt_begin + kt) * kSplitUnscale);
     }
     if (kt < nwhole) {
       step(kt, 0, fA, fB);
-      flush(tile_sign(kt_begin + kt));
+      flush(tile_sign(kt_begin + kt) * kSplitUnscale);
     }
   } else {
     while (kt + 1 < nwhole) {
@@ -858,8 +880,8 @@ __device__ __forceinline__ void split16(const float (&a)[16], float sgn, u32x4 (
   }
 }
 
-// acc + sgn times the six products of one tile with one block of 32 probes,
-// the tile's products in fresh registers (smallest first).
+// acc + sgn times the six products of one tile with one block of 32 probes
+// (both scaled), the tile's products in fresh registers (smallest first).
 __device__ __forceinline__ floatx16 block_products(const u32x4 (&f)[3][2], const u32x4 (&b)[3][2],
                                                    float sgn, floatx16 acc) {
   floatx16 tmp;
@@ -869,7 +891,7 @@ __device__ __forceinline__ floatx16 block_products(const u32x4 (&f)[3][2], const
 #pragma unroll
   for (int i = 0; i < 12; ++i) tmp = mfma_bf16(f[pa[i / 2]][i & 1], b[pb[i / 2]][i & 1], tmp);
 #pragma unroll
-  for (int e = 0; e < 16; ++e) acc[e] = fmaf(sgn, tmp[e], acc[e]);
+  for (int e = 0; e < 16; ++e) acc[e] = fmaf(sgn * kSplitUnscale, tmp[e], acc[e]);
   return acc;
 }
 
@@ -1026,7 +1048,16 @@ __global__ void __launch_bounds__(kThreads, 3)
         a[4 * g + m] = rbf_entry<DIM>(xr, make_float4(comp(0), comp(1), comp(2), comp(3)));
       }
     }
-    split16(a, 1.f, f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      uint32_t hi, mid;
+      float r1, q1;
+      const float r0 = split_entries(a[2 * e], a[2 * e + 1], hi, r1);
+      const float q0 = split_part(r0, r1, mid, q1);
+      f[0][e / 4][e % 4] = hi;
+      f[1][e / 4][e % 4] = mid;
+      f[2][e / 4][e % 4] = pack_bf16(q0, q1);
+    }
   };
   auto flush = [&] {
 #pragma unroll
@@ -1059,7 +1090,7 @@ __global__ void __launch_bounds__(kThreads, 3)
     u32x4 f[3][2];
     const float sgn = tile_sign(kt0 + 4 * i);
     fragment(buf, f);
-    if (!PLANES) split16(vc, sgn, bc);
+    if (!PLANES) split16(vc, sgn * kSplitScale, bc);
     acc = block_products(f, bc, sgn, acc);
     store_x(tile(i + 1), buf ^ 1, xn);
   };
@@ -1085,7 +1116,7 @@ __global__ void __launch_bounds__(kThreads, 3)
     store_x(kt, 0, xn);
     u32x4 f[3][2];
     fragment(0, f);
-    split16(va, sgn, bA);
+    split16(va, sgn * kSplitScale, bA);
     acc = block_products(f, bA, sgn, acc);
   }
   flush();

@@ -73,8 +73,10 @@ inline int choose_splitk_f32(int64_t n, int64_t P, bool rbf) {
   return best;
 }
 
-// Tiles of one plane sign (see k_matvec_f32).
+// The FP32 matvec's planes hold V and -V in turns of this many tiles (see
+// k_matvec_f32), times this power of two (see kSplitScale).
 constexpr int kPlaneSignRun = 2;
+constexpr float kPlaneScale = 65536.f;
 
 // Floats of the FP32 matvec's three BF16 planes of `probes` (padded) probes.
 inline int64_t f32_plane_floats(int64_t npad, int64_t probes) { return 3 * npad * probes / 2; }
