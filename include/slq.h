@@ -157,16 +157,24 @@ int slq_hessenberg(slq_context* ctx, const slq_operator* op, const float* V0, in
 /* slq_hessenberg with the forward's reorthogonalisation selectable:
  * reortho = 0 runs one classical Gram-Schmidt pass per step (the forward of
  * decomp.hessenberg(..., reortho_vjp="none"), decomp.py:394-396, 466-468),
- * reortho != 0 two (as slq_hessenberg). */
+ * reortho != 0 two (as slq_hessenberg).  SLQ_ARNOLDI_FP32_UNITS may be added:
+ * a stored FP32 matrix in FP32 precision is then multiplied on the FP32 matrix
+ * cores at every P (no effect on other operators).  The reverse pass multiplies
+ * the rounding of the basis it is taken at by a hundred to a thousand; a caller
+ * adds the flag to both calls where cotangents are to keep the values of those
+ * products. */
+#define SLQ_ARNOLDI_FP32_UNITS 0x40000000
 int slq_arnoldi(slq_context* ctx, const slq_operator* op, const float* V0, int64_t P, int64_t k,
                 int reortho, float* Q, float* H, float* R, float* c);
 
 /* Reverse mode of the Arnoldi decomposition for general output cotangents:
  * the custom VJP of decomp.hessenberg (decomp.py:398-422) and
- * _hessenberg_adjoint (decomp.py:480-600).  The forward pass on V0 (as
- * slq_arnoldi with `reortho`) is recomputed, then the adjoint runs with its
- * reorthogonalisation on (reortho_adjoint != 0, the reference's
- * reortho="full") or off.  Cotangents (device, any may be NULL = zero):
+ * _hessenberg_adjoint (decomp.py:480-600).  The forward pass on V0 is
+ * recomputed as slq_arnoldi with the same `reortho` (flag included), so the
+ * cotangents are taken at the decomposition which that call returned.  Then
+ * the adjoint runs with its reorthogonalisation on (reortho_adjoint != 0, the
+ * reference's reortho="full") or off.  Cotangents (device, any may be NULL =
+ * zero):
  *   dQ: k x P x n (the layout of slq_hessenberg's Q), dH: P x k x k
  *   (column-major like H), dr: P x n, dc: P.
  * Outputs: dv (P x n, cotangent of V0 = c lambda, decomp.py:602; may be

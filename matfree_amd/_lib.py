@@ -21,6 +21,8 @@ SLQ_EUNSUPPORTED = -5
 SLQ_EADJOINT_K0 = -6
 # bytes of the static device scratch of slq_logdet_noalloc (SLQ_NOALLOC_SCRATCH_BYTES)
 NOALLOC_SCRATCH_BYTES = 256 << 20
+# added to the reortho of slq_arnoldi and slq_arnoldi_vjp (SLQ_ARNOLDI_FP32_UNITS)
+ARNOLDI_FP32_UNITS = 0x40000000
 
 # operator kinds / precisions
 SLQ_OP_DENSE = 0

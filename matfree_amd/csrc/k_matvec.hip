@@ -1330,9 +1330,10 @@ __global__ void __launch_bounds__(64 * kStreamWaves, 3)
               [](float (&)[4]) {});
 }
 
-// FP32-unit form, for the forward pass that a reverse pass is taken at
-// (kPrecFp32Units): products and sums on the FP32 matrix cores, 128 rows per
-// workgroup, 32 per wave, the rows' fragments loaded a tile ahead by each
+// FP32-unit form, for a decomposition that is differentiated, in the forward
+// pass and where the reverse pass recomputes it (kPrecFp32Units): products and
+// sums on the FP32 matrix cores, 128 rows per workgroup, 32 per wave, the
+// rows' fragments loaded a tile ahead by each
 // wave, the probe tiles staged in LDS.  A general cotangent's reverse scan
 // multiplies the rounding of the basis it is taken at by a hundred to a
 // thousand (n = 1500, 32 steps: T good to 8e-8, the start vectors' cotangent

@@ -247,6 +247,14 @@ inline int64_t basis_stride(int64_t P, int64_t n) {
   return (P * n + 63) / 64 * 64 + kBasisSkew;
 }
 
+// The operator of slq_arnoldi's and slq_arnoldi_vjp's forward pass.
+slq_operator arnoldi_operator(slq_operator op, int reortho) {
+  if ((reortho & SLQ_ARNOLDI_FP32_UNITS) && op.kind == SLQ_OP_DENSE &&
+      op.storage == SLQ_STORE_FP32 && op.precision == SLQ_PREC_FP32)
+    op.precision = kPrecFp32Units;
+  return op;
+}
+
 // Forward Arnoldi (decomp.py:426-477) for P start vectors; see slq.h.
 // reortho = false: one classical Gram-Schmidt pass per step (the forward of
 // hessenberg(..., reortho_vjp="none"), decomp.py:466-468).
@@ -1066,7 +1074,8 @@ int slq_arnoldi(slq_context* ctx, const slq_operator* op, const float* V0, int64
   if (!V0 || !R || !c || (k > 0 && (!Q || !H)))
     return fail(ctx, SLQ_EINVAL, "input or output pointer is NULL");
   SLQ_TRY(set_device(ctx));
-  return hessenberg_core(ctx, *op, V0, P, k, Q, P * op->n, H, R, c, reortho != 0);
+  return hessenberg_core(ctx, arnoldi_operator(*op, reortho), V0, P, k, Q, P * op->n, H, R, c,
+                         (reortho & ~SLQ_ARNOLDI_FP32_UNITS) != 0);
 }
 
 int slq_arnoldi_vjp(slq_context* ctx, const slq_operator* op, const float* V0, int64_t P,
@@ -1093,11 +1102,8 @@ int slq_arnoldi_vjp(slq_context* ctx, const slq_operator* op, const float* V0, i
   SLQ_TRY(ensure_t(ctx, ctx->hmat, size_t(P * k * k), &st.H));
   SLQ_TRY(ensure_t(ctx, ctx->resid, size_t(P * n), &st.R));
   SLQ_TRY(ensure_t(ctx, ctx->scal1, size_t(P), &st.c));
-  // the cotangents move with the basis's rounding: see k_matvec_f32_units
-  slq_operator fwd = *op;
-  if (op->kind == SLQ_OP_DENSE && op->storage == SLQ_STORE_FP32 && op->precision == SLQ_PREC_FP32)
-    fwd.precision = kPrecFp32Units;
-  SLQ_TRY(hessenberg_core(ctx, fwd, V0, P, k, st.Q, st.ldc, st.H, st.R, st.c, reortho != 0));
+  SLQ_TRY(hessenberg_core(ctx, arnoldi_operator(*op, reortho), V0, P, k, st.Q, st.ldc, st.H, st.R,
+                          st.c, (reortho & ~SLQ_ARNOLDI_FP32_UNITS) != 0));
   Timed tm(ctx, SLQ_KC_ADJOINT);
   return arnoldi_reverse(ctx, *op, P, k, st, reortho_adjoint != 0, dQ, dH, dr, dc, dv, dparams,
                          dmatrix);

@@ -212,8 +212,7 @@ int64_t matvec_scratch_floats(const slq_operator& op, int64_t P, bool lean = fal
 // kMvPointsReady -- the RBF point records in the scratch are those of op
 // (a previous call with the same operator and scratch).
 // An internal precision of a stored FP32 matrix: the products on the FP32
-// matrix cores (k_matvec_f32_units), for the forward pass a reverse pass is
-// taken at.
+// matrix cores (k_matvec_f32_units; SLQ_ARNOLDI_FP32_UNITS).
 constexpr int32_t kPrecFp32Units = -1;
 constexpr int kMvPlanesReady = 1;
 constexpr int kMvPointsReady = 2;

@@ -18,7 +18,7 @@ from typing import Any, NamedTuple
 
 import torch
 
-from . import _runtime, _tree, operators
+from . import _lib, _runtime, _tree, operators
 
 
 class _DecompResult(NamedTuple):
@@ -37,7 +37,13 @@ def _error_num_matvecs(num, maxval, minval):
     return msg1 + msg2
 
 
-def _arnoldi_raw(op, V, k, params, reortho=True):
+def _reortho_flags(reortho, differentiated):
+    # differentiated: the forward and the one that slq_arnoldi_vjp recomputes take the same
+    # products, so that the cotangents are taken at the decomposition that was returned
+    return (1 if reortho else 0) | (_lib.ARNOLDI_FP32_UNITS if differentiated else 0)
+
+
+def _arnoldi_raw(op, V, k, params, reortho=True, differentiated=False):
     P, n = tuple(V.shape)
     if k < 0 or k > n:  # decomp.py:427-429
         raise ValueError(_error_num_matvecs(k, maxval=n, minval=0))
@@ -55,7 +61,7 @@ def _arnoldi_raw(op, V, k, params, reortho=True):
         _runtime.ptr(V),
         P,
         k,
-        1 if reortho else 0,
+        _reortho_flags(reortho, differentiated),
         _runtime.ptr(Q) if k > 0 else None,
         _runtime.ptr(Hc) if k > 0 else None,
         _runtime.ptr(R),
@@ -96,7 +102,7 @@ class _ArnoldiFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, matvec, k, reortho_fwd, reortho_adj, V, *params):
         op = operators.resolve(matvec)
-        Q, H, R, c = _arnoldi_raw(op, V.detach(), k, params, reortho_fwd)
+        Q, H, R, c = _arnoldi_raw(op, V.detach(), k, params, reortho_fwd, differentiated=True)
         ctx.op, ctx.k, ctx.reortho_fwd, ctx.reortho_adj = op, k, reortho_fwd, reortho_adj
         ctx.params = params
         ctx.save_for_backward(V)
@@ -118,7 +124,7 @@ class _ArnoldiFn(torch.autograd.Function):
         dRc, dcc = f32(dR), f32(dc)
         cx = _runtime.context(device)
         cx.call("slq_arnoldi_vjp", ctypes.byref(desc), _runtime.ptr(V32), P, k,
-                1 if ctx.reortho_fwd else 0, 1 if ctx.reortho_adj else 0,
+                _reortho_flags(ctx.reortho_fwd, True), 1 if ctx.reortho_adj else 0,
                 _runtime.ptr(dQc), _runtime.ptr(dHc), _runtime.ptr(dRc), _runtime.ptr(dcc),
                 _runtime.ptr(dv), _runtime.ptr(dparams), _runtime.ptr(dmatrix))
         del keep
