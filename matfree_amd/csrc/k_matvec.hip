@@ -1339,8 +1339,8 @@ __global__ void __launch_bounds__(64 * kStreamWaves, 3)
 // thousand (n = 1500, 32 steps: T good to 8e-8, the start vectors' cotangent
 // to 2e-6 .. 1e-4 from one matrix to the next), so any other order of these
 // sums gives another cotangent, no nearer and no further on average; the
-// scan's own products do not matter in that way.  n = 4096, 32 probes: 19 us,
-// as the stream form.
+// scan's own products do not matter in that way.  n = 4096, 32 probes: 22.5 us
+// (stream form 20), 10413: 144 us (117).
 constexpr int LDU = BK + 4;  // padded LDS row of floats
 
 template <int NACC>
@@ -1360,21 +1360,25 @@ __global__ void __launch_bounds__(kThreads)
   const int64_t mbase = kt_begin * BK;
   float* Wout = W + int64_t(blockIdx.z) * P * n;
 
-  // four values from column m of a row of n (zeros past it)
-  auto load4 = [&](const float* base, int64_t m) {
-    if (m + 4 <= n) return load4u(base + m);
+  // four values from column m of a row of n (zeros past it); a whole tile is
+  // read without a check (per group of four they took up to a third of the
+  // kernel's time), rows past n and probes past P as the last (not stored)
+  auto load4 = [&](const float* base, int64_t m, bool whole) {
+    if (whole) return load4u(base + m);
     return make_float4(m + 0 < n ? base[m + 0] : 0.f, m + 1 < n ? base[m + 1] : 0.f,
-                       m + 2 < n ? base[m + 2] : 0.f, 0.f);
+                       m + 2 < n ? base[m + 2] : 0.f, m + 3 < n ? base[m + 3] : 0.f);
   };
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
   // probe tile: thread t moves float4 t & 7 of probes t / 8 + 32 u
   float4 vreg[NACC], an[4], ac[4];
-  auto load_v = [&](int64_t m0) {
+  const float* vrow[NACC];
 #pragma unroll
-    for (int u = 0; u < NACC; ++u) {
-      const int64_t p = p0 + (t >> 3) + 32 * u;
-      vreg[u] = p < P ? load4(V + p * n, m0 + 4 * (t & 7)) : zero;
-    }
+  for (int u = 0; u < NACC; ++u) {
+    const int64_t p = p0 + (t >> 3) + 32 * u;
+    vrow[u] = V + (p < P ? p : P - 1) * n;
+  }
+  auto load_v = [&](int64_t m0, bool whole) {
+#pragma unroll
+    for (int u = 0; u < NACC; ++u) vreg[u] = load4(vrow[u], m0 + 4 * (t & 7), whole);
   };
   auto store_v = [&](int buf) {
 #pragma unroll
@@ -1382,9 +1386,10 @@ __global__ void __launch_bounds__(kThreads)
       *reinterpret_cast<float4*>(&Vs[buf][((t >> 3) + 32 * u) * LDU + 4 * (t & 7)]) = vreg[u];
   };
   // the lane's 16 values A[row][m0 + 16 h + 0 .. 15]
-  auto load_a = [&](int64_t m0) {
+  const float* arow = A + (row < n ? row : n - 1) * n;
+  auto load_a = [&](int64_t m0, bool whole) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) an[g] = row < n ? load4(A + row * n, m0 + 16 * h + 4 * g) : zero;
+    for (int g = 0; g < 4; ++g) an[g] = load4(arow, m0 + 16 * h + 4 * g, whole);
   };
 
   floatx16 acc[NACC];
@@ -1392,9 +1397,9 @@ __global__ void __launch_bounds__(kThreads)
   for (int c = 0; c < NACC; ++c)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[c][e] = 0.f;
-  load_v(mbase);
+  load_v(mbase, mbase + BK <= n);
   store_v(0);
-  load_a(mbase);
+  load_a(mbase, mbase + BK <= n);
   __syncthreads();
   for (int64_t kt = 0; kt < ntiles; ++kt) {
     const int buf = int(kt & 1);
@@ -1403,8 +1408,13 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
     for (int g = 0; g < 4; ++g) ac[g] = an[g];
     if (more) {
-      load_v(m0 + BK);
-      load_a(m0 + BK);
+      if (m0 + 2 * BK <= n) {
+        load_v(m0 + BK, true);
+        load_a(m0 + BK, true);
+      } else {
+        load_v(m0 + BK, false);
+        load_a(m0 + BK, false);
+      }
     }
     floatx16 tmp[NACC];
 #pragma unroll
