@@ -680,18 +680,19 @@ __global__ void __launch_bounds__(kThreads, 2)
         if (DIM > 3) xm.w = comp(ga[DIM > 3 ? 3 : 0], m);
         ev[m] = rbf_entry<DIM>(xr, xm);
       } else {
-        ev[m] = comp(ga[0], m) * kSplitScale;
+        ev[m] = comp(ga[0], m);
       }
       return;
     }
     const int e = 2 * ((m - 4) >> 1);  // pair of the group
     const int kb = g >> 1, word = 2 * (g & 1) + e / 2;
     uint32_t w;
-    ev[e] = RBF && (m & 1) == 0 ? split_entries(ev[e], ev[e + 1], w, ev[e + 1])
-                                : split_part(ev[e], ev[e + 1], w, ev[e + 1]);
     if ((m & 1) == 0) {
+      ev[e] = RBF ? split_entries(ev[e], ev[e + 1], w, ev[e + 1])
+                  : split_part(ev[e] * kSplitScale, ev[e + 1] * kSplitScale, w, ev[e + 1]);
       nxt[0][kb][word] = w;
     } else {
+      ev[e] = split_part(ev[e], ev[e + 1], w, ev[e + 1]);
       nxt[1][kb][word] = w;
       nxt[2][kb][word] = pack_bf16(ev[e], ev[e + 1]);
     }
@@ -834,15 +835,22 @@ __global__ void __launch_bounds__(kThreads, 2)
   }
   if (part) {
     load_b(nwhole, 0);
+    // every load is issued first (columns past n read the last one)
     const float* src = A + (row < n ? row : n - 1) * n;
+    float av[16];
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      const int64_t m = (all_tiles - 1) * BK + 16 * (s >> 3) + 8 * h + (s & 7);
+      av[s] = src[m < n ? m : n - 1];
+    }
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int64_t m = (all_tiles - 1) * BK + 16 * (g >> 1) + 8 * h + 4 * (g & 1);
       float4 ga[DIM];
-      ga[0].x = m < n ? src[m] : 0.f;
-      ga[0].y = m + 1 < n ? src[m + 1] : 0.f;
-      ga[0].z = m + 2 < n ? src[m + 2] : 0.f;
-      ga[0].w = m + 3 < n ? src[m + 3] : 0.f;
+      ga[0].x = m < n ? av[4 * g] : 0.f;
+      ga[0].y = m + 1 < n ? av[4 * g + 1] : 0.f;
+      ga[0].z = m + 2 < n ? av[4 * g + 2] : 0.f;
+      ga[0].w = m + 3 < n ? av[4 * g + 3] : 0.f;
 #pragma unroll
       for (int q = 0; q < 8; ++q) piece(g, q, ga, fA);
     }
@@ -2946,7 +2954,8 @@ hipError_t launch_matvec(hipStream_t s, const slq_operator& op, const float* V, 
     // pass over the slices unless the scratch is the least size
     const F32Plan pl(n, P, op.kind == SLQ_OP_RBF);
     S = pl.S;
-    partial = scratch + (scratch_floats - pl.sum_floats()) / 4 * 4;
+    partial = scratch + (pl.whole(scratch_floats) ? pl.input_floats()
+                                                  : (scratch_floats - pl.sum_floats()) / 4 * 4);
     u32x4* input = reinterpret_cast<u32x4*>(scratch);
     const bool ready = pl.input == F32Plan::kRows ||
                        ((flags & kMvPlanesReady) && pl.whole(scratch_floats));
