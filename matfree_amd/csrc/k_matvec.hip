@@ -903,14 +903,15 @@ __device__ __forceinline__ floatx16 block_products(const u32x4 (&f)[3][2], const
   return acc;
 }
 
-// The end of a 32-row, 32-probe workgroup: the sums of waves 0-3 are added in
-// the order of the waves (red: 16 KB of LDS, free) and written, with the nugget
-// where asked; check(o) may replace a thread's four values in between.
+// The end of a 32-row, 32-probe workgroup (probes p0 + 0..31): the sums of
+// waves 0-3 are added in the order of the waves (red: 16 KB of LDS, free) and
+// written, with the nugget where asked; check(o) may replace a thread's four
+// values in between.
 template <typename Check>
 __device__ __forceinline__ void store_block(float* red, const floatx16& sum, const RBFParams& prm,
                                             bool nugget, const float* __restrict__ V, int64_t P,
-                                            int64_t n, int64_t i0, float* __restrict__ W,
-                                            int64_t wstride, Check check) {
+                                            int64_t n, int64_t i0, int64_t p0,
+                                            float* __restrict__ W, int64_t wstride, Check check) {
   const int t = threadIdx.x;
   const int lane = t & 63, wave = t >> 6, r = lane & 31, h = lane >> 5;
   __syncthreads();
@@ -919,7 +920,7 @@ __device__ __forceinline__ void store_block(float* red, const floatx16& sum, con
     for (int e = 0; e < 16; ++e) red[(wave * 16 + e) * 64 + lane] = sum[e];
   }
   __syncthreads();
-  // thread t (waves 0-3): rows 8 wave + 4 h + 0..3 of probe r
+  // thread t (waves 0-3): rows 8 wave + 4 h + 0..3 of probe p0 + r
   float o[4] = {0.f, 0.f, 0.f, 0.f};
   if (wave < 4) {
 #pragma unroll
@@ -931,10 +932,10 @@ __device__ __forceinline__ void store_block(float* red, const floatx16& sum, con
     }
   }
   check(o);
-  float* out = W + int64_t(blockIdx.z) * wstride + int64_t(r) * n;
+  float* out = W + int64_t(blockIdx.z) * wstride + (p0 + r) * n;
   const int64_t io = i0 + 8 * wave + 4 * h;
-  if (wave < 4 && r < P) {
-    const float* vp = V + int64_t(r) * n;
+  if (wave < 4 && p0 + r < P) {
+    const float* vp = V + (p0 + r) * n;
     if (io + 4 <= n) {
       if (nugget) {
         const float4 v = load4u(vp + io);
@@ -953,7 +954,8 @@ __device__ __forceinline__ void store_block(float* red, const floatx16& sum, con
 }
 
 // Wave form, for the RBF kernel and up to 32 probes, where forming the entries
-// on the vector units is the bound: a workgroup owns 32 rows, its four waves
+// on the vector units is the bound, and for small problems of more (blocks of
+// 32 probes) and of a stored matrix: a workgroup owns 32 rows, its four waves
 // take every fourth tile of the slice and their sums are added at the end, so
 // that small problems still give every CU work.  PLANES: the probes' parts
 // come from the planes, one tile ahead in registers; otherwise (small n, where
@@ -961,25 +963,27 @@ __device__ __forceinline__ void store_block(float* red, const floatx16& sum, con
 // splits them itself.  Whole calls, FP32 MFMAs before: n = 10413, 2-D, 32
 // probes 95.5 -> 70.6 us; n = 32768, 3-D 792 -> 615; n = 2048, 16 probes
 // 16.4 -> 14.6 us.
-template <int DIM, bool PLANES>
+template <bool RBF, int DIM, bool PLANES>
 __global__ void __launch_bounds__(kThreads, 3)
-    k_matvec_f32_wave(RBFParams prm, const u32x4* __restrict__ planes, int64_t plane_words,
+    k_matvec_f32_wave(const float* __restrict__ A, RBFParams prm,
+                      const u32x4* __restrict__ planes, int64_t plane_words,
                       const float* __restrict__ V, int64_t P, int64_t n,
                       float* __restrict__ W, int64_t wstride) {
+  static_assert(!PLANES || RBF, "planes are read as one block of 32 probes");
   constexpr int kXW = (32 * DIM + 63) / 64;  // point coordinates per lane and tile
   __shared__ __attribute__((aligned(16))) float lds[4096];
   const int t = threadIdx.x;
   const int lane = t & 63, wave = t >> 6, r = lane & 31, h = lane >> 5;
   const int uwave = __builtin_amdgcn_readfirstlane(wave);
-  const int64_t i0 = int64_t(blockIdx.x) * 32;
-  const int64_t row = i0 + r;
+  const int64_t i0 = int64_t(blockIdx.x) * 32, p0 = int64_t(blockIdx.y) * 32;
+  const int64_t row = i0 + r, p = p0 + r;
   const int64_t all_tiles = (n + BK - 1) / BK;
   const int64_t runs = (all_tiles + kSignRun - 1) / kSignRun;
   const int64_t kt_begin = runs * blockIdx.z / gridDim.z * kSignRun;
   int64_t kt_end = runs * (blockIdx.z + 1) / gridDim.z * kSignRun;
   if (kt_end > all_tiles) kt_end = all_tiles;
   // the wave's tiles: kt_begin + uwave + 4 i, i < nw; without planes the last,
-  // partial tile of the vectors follows by itself with masked loads
+  // partial tile follows by itself with masked loads
   const bool part = !PLANES && kt_end == all_tiles && n % BK != 0;
   const int64_t kt_whole = part ? kt_end - 1 : kt_end;
   const int64_t kt0 = kt_begin + uwave;
@@ -995,14 +999,16 @@ __global__ void __launch_bounds__(kThreads, 3)
   float xr[4] = {0.f, 0.f, 0.f, 0.f};
   float xo[kXW];
   float* xs = lds + wave * (2 * DIM * BK);  // the wave's tile points, two buffers
+  if constexpr (RBF) {
 #pragma unroll
-  for (int d = 0; d < DIM; ++d) x0[d] = prm.X[d];
-  if (row < n) {
+    for (int d = 0; d < DIM; ++d) x0[d] = prm.X[d];
+    if (row < n) {
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) xr[d] = (prm.X[row * DIM + d] - x0[d]) * prm.scale;
+      for (int d = 0; d < DIM; ++d) xr[d] = (prm.X[row * DIM + d] - x0[d]) * prm.scale;
+    }
+#pragma unroll
+    for (int u = 0; u < kXW; ++u) xo[u] = prm.X[((64 * u + lane) >> 5) % DIM];
   }
-#pragma unroll
-  for (int u = 0; u < kXW; ++u) xo[u] = prm.X[((64 * u + lane) >> 5) % DIM];
   // coordinate ((64 u + lane) / 32) % DIM of point lane % 32 of tile kt
   auto load_x = [&](int64_t kt, float (&x)[kXW]) {
     const int64_t m = kt * BK + r;
@@ -1017,17 +1023,26 @@ __global__ void __launch_bounds__(kThreads, 3)
       xs[(buf * DIM + ((64 * u + lane) >> 5) % DIM) * BK + r] =
           ok ? (x[u] - xo[u]) * prm.scale : kFarPoint;
   };
-  // slots 8 kb + 0..7 of a lane: columns 16 kb + 8 h + 0..7 of tile kt; probes
-  // past P read probe P - 1 (not stored)
-  const float* vrow = V + (r < P ? r : P - 1) * n + 8 * h;
-  auto load_v = [&](int64_t kt, float (&a)[16]) {
+  // slots 8 kb + 0..7 of a lane: columns 16 kb + 8 h + 0..7 of tile kt, of its
+  // probe and of its matrix row; probes past P read probe P - 1, rows past n
+  // row n - 1 (not stored)
+  const float* vrow = V + (p < P ? p : P - 1) * n + 8 * h;
+  const float* arow = RBF ? nullptr : A + (row < n ? row : n - 1) * n + 8 * h;
+  auto load_row = [&](const float* src, int64_t kt, float (&a)[16]) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      const float4 v = load4u(vrow + kt * BK + 16 * (g >> 1) + 4 * (g & 1));
+      const float4 v = load4u(src + kt * BK + 16 * (g >> 1) + 4 * (g & 1));
       a[4 * g + 0] = v.x;
       a[4 * g + 1] = v.y;
       a[4 * g + 2] = v.z;
       a[4 * g + 3] = v.w;
+    }
+  };
+  auto load_part = [&](const float* src, int64_t kt, float (&a)[16]) {
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      const int col = 16 * (s >> 3) + (s & 7);
+      a[s] = kt * BK + 8 * h + col < n ? src[kt * BK + col] : 0.f;
     }
   };
   auto load_b = [&](int64_t kt, u32x4 (&b)[3][2]) {
@@ -1075,67 +1090,83 @@ __global__ void __launch_bounds__(kThreads, 3)
     }
   };
 
+  // the tile's entries: a tile's points, or the matrix values a[]
+  auto entries = [&](int buf, const float (&a)[16], u32x4 (&f)[3][2]) {
+    if constexpr (RBF)
+      fragment(buf, f);
+    else
+      split16(a, kSplitScale, f);
+  };
+
   u32x4 bA[3][2], bB[3][2];
-  float va[16], vb[16], xn[kXW];
+  float va[16], vb[16], aa[16], ab[16], xn[kXW];
   if (nw > 0) {
     if (PLANES)
       load_b(tile(0), bA);
     else
-      load_v(tile(0), va);
-    load_x(tile(0), xn);
-    store_x(tile(0), 0, xn);
+      load_row(vrow, tile(0), va);
+    if constexpr (RBF) {
+      load_x(tile(0), xn);
+      store_x(tile(0), 0, xn);
+    } else {
+      load_row(arow, tile(0), aa);
+    }
   }
   // Step i: the loads of the next tile are issued, then tile i's entries are
   // formed, split and multiplied.
   auto step = [&](int64_t i, int buf, u32x4 (&bc)[3][2], u32x4 (&bn)[3][2], const float (&vc)[16],
-                  float (&vn)[16]) {
+                  float (&vn)[16], const float (&ac)[16], float (&an)[16]) {
     if (PLANES)
       load_b(tile(i + 1), bn);
     else
-      load_v(tile(i + 1), vn);
-    load_x(tile(i + 1), xn);
+      load_row(vrow, tile(i + 1), vn);
+    if constexpr (RBF)
+      load_x(tile(i + 1), xn);
+    else
+      load_row(arow, tile(i + 1), an);
     __builtin_amdgcn_sched_barrier(0);
     u32x4 f[3][2];
     const float sgn = tile_sign(kt0 + 4 * i);
-    fragment(buf, f);
+    entries(buf, ac, f);
     if (!PLANES) split16(vc, sgn * kSplitScale, bc);
     acc = block_products(f, bc, sgn, acc);
-    store_x(tile(i + 1), buf ^ 1, xn);
+    if constexpr (RBF) store_x(tile(i + 1), buf ^ 1, xn);
   };
   int64_t i = 0;
   while (i + 1 < nw) {
     const int64_t stop = i + kTileRun < nw ? i + kTileRun : nw;
     for (; i + 1 < stop; i += 2) {
-      step(i, 0, bA, bB, va, vb);
-      step(i + 1, 1, bB, bA, vb, va);
+      step(i, 0, bA, bB, va, vb, aa, ab);
+      step(i + 1, 1, bB, bA, vb, va, ab, aa);
     }
     flush();
   }
-  if (i < nw) step(i, 0, bA, bB, va, vb);
+  if (i < nw) step(i, 0, bA, bB, va, vb, aa, ab);
   if (part && (all_tiles - 1 - kt_begin) % 4 == uwave) {
     const int64_t kt = all_tiles - 1;
     const float sgn = tile_sign(kt);
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      const int col = 16 * (s >> 3) + (s & 7);
-      va[s] = kt * BK + 8 * h + col < n ? vrow[kt * BK + col] : 0.f;
+    load_part(vrow, kt, va);
+    if constexpr (RBF) {
+      load_x(kt, xn);
+      store_x(kt, 0, xn);
+    } else {
+      load_part(arow, kt, aa);
     }
-    load_x(kt, xn);
-    store_x(kt, 0, xn);
     u32x4 f[3][2];
-    fragment(0, f);
+    entries(0, aa, f);
     split16(va, sgn * kSplitScale, bA);
     acc = block_products(f, bA, sgn, acc);
   }
   flush();
 
-  store_block(lds, sum, prm, gridDim.z == 1, V, P, n, i0, W, wstride, [&](float (&o)[4]) {
+  store_block(lds, sum, prm, RBF && gridDim.z == 1, V, P, n, i0, p0, W, wstride,
+              [&](float (&o)[4]) {
     bool bad = false;
 #pragma unroll
     for (int u = 0; u < 4; ++u) bad |= !(fabsf(o[u]) <= 3.4028235e38f);
-    if (__syncthreads_or(bad && r < P)) {
-      const floatx16 full = f32_block<true, DIM>(nullptr, prm, x0, xr, V, P, n, row, r, kt_begin,
-                                                 kt_end);
+    if (__syncthreads_or(bad && p < P)) {
+      const floatx16 full =
+          f32_block<RBF, DIM>(A, prm, x0, xr, V, P, n, row, p, kt_begin, kt_end);
 #pragma unroll
       for (int u = 0; u < 4; ++u)
         o[u] = wave == 0 ? full[u] : wave == 1 ? full[4 + u] : wave == 2 ? full[8 + u]
@@ -1334,7 +1365,7 @@ __global__ void __launch_bounds__(64 * kStreamWaves, 3)
     for (int e = 0; e < 16; ++e) sum[e] += acc[e];
   }
   RBFParams prm{};
-  store_block(reinterpret_cast<float*>(as), sum, prm, false, V, P, n, i0, W, wstride,
+  store_block(reinterpret_cast<float*>(as), sum, prm, false, V, P, n, i0, 0, W, wstride,
               [](float (&)[4]) {});
 }
 
@@ -2607,7 +2638,7 @@ hipError_t launch_f32(hipStream_t s, const F32Plan& pl, const float* A, const RB
                       const u32x4* input, int64_t plane_words, const float* V, float* out, int z0,
                       int z1) {
   const int64_t n = pl.n, P = pl.P, wstride = P * n;
-  const dim3 rows(unsigned((n + 31) / 32), 1, unsigned(pl.S));
+  const dim3 rows(unsigned((n + 31) / 32), unsigned((P + 31) / 32), unsigned(pl.S));
   if (pl.form == F32Plan::kWorkgroup) {
     const dim3 grid(unsigned((n + BI - 1) / BI), unsigned(pl.z.Ppad / (32 * pl.nacc)),
                     unsigned(z1 - z0));
@@ -2617,14 +2648,17 @@ hipError_t launch_f32(hipStream_t s, const F32Plan& pl, const float* A, const RB
     else
       hipLaunchKernelGGL((k_matvec_f32<4, RBF, DIM>), grid, dim3(kThreads), 0, s, A, prm, input,
                          plane_words, pl.z.Ppad / 32, V, P, n, out, wstride, pl.S, z0);
-  } else if constexpr (RBF) {
-    if (pl.input == F32Plan::kPlanes)
-      hipLaunchKernelGGL((k_matvec_f32_wave<DIM, true>), rows, dim3(kThreads), 0, s, prm, input,
-                         plane_words, V, P, n, out, wstride);
-    else
-      hipLaunchKernelGGL((k_matvec_f32_wave<DIM, false>), rows, dim3(kThreads), 0, s, prm, input,
-                         plane_words, V, P, n, out, wstride);
-  } else {
+  } else if (pl.form == F32Plan::kWave) {
+    if constexpr (RBF) {
+      if (pl.input == F32Plan::kPlanes) {
+        hipLaunchKernelGGL((k_matvec_f32_wave<true, DIM, true>), rows, dim3(kThreads), 0, s, A, prm,
+                           input, plane_words, V, P, n, out, wstride);
+        return hipGetLastError();
+      }
+    }
+    hipLaunchKernelGGL((k_matvec_f32_wave<RBF, DIM, false>), rows, dim3(kThreads), 0, s, A, prm,
+                       input, plane_words, V, P, n, out, wstride);
+  } else if constexpr (!RBF) {
     const float4* tiles = reinterpret_cast<const float4*>(input);
     if (pl.input == F32Plan::kTiles)
       hipLaunchKernelGGL(k_matvec_f32_stream<true>, rows, dim3(64 * kStreamWaves), 0, s, A, tiles,
@@ -2830,7 +2864,7 @@ PlaneOut matvec_planes(const slq_operator& op, int64_t P, float* scratch, int64_
   const PlaneSizes z(op.n, P);
   if (fp32_op(op)) {
     // with less scratch the launch splits the vectors pass by pass
-    const F32Plan pl(op.n, P, op.kind == SLQ_OP_RBF);
+    const F32Plan pl(op.n, P, op.kind == SLQ_OP_RBF, true);
     if (pl.input == F32Plan::kRows || !pl.whole(scratch_floats)) return out;
     out.Ppad = z.Ppad;
     out.hi = reinterpret_cast<__bf16*>(scratch);
@@ -2952,7 +2986,7 @@ hipError_t launch_matvec(hipStream_t s, const slq_operator& op, const float* V, 
   } else if (fp32) {
     // scratch layout: [the input's planes or tiles][split-K partial sums]; one
     // pass over the slices unless the scratch is the least size
-    const F32Plan pl(n, P, op.kind == SLQ_OP_RBF);
+    const F32Plan pl(n, P, op.kind == SLQ_OP_RBF, flags & kMvPlaned);
     S = pl.S;
     partial = scratch + (pl.whole(scratch_floats) ? pl.input_floats()
                                                   : (scratch_floats - pl.sum_floats()) / 4 * 4);

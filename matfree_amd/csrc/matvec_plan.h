@@ -46,26 +46,48 @@ inline int choose_splitk(int64_t n, int64_t P, int64_t avail_floats, bool fp32) 
   return S;
 }
 
+// More than 32 probes of a small problem take the wave form (blocks of 32
+// probes) as well.  The workgroup form there has a launch of its own for the
+// planes and a few workgroups, each a chain of tiles as long as the row (stored
+// n = 512, 64 probes: 23.0 us, wave form 7.0; RBF 23.8 and 7.7).  The wave
+// form's work grows with n^2 and the blocks, every block forming and splitting
+// the entries again: 2^25 is where the two meet (stored, wave and workgroup
+// form: n = 2048, 256 probes 33.1 and 36.3 us, 3700, 40: 27.2 and 34.7; beyond,
+// 4096, 40: 35.1 and 30.6, 3000, 128: 40.1 and 39.9, 2500, 256: 53.8 and 49.2).
+// planed: calls of a loop whose inputs come with their planes, which saves the
+// workgroup form 3.5 us; the two meet at three quarters of that (decomposition of
+// 20 steps: n = 2048, 256 probes 1023 and 983 us, 3500, 64: 733 and 838).
+inline bool wave_blocks(int64_t n, int64_t P, bool planed) {
+  const int64_t blocks = (P + 31) / 32, limit = planed ? int64_t(3) << 23 : int64_t(1) << 25;
+  return blocks > 1 && blocks <= 65535 && n < 4096 && n * n * blocks <= limit;
+}
+
 // Column slices of the FP32 matvec, up to the factor above (which sizes the
 // scratch).  Workgroup form: the last round of resident workgroups (two per
 // CU) filled best.  Wave form: three per CU.  Stream form: one per CU runs
 // faster than two that share the CU's part of the bandwidth (n = 4096, 32
 // probes: 20 us in 256 workgroups, 27 in 512), so rounds of 256, by up to
-// three slices (10413: 1, 2, 3 slices take 143, 121, 117 us).
-inline int choose_splitk_f32(int64_t n, int64_t P, bool rbf) {
+// three slices (10413: 1, 2, 3 slices take 143, 121, 117 us).  Blocks of the wave
+// form: rounds of 256 as well, by up to four (stored n = 2500, 128 probes: 1 to 4
+// slices take 37.0, 33.8, 32.3, 31.1 us; 2048, 64: 17.7, 13.4, 15.6, 14.8), RBF,
+// which computes more, of 512 (4095, 33 probes: 1 slice 33.1, 2 slices 31.0); more
+// of them only for a sixth more of the round, which their sum costs (stored
+// 2048, 224 probes: 1 slice 32.8, 4 slices 38.2).
+inline int choose_splitk_f32(int64_t n, int64_t P, bool rbf, bool planed) {
   const int most = choose_splitk(n, P, int64_t(1) << 60, true);
   const int64_t nacc = nacc_for(P);
-  const bool stream = nacc == 1 && !rbf;
+  const bool stream = nacc == 1 && !rbf, blocks = wave_blocks(n, P, planed);
   const int64_t wgs = nacc == 1 ? (n + 31) / 32
+                      : blocks  ? (n + 31) / 32 * ((P + 31) / 32)
                                 : (n + kMvRows - 1) / kMvRows * ((P + 32 * nacc - 1) / (32 * nacc));
-  const int64_t resident = stream ? 256 : (nacc == 1 ? 768 : 512);
+  const int64_t resident = stream || (blocks && !rbf) ? 256 : (nacc == 1 ? 768 : 512);
   if (stream && wgs <= resident) return int(std::min<int64_t>(most, resident / wgs));
   int best = 1;
   double fill = 0.0;
-  for (int S = 1; S <= (stream ? std::min(most, 3) : most); ++S) {
+  for (int S = 1; S <= std::min(most, stream ? 3 : blocks ? 4 : most); ++S) {
     const double rounds = double(wgs * S) / double(resident);
     const double f = rounds / std::ceil(rounds);
-    if (f > fill + 0.02) {
+    if (f > (blocks ? fill * 1.16 : fill + 0.02)) {
       fill = f;
       best = S;
     }
@@ -94,20 +116,22 @@ struct F32Plan {
   int nacc;  // workgroup form: blocks of 32 probes a workgroup
   int S;     // column slices
 
-  F32Plan(int64_t n_, int64_t P_, bool rbf) : n(n_), P(P_), z(n_, P_), nacc(nacc_for(P_)) {
-    form = nacc > 1 ? kWorkgroup : rbf ? kWave : kStream;
+  // planed: one of a loop of calls whose inputs come with their planes
+  F32Plan(int64_t n_, int64_t P_, bool rbf, bool planed)
+      : n(n_), P(P_), z(n_, P_), nacc(nacc_for(P_)) {
+    form = wave_blocks(n, P, planed) ? kWave : nacc > 1 ? kWorkgroup : rbf ? kWave : kStream;
     input = kRows;
     // The wave form reads rows at small n, where its waves split the vectors
     // themselves (the launch that writes the planes costs about 3.5 us,
     // splitting in the waves 0.2 us per 1000 columns).
-    if (form == kWorkgroup || (form == kWave && n >= 4096)) input = kPlanes;
+    if (form == kWorkgroup || (form == kWave && nacc == 1 && n >= 4096)) input = kPlanes;
     // The stream form's tiles are written by the producer of the input where
     // there is one, in a launch of about 3.5 us otherwise.  With up to 16
     // probes most of a tile is padding, and its lines cost more than the rows'
     // (15001, 16 probes: 199 -> 208 us); up to n = 8400 the launch costs what
     // the tiles save.
     if (form == kStream && n > 8960 && P > 24) input = kTiles;
-    S = choose_splitk_f32(n, P, rbf);
+    S = choose_splitk_f32(n, P, rbf, planed);
   }
 
   // First tile of slice z of the workgroup form: whole runs of one plane sign.

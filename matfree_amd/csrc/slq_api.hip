@@ -298,7 +298,8 @@ int hessenberg_core(slq_context* ctx, const slq_operator& op, const float* V0, i
     // split-K result is summed into w by the first dots pass (pend).
     {
       const auto ev = take_events(ctx, SLQ_KC_MATVEC);
-      const int flags = j == 0 ? 0 : (kMvPointsReady | (planes.hi ? kMvPlanesReady : 0));
+      const int flags =
+          kMvPlaned | (j == 0 ? 0 : (kMvPointsReady | (planes.hi ? kMvPlanesReady : 0)));
       SLQ_HIP(ctx, launch_matvec(s, op, qj, P, w, mvs, mv_floats, ev.first, ev.second, flags,
                                  &pend));
     }
@@ -405,7 +406,8 @@ int lanczos_core(slq_context* ctx, const slq_operator& op, const float* V0, int6
     const float* qm = j > 0 ? vec(j - 1) : nullptr;
     {
       const auto ev = take_events(ctx, SLQ_KC_MATVEC);
-      const int flags = j == 0 ? 0 : (kMvPointsReady | (planes.hi ? kMvPlanesReady : 0));
+      const int flags =
+          kMvPlaned | (j == 0 ? 0 : (kMvPointsReady | (planes.hi ? kMvPlanesReady : 0)));
       SLQ_HIP(ctx, launch_matvec(s, op, q, P, w, mvs, mv_floats, ev.first, ev.second, flags,
                                  &pend));
     }
@@ -576,6 +578,7 @@ struct AdjointMatvec {
   hipError_t run(hipStream_t s, const float* x, float* w, const float* Q, int64_t ldc, int ncols,
                  float* part, int pstride, bool projected) {
     int flags = first ? 0 : kMvPointsReady;
+    if (projected && planes.hi && op.n % 4 == 0) flags |= kMvPlaned;
     if (projected && planes_out()) flags |= kMvPlanesReady;
     first = false;
     MvSplitSum pend;

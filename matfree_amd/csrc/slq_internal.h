@@ -210,19 +210,23 @@ int64_t matvec_scratch_floats(const slq_operator& op, int64_t P, bool lean = fal
 // flags: kMvPlanesReady -- the scratch planes already hold V (written by a
 // PlaneOut producer after a call that split them, so the padding is zero);
 // kMvPointsReady -- the RBF point records in the scratch are those of op
-// (a previous call with the same operator and scratch).
+// (a previous call with the same operator and scratch);
+// kMvPlaned -- one of a loop of calls whose later inputs come with the planes
+// of matvec_planes (given to all of them, so that they take one form).
 // An internal precision of a stored FP32 matrix: the products on the FP32
 // matrix cores (k_matvec_f32_units; SLQ_ARNOLDI_FP32_UNITS).
 constexpr int32_t kPrecFp32Units = -1;
 constexpr int kMvPlanesReady = 1;
 constexpr int kMvPointsReady = 2;
+constexpr int kMvPlaned = 4;
 // With defer non-null a split-K result is not reduced into W; *defer
 // describes it instead (W is then not written).
 hipError_t launch_matvec(hipStream_t s, const slq_operator& op, const float* V, int64_t P,
                          float* W, float* scratch, int64_t scratch_floats,
                          hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr, int flags = 0,
                          MvSplitSum* defer = nullptr);
-// The planes launch_matvec reads for (op, P) in a scratch of this size.
+// The planes launch_matvec reads for (op, P) in a scratch of this size with
+// kMvPlaned.
 PlaneOut matvec_planes(const slq_operator& op, int64_t P, float* scratch, int64_t scratch_floats);
 // Packed storage of a stored matrix (slq_storage): sizes (false for FP32 or
 // an unknown storage) and the packing kernel.
