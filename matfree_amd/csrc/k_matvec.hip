@@ -1194,147 +1194,193 @@ __global__ void __launch_bounds__(256)
 // Stream form, for a stored matrix and up to 32 probes: the matrix's bytes are
 // the bound, and with one probe block per entry the FP32 matrix cores (1024
 // cycles a tile) keep up with HBM while splitting the entries for the BF16
-// ones does not.  A workgroup owns 32 rows, four waves multiply one tile each
-// of a block of 32 rows x 128 columns, and a fifth wave does nothing but load
-// the blocks to LDS, four ahead of the one in use.  Loads finish in the order
-// of issue within a wave, so a wave that loads both the matrix and the vectors
-// would wait for all of its matrix loads whenever it needs a vector; the
-// loader keeps up to 64 KB per workgroup in flight (two workgroups fill the
-// CU's LDS).  A row's piece of a block is 512 contiguous bytes: unaligned rows
-// read in the 128-byte rows of a tile reach 4.2 TB/s, in these pieces 4.9.
+// ones does not.  A workgroup works on 32 rows at a time, four waves multiply
+// one tile each of a block of 32 rows x 128 columns, and a fifth wave does
+// nothing but load the blocks to LDS, four ahead of the one in use.  Loads
+// finish in the order of issue within a wave, so a wave that loads both the
+// matrix and the vectors would wait for all of its matrix loads whenever it
+// needs a vector; the loader keeps up to 64 KB in flight.  A row's piece of a
+// block is 512 contiguous bytes: unaligned rows read in the 128-byte rows of a
+// tile reach 4.2 TB/s, in these pieces 4.9 and more.
+// One workgroup a CU: up to n = 4096 a row block, or a slice of one, each;
+// beyond, every workgroup takes an equal share of all blocks, through as many
+// row blocks as it reaches into (`even`; each row block's segments are planes
+// of the split sum), and the loader runs on into the next row block.  In
+// rounds of row blocks the last one left up to half of the CUs idle: 16 vectors,
+// n = 4224 27.7 -> 21.9 us, 8448 79.5 -> 58.4, 8960 87.6 -> 71.4, 10413 107 ->
+// 99, 16384 220 -> 218.
 // TILED: the vectors in the order of the fragments (k_tile_probes).  A lane's own
 // row in 16-byte pieces touches 32 rows an instruction, which the L1 takes one
 // at a time.  Decomposition of depth 8 with 32 probes, without: n = 10413 1108 ->
-// 1060 us, 15001 1927 -> 1766, 16384 2024 -> 1941; a single product 222 -> 212 us
-// at 15001.
+// 1060 us, 15001 1927 -> 1766, 16384 2024 -> 1941.
 // Whole calls with 32 probes, each wave loading its own rows before: n = 10413
-// 149 -> 117 us, 15001 271 -> 216, 4096 23.6 -> 19.7, 16384 225 -> 232 us.
+// 147 -> 108 us, 15000 247 -> 207, 4096 23.4 -> 19.6, 16384 230 -> 222.
 constexpr int kStreamWaves = 5;
 constexpr int kStreamStages = 5;
 template <bool TILED>
-__global__ void __launch_bounds__(64 * kStreamWaves, 3)
+__global__ void __launch_bounds__(64 * kStreamWaves, 2)
     k_matvec_f32_stream(const float* __restrict__ A, const float4* __restrict__ tiles,
                         const float* __restrict__ V, int64_t P, int64_t n, float* __restrict__ W,
-                        int64_t wstride) {
-  constexpr int kBlockTiles = 4;
+                        int64_t wstride, int S, bool even) {
   __shared__ __attribute__((aligned(16))) float4 as[kStreamStages * 1024];
+  __shared__ __attribute__((aligned(16))) float red[4096];
   const int t = threadIdx.x;
   const int lane = t & 63, wave = t >> 6, r = lane & 31, h = lane >> 5;
   const int uwave = __builtin_amdgcn_readfirstlane(wave);
-  const int64_t i0 = int64_t(blockIdx.x) * 32;
-  const int64_t all_tiles = (n + BK - 1) / BK;
-  const int64_t runs = (all_tiles + kBlockTiles - 1) / kBlockTiles;
-  const int64_t kt_begin = runs * blockIdx.z / gridDim.z * kBlockTiles;
-  int64_t kt_end = runs * (blockIdx.z + 1) / gridDim.z * kBlockTiles;
-  if (kt_end > all_tiles) kt_end = all_tiles;
-  // the matrix's last, partial tile follows by itself with masked loads
-  const bool part = kt_end == all_tiles && n % BK != 0;
-  const int64_t nwhole = kt_end - kt_begin - (part ? 1 : 0);
-  const int64_t nblocks = (nwhole + kBlockTiles - 1) / kBlockTiles;
+  const int64_t all_tiles = (n + BK - 1) / BK, runs = stream_runs(n);
+  const int64_t g = blockIdx.x, z = blockIdx.z;
+  // `count` blocks from block k0 of row block rb0 on
+  int64_t rb0 = g, k0 = uint32_t(runs * z) / uint32_t(S);
+  int64_t count = uint32_t(runs * (z + 1)) / uint32_t(S) - k0;
+  if (even) {
+    const int64_t u0 = stream_split(n, gridDim.x, g);
+    count = stream_split(n, gridDim.x, g + 1) - u0;
+    rb0 = u0 / runs;
+    k0 = u0 - rb0 * runs;
+  }
 
-  // The i-th block in the workgroup's order: every row block starts at another
-  // one, since rows a multiple of 4 KB apart have a column of every row on the
-  // same memory channel (32 probes, n = 16384: 258 -> 232 us, 12288: 148 -> 139,
-  // other n the same).
-  const int64_t rot = nblocks > 1 ? int64_t(blockIdx.x) % nblocks : 0;
-  auto order = [&](int64_t i) {
-    const int64_t b = i + rot;
-    return b < nblocks ? b : b - nblocks;
+  // The i-th block of a segment in the workgroup's order: every row block
+  // starts at another one, since rows a multiple of 4 KB apart have a column of
+  // every row on the same memory channel (32 probes, n = 16384: 258 -> 232 us,
+  // 12288: 148 -> 139, other n the same).
+  auto rotation = [](const StreamSegment& sg) {
+    return sg.nblocks > 1 ? int(uint32_t(sg.rb) % uint32_t(sg.nblocks)) : 0;
+  };
+  auto order = [](int i, int rot, int nblocks) {
+    return i + rot < nblocks ? i + rot : i + rot - nblocks;
   };
 
-  floatx16 sum;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) sum[e] = 0.f;
   if (uwave == kStreamWaves - 1) {
+    // The next block to load: block lb of segment ls, after which `later` blocks
+    // follow, or none.
+    StreamSegment ls = stream_segment(n, rb0, k0, count);
+    int64_t later = count;
+    int lb = 0, lblocks = 0, rot = 0;
+    const int rr = lane >> 5;
+    const char* src[16];
+    auto enter = [&] {
+      later -= ls.k1 - ls.k0;
+      lb = 0;
+      lblocks = int(ls.nblocks);
+      rot = rotation(ls);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const int64_t i = ls.rb * 32 + 2 * u + rr;
+        src[u] = reinterpret_cast<const char*>(A + (i < n ? i : n - 1) * n);
+      }
+    };
+    auto settle = [&] {
+      while (lb >= lblocks && later > 0) {
+        ls = stream_segment(n, ls.rb + 1, 0, later);
+        enter();
+      }
+    };
+    enter();
     // instruction u of a block: rows 2 u, 2 u + 1; piece q of a row goes to
     // slot q ^ (row & 7) (conflict-free fragment reads).  Pieces past the
     // row's last whole one are clamped (their tile is not whole), rows past n
-    // read row n - 1, blocks past the last one the last.
-    const uint32_t last = uint32_t(n - 4 - kt_begin * BK) * 4;
-    const int rr = lane >> 5;
-    auto load_block = [&](int64_t b, int stage) {
-      const uint32_t c0 = uint32_t(order(b < nblocks ? b : nblocks - 1)) * (kBlockTiles * BK * 4);
+    // read row n - 1; after the last block the row's first columns are loaded
+    // (to a stage nobody reads), so that as many loads stay in flight.
+    const uint32_t last = uint32_t(n - 4) * 4;
+    auto load_block = [&](int stage) {
+      const uint32_t c0 =
+          lb < lblocks
+              ? (uint32_t(ls.tile0) + uint32_t(order(lb, rot, lblocks)) * kStreamTiles) * (BK * 4)
+              : 0;
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
-        const int64_t i = i0 + 2 * u + rr;
         const uint32_t c = c0 + 16u * uint32_t((lane & 31) ^ ((2 * u + rr) & 7));
-        const char* src = reinterpret_cast<const char*>(A + (i < n ? i : n - 1) * n +
-                                                        kt_begin * BK);
-        __builtin_amdgcn_global_load_lds((GlobalPtr)(src + (c < last ? c : last)),
+        __builtin_amdgcn_global_load_lds((GlobalPtr)(src[u] + (c < last ? c : last)),
                                          (LdsPtr)(as + stage * 1024 + 64 * u), 16, 0, 0);
       }
+      ++lb;
+      settle();
     };
-    if (nblocks > 0) {
+    settle();
+    if (lb < lblocks) {
 #pragma unroll
-      for (int b = 0; b < kStreamStages - 1; ++b) load_block(b, b);
-      int stage = kStreamStages - 1;
-      for (int64_t b = 0; b < nblocks; ++b) {
-        wait_loads<16 * (kStreamStages - 2)>();  // block b is in LDS
+      for (int b = 0; b < kStreamStages - 1; ++b) load_block(b);
+    }
+    int stage = kStreamStages - 1;
+    int64_t rb = rb0, k = k0;
+    for (int64_t left = count; left > 0;) {
+      const StreamSegment sg = stream_segment(n, rb, k, left);
+      for (int b = 0; b < int(sg.nblocks); ++b) {
+        wait_loads<16 * (kStreamStages - 2)>();  // the block is in LDS
         // (a bare barrier: __syncthreads() waits for every load to LDS)
-        __builtin_amdgcn_s_barrier();  // and block b - 1 is free
+        __builtin_amdgcn_s_barrier();  // and the one before is free
         __builtin_amdgcn_sched_barrier(0);
-        load_block(b + kStreamStages - 1, stage);
+        load_block(stage);
         stage = stage == kStreamStages - 1 ? 0 : stage + 1;
       }
+      __builtin_amdgcn_s_barrier();  // store_block's two
+      __builtin_amdgcn_s_barrier();
+      left -= sg.k1 - sg.k0;
+      ++rb;
+      k = 0;
     }
     wait_loads<0>();
-  } else {
-    // An MFMA carries two contraction indices, one per lane half: half h walks
-    // columns 16 h .. 16 h + 15 of the tile for both operands.  Probes past P
-    // read probe P - 1 (not stored).
-    floatx16 acc;
+    return;
+  }
+
+  // An MFMA carries two contraction indices, one per lane half: half h walks
+  // columns 16 h .. 16 h + 15 of the tile for both operands.  Probes past P
+  // read probe P - 1 (not stored).
+  floatx16 acc, sum;
+  const float* vrow = V + (r < P ? r : P - 1) * n + 16 * h;
+  auto load_v = [&](int64_t kt, float4 (&v)[4]) {
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-    const float* vrow = V + (r < P ? r : P - 1) * n + kt_begin * BK + 16 * h;
-    auto load_v = [&](int64_t kt, float4 (&v)[4]) {
+    for (int q = 0; q < 4; ++q)
+      v[q] = TILED ? tiles[(kt * 4 + q) * 64 + lane] : load4u(vrow + kt * BK + 4 * q);
+  };
+  auto tile_products = [&](const float4 (&a)[4], const float4 (&v)[4]) {
+    floatx16 tmp;
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
-        v[g] = TILED ? tiles[((kt_begin + kt) * 4 + g) * 64 + lane] : load4u(vrow + kt * BK + 4 * g);
-    };
-    auto tile_products = [&](const float4 (&a)[4], const float4 (&v)[4]) {
-      floatx16 tmp;
+    for (int e = 0; e < 16; ++e) tmp[e] = 0.f;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) tmp[e] = 0.f;
+    for (int q = 0; q < 4; ++q) {
+      tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].x, v[q].x, tmp, 0, 0, 0);
+      tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].y, v[q].y, tmp, 0, 0, 0);
+      tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].z, v[q].z, tmp, 0, 0, 0);
+      tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].w, v[q].w, tmp, 0, 0, 0);
+    }
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].x, v[g].x, tmp, 0, 0, 0);
-        tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].y, v[g].y, tmp, 0, 0, 0);
-        tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].z, v[g].z, tmp, 0, 0, 0);
-        tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].w, v[g].w, tmp, 0, 0, 0);
-      }
+    for (int e = 0; e < 16; ++e) acc[e] += tmp[e];
+  };
+  int stage = 0;
+  auto next = [&] { stage = stage == kStreamStages - 1 ? 0 : stage + 1; };
+  int64_t rb = rb0, k = k0;
+  for (int64_t left = count; left > 0;) {
+    const StreamSegment sg = stream_segment(n, rb, k, left);
+    const int64_t i0 = sg.rb * 32;
+    const int nblocks = int(sg.nblocks), nwhole = int(sg.nwhole), rot = rotation(sg);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[e] += tmp[e];
-    };
+    for (int e = 0; e < 16; ++e) acc[e] = sum[e] = 0.f;
     // Block b: its fragment is read from LDS and its vectors loaded while the
     // products of the block before run.
     float4 aA[4], aB[4], vA[4], vB[4];
     bool live = false;  // the tile read last exists (the last block may miss some)
-    auto block = [&](int64_t b, int stage, const float4 (&ac)[4], float4 (&an)[4],
-                     const float4 (&vc)[4], float4 (&vn)[4]) {
-      const int64_t kt = order(b) * kBlockTiles + uwave;
+    auto block = [&](int b, const float4 (&ac)[4], float4 (&an)[4], const float4 (&vc)[4],
+                     float4 (&vn)[4]) {
+      const int kt = order(b, rot, nblocks) * kStreamTiles + uwave;
       __syncthreads();
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int q = 8 * uwave + 4 * h + g;
-        an[g] = as[stage * 1024 + r * 32 + (q ^ (r & 7))];
-      }
-      load_v(kt < nwhole ? kt : nwhole - 1, vn);
+      for (int q = 0; q < 4; ++q)
+        an[q] = as[stage * 1024 + r * 32 + ((8 * uwave + 4 * h + q) ^ (r & 7))];
+      load_v(sg.tile0 + (kt < nwhole ? kt : nwhole - 1), vn);
       __builtin_amdgcn_sched_barrier(0);
       if (live) tile_products(ac, vc);
       live = kt < nwhole;
+      next();
     };
-    int stage = 0;
-    int64_t b = 0;
-    auto next = [&] { stage = stage == kStreamStages - 1 ? 0 : stage + 1; };
+    int b = 0;
     while (b < nblocks) {
-      const int64_t stop = b + kTileRun < nblocks ? b + kTileRun : nblocks;
+      const int stop = b + kTileRun < nblocks ? b + kTileRun : nblocks;
       for (; b + 1 < stop; b += 2) {
-        block(b, stage, aB, aA, vB, vA);
-        next();
-        block(b + 1, stage, aA, aB, vA, vB);
-        next();
+        block(b, aB, aA, vB, vA);
+        block(b + 1, aA, aB, vA, vB);
       }
-      if (b < stop) break;  // the slice's odd last block
+      if (b < stop) break;  // the segment's odd last block
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         sum[e] += acc[e];
@@ -1342,31 +1388,45 @@ __global__ void __launch_bounds__(64 * kStreamWaves, 3)
       }
     }
     if (b < nblocks) {
-      block(b, stage, aB, aA, vB, vA);
+      block(b, aB, aA, vB, vA);
       if (live) tile_products(aA, vA);
     } else if (nblocks > 0 && live) {
       tile_products(aB, vB);
     }
-    if (part && (all_tiles - 1) % 4 == uwave) {
+    if (sg.part && (all_tiles - 1) % 4 == uwave) {
       const int64_t m0 = (all_tiles - 1) * BK + 16 * h;
       const float* src = A + (i0 + r < n ? i0 + r : n - 1) * n;
       const float* vp = V + (r < P ? r : P - 1) * n;
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int64_t m = m0 + 4 * g;
-        aA[g] = make_float4(m < n ? src[m] : 0.f, m + 1 < n ? src[m + 1] : 0.f,
+      for (int q = 0; q < 4; ++q) {
+        const int64_t m = m0 + 4 * q;
+        aA[q] = make_float4(m < n ? src[m] : 0.f, m + 1 < n ? src[m + 1] : 0.f,
                            m + 2 < n ? src[m + 2] : 0.f, m + 3 < n ? src[m + 3] : 0.f);
-        vA[g] = make_float4(m < n ? vp[m] : 0.f, m + 1 < n ? vp[m + 1] : 0.f,
+        vA[q] = make_float4(m < n ? vp[m] : 0.f, m + 1 < n ? vp[m + 1] : 0.f,
                             m + 2 < n ? vp[m + 2] : 0.f, m + 3 < n ? vp[m + 3] : 0.f);
       }
       tile_products(aA, vA);
     }
 #pragma unroll
     for (int e = 0; e < 16; ++e) sum[e] += acc[e];
+    const int plane = even ? stream_plane(n, gridDim.x, g, sg.rb) : int(z);
+    store_block(red, sum, RBFParams{}, false, V, P, n, i0, 0, W + plane * wstride, 0,
+                [](float (&)[4]) {});
+    // a row block of fewer segments than planes: zeros in the others
+    if (even && sg.k1 == runs) {
+      for (int q = plane + 1; q < S; ++q) {
+        float* out = W + q * wstride + int64_t(r) * n;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int64_t i = i0 + 8 * uwave + 4 * h + e;
+          if (r < P && i < n) out[i] = 0.f;
+        }
+      }
+    }
+    left -= sg.k1 - sg.k0;
+    ++rb;
+    k = 0;
   }
-  RBFParams prm{};
-  store_block(reinterpret_cast<float*>(as), sum, prm, false, V, P, n, i0, 0, W, wstride,
-              [](float (&)[4]) {});
 }
 
 // FP32-unit form, for a decomposition that is differentiated, in the forward
@@ -2660,12 +2720,13 @@ hipError_t launch_f32(hipStream_t s, const F32Plan& pl, const float* A, const RB
                        input, plane_words, V, P, n, out, wstride);
   } else if constexpr (!RBF) {
     const float4* tiles = reinterpret_cast<const float4*>(input);
+    const dim3 grid = pl.even ? dim3(unsigned(pl.even)) : rows;
     if (pl.input == F32Plan::kTiles)
-      hipLaunchKernelGGL(k_matvec_f32_stream<true>, rows, dim3(64 * kStreamWaves), 0, s, A, tiles,
-                         V, P, n, out, wstride);
+      hipLaunchKernelGGL(k_matvec_f32_stream<true>, grid, dim3(64 * kStreamWaves), 0, s, A, tiles,
+                         V, P, n, out, wstride, pl.S, pl.even > 0);
     else
-      hipLaunchKernelGGL(k_matvec_f32_stream<false>, rows, dim3(64 * kStreamWaves), 0, s, A, tiles,
-                         V, P, n, out, wstride);
+      hipLaunchKernelGGL(k_matvec_f32_stream<false>, grid, dim3(64 * kStreamWaves), 0, s, A, tiles,
+                         V, P, n, out, wstride, pl.S, pl.even > 0);
   }
   return hipGetLastError();
 }

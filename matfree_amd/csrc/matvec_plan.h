@@ -66,8 +66,8 @@ inline bool wave_blocks(int64_t n, int64_t P, bool planed) {
 // scratch).  Workgroup form: the last round of resident workgroups (two per
 // CU) filled best.  Wave form: three per CU.  Stream form: one per CU runs
 // faster than two that share the CU's part of the bandwidth (n = 4096, 32
-// probes: 20 us in 256 workgroups, 27 in 512), so rounds of 256, by up to
-// three slices (10413: 1, 2, 3 slices take 143, 121, 117 us).  Blocks of the wave
+// probes: 20 us in 256 workgroups, 27 in 512), so as many slices as fit 256
+// workgroups (larger matrices are split evenly: F32Plan).  Blocks of the wave
 // form: rounds of 256 as well, by up to four (stored n = 2500, 128 probes: 1 to 4
 // slices take 37.0, 33.8, 32.3, 31.1 us; 2048, 64: 17.7, 13.4, 15.6, 14.8), RBF,
 // which computes more, of 512 (4095, 33 probes: 1 slice 33.1, 2 slices 31.0); more
@@ -84,7 +84,7 @@ inline int choose_splitk_f32(int64_t n, int64_t P, bool rbf, bool planed) {
   if (stream && wgs <= resident) return int(std::min<int64_t>(most, resident / wgs));
   int best = 1;
   double fill = 0.0;
-  for (int S = 1; S <= std::min(most, stream ? 3 : blocks ? 4 : most); ++S) {
+  for (int S = 1; S <= (stream ? 1 : blocks ? std::min(most, 4) : most); ++S) {
     const double rounds = double(wgs * S) / double(resident);
     const double f = rounds / std::ceil(rounds);
     if (f > (blocks ? fill * 1.16 : fill + 0.02)) {
@@ -93,6 +93,55 @@ inline int choose_splitk_f32(int64_t n, int64_t P, bool rbf, bool planed) {
     }
   }
   return best;
+}
+
+// The stream form's work: blocks of 32 rows x 128 columns, the row's last one
+// whatever is left.  A workgroup takes blocks [u0, u1) in the order of the rows
+// and goes through them in segments of one row block each.
+constexpr int kStreamTiles = 4;    // tiles of a block
+constexpr int kStreamGroups = 256;  // workgroups of the even split, one a CU
+struct StreamSegment {
+  int64_t rb, k0, k1;  // blocks [k0, k1) of row block rb
+  int64_t tile0;       // first tile
+  int64_t nwhole;      // whole tiles
+  int64_t nblocks;     // blocks that hold whole tiles
+  bool part;           // the matrix's partial last tile too
+};
+constexpr int64_t stream_runs(int64_t n) {
+  return (n + kStreamTiles * kMvTile - 1) / (kStreamTiles * kMvTile);
+}
+// The segment from block k0 of row block rb on, of `left` blocks still to do.
+constexpr StreamSegment stream_segment(int64_t n, int64_t rb, int64_t k0, int64_t left) {
+  const int64_t tiles = (n + kMvTile - 1) / kMvTile, runs = stream_runs(n);
+  StreamSegment s{};
+  s.rb = rb;
+  s.k0 = k0;
+  s.k1 = left < runs - k0 ? k0 + left : runs;
+  s.tile0 = s.k0 * kStreamTiles;
+  const int64_t end = s.k1 == runs ? tiles : s.k1 * kStreamTiles;
+  s.part = end == tiles && n % kMvTile != 0;
+  s.nwhole = end - s.tile0 - (s.part ? 1 : 0);
+  s.nblocks = (s.nwhole + kStreamTiles - 1) / kStreamTiles;
+  return s;
+}
+// Even split of all blocks over G workgroups: workgroup g's first block, and
+// the partial plane of its segment in row block rb (the row block's segments in
+// order).
+constexpr int64_t stream_split(int64_t n, int64_t G, int64_t g) {
+  return (n + kMvTile - 1) / kMvTile * stream_runs(n) * g / G;
+}
+constexpr int stream_plane(int64_t n, int64_t G, int64_t g, int64_t rb) {
+  const int64_t units = (n + kMvTile - 1) / kMvTile * stream_runs(n);
+  // the workgroup that holds the row block's first block
+  const int64_t first = ((rb * stream_runs(n) + 1) * G + units - 1) / units - 1;
+  return int(g - first);
+}
+// Planes that the even split needs: the most segments of a row block.
+inline int stream_planes(int64_t n, int64_t G) {
+  const int64_t runs = stream_runs(n), units = (n + kMvTile - 1) / kMvTile * runs;
+  if (units % G == 0 && units / G % runs == 0) return 1;
+  const int64_t least = units / G;
+  return least >= runs ? 2 : int((runs + least - 1) / least) + 1;
 }
 
 // The FP32 matvec's planes hold V and -V in turns of this many tiles (see
@@ -114,12 +163,20 @@ struct F32Plan {
   Form form;
   Input input;
   int nacc;  // workgroup form: blocks of 32 probes a workgroup
-  int S;     // column slices
+  int S;     // column slices (partial planes)
+  int even;  // stream form: workgroups of the even split, 0: row blocks x slices
 
   // planed: one of a loop of calls whose inputs come with their planes
   F32Plan(int64_t n_, int64_t P_, bool rbf, bool planed)
       : n(n_), P(P_), z(n_, P_), nacc(nacc_for(P_)) {
-    form = wave_blocks(n, P, planed) ? kWave : nacc > 1 ? kWorkgroup : rbf ? kWave : kStream;
+    // a stored matrix of one to three tiles a row has no stream to speak of (n =
+    // 32, 32 vectors: wave form 3.3 us, stream form 4.5; 96: 3.8 and 4.7; less
+    // than a tile, n = 16: 4.3 and 3.7)
+    const bool few = n >= kMvTile && n <= 3 * kMvTile;
+    form = wave_blocks(n, P, planed) ? kWave
+           : nacc > 1                ? kWorkgroup
+           : rbf || few              ? kWave
+                                     : kStream;
     input = kRows;
     // The wave form reads rows at small n, where its waves split the vectors
     // themselves (the launch that writes the planes costs about 3.5 us,
@@ -132,6 +189,18 @@ struct F32Plan {
     // the tiles save.
     if (form == kStream && n > 8960 && P > 24) input = kTiles;
     S = choose_splitk_f32(n, P, rbf, planed);
+    even = 0;
+    // Even split of a matrix beyond 4096, unless its row blocks nearly fill the
+    // CUs once (n = 8000, 1 to 32 vectors: 49.5 to 53.8 us a row block each, 52.6
+    // to 57.0 split; 7168: 44.2 to 45.6 and 43.4 to 46.0) or a partial plane more
+    // is more than the scratch holds.
+    if (form == kStream && n > 4096 && !(n <= 8192 && n > 7360)) {
+      const int planes = stream_planes(n, kStreamGroups);
+      if (planes <= choose_splitk(n, P, int64_t(1) << 60, true)) {
+        even = kStreamGroups;
+        S = planes;
+      }
+    }
   }
 
   // First tile of slice z of the workgroup form: whole runs of one plane sign.
