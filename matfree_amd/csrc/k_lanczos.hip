@@ -191,6 +191,12 @@ constexpr int kColBatch = 8;
 // the memory rather than by the latency of a block's own chain of loads.
 constexpr int64_t kManyBlocks = 1024;
 
+// Blocks below which the projection keeps a batch of columns in flight ahead of
+// the one it adds: with more, the registers cost waves (log-determinant of depth
+// 48, ahead and not: 384 blocks, n = 12288, 64 probes 4.90 and 5.07 ms; 768,
+// 12288, 128: 8.03 and 8.00; 896, 14000, 128: 10.27 and 10.14).
+constexpr int64_t kAheadBlocks = 640;
+
 // Columns of a block of the dots kernels; the other columns of a chunk are
 // blocks of their own.  As many as leave two blocks a CU: with fewer no block
 // should wait for one batch of loads after the other (n = 1001, 16 probes, 8
@@ -1214,8 +1220,8 @@ hipError_t launch_project(hipStream_t s, const float* Q, int64_t ldc, const floa
   const size_t shmem = size_t(ncols > 0 ? ncols : 1) * sizeof(float);
   const int V = stream_width(n, ldc, {x, y, Q});
   if (planes && V != 4) return hipErrorInvalidValue;
-  const bool ahead = nb * P < kManyBlocks;
-  if (ahead) back = 0;
+  const bool ahead = nb * P < kAheadBlocks;
+  if (nb * P < kManyBlocks) back = 0;
 #define SLQ_PROJECT(K, ...)                                                                     \
   hipLaunchKernelGGL(K, grid, dim3(kStreamThreads), shmem, s, Q, ldc, x, y, n, ncols, hpart,    \
                      pstride, norm2part, hout, hout_stride, hsub, hsub_stride, back, ##__VA_ARGS__)
