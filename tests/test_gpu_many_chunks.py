@@ -1,10 +1,11 @@
-"""The Gram-Schmidt passes on both sides of their few / many blocks rule.
+"""The Gram-Schmidt passes of many blocks (chunks of 2048 elements times probes).
 
-From 1024 blocks (chunks of 2048 elements times probes) the dots take up to 32
-columns a block and the projection keeps one batch of columns in flight; below,
-8 columns a block and one batch ahead.  ``tridiag_sym`` of a stored matrix with
-spectrum in [1, 2] against the FP64 restatement, at depths on both sides of the
-column groups, rows of whole float4 groups and rows of odd length.  Tolerances:
+From 1024 blocks the passes over the basis take the probes in alternating order
+(n = 2052 and 2050 here; rows of one chunk, n = 131 and 132, take a step in one
+workgroup a probe).  ``tridiag_sym`` of a stored matrix with spectrum in [1, 2]
+against the FP64 restatement, rows of whole float4 groups and others.  The
+columns a block of the dots takes and the projection's rule:
+test_gpu_pass_rules.py.  Tolerances:
 the FP32 products are good to 1e-6 and the recurrence at these depths grows an
 error by less than 100 (1e-4 normwise); two classical passes keep the basis
 orthonormal to a few FP32 roundings of sums over n (1e-5).

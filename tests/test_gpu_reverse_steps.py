@@ -5,8 +5,9 @@ the rows are whole groups of four (n % 4 == 0), the product's split-K sum is
 formed by the dots that read it, and the rows of dQ^T Q are done together
 unless the rows of dQ differ in alignment (P n not a multiple of 4).  Random
 cotangents on every output of ``hessenberg`` against the FP64 restatement of
-decomp.py:480-600, one chunk of a probe's vector and two, more than 32 probes
-(three planes) and fewer.  Tolerances: 1e-4 normwise for FP32 operators of
+decomp.py:480-600, one chunk of a probe's vector (a step in one workgroup a
+probe) and two, more than 32 probes and fewer.  The planes from the projection
+of longer rows: test_gpu_pass_rules.py.  Tolerances: 1e-4 normwise for FP32 operators of
 condition number below ten at depth 6 (products to 1e-6, growth through the
 scan below 100); for bf16x3, whose products are good to 2^-16, the same growth
 gives 1.5e-3.
