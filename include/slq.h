@@ -48,7 +48,8 @@ typedef enum slq_operator_kind {
 } slq_operator_kind;
 
 typedef enum slq_precision {
-  SLQ_PREC_FP32 = 0,   /* FP32 MFMA, FP32 operands                                */
+  SLQ_PREC_FP32 = 0,   /* FP32 operands: FP32 MFMA, or six BF16 products of       */
+                       /* three-part splits (products to 2^-26 relative)          */
   SLQ_PREC_BF16 = 1,   /* one BF16 MFMA product, FP32 accumulation                 */
   SLQ_PREC_BF16X3 = 2, /* split hi+lo BF16: hi*hi + hi*lo + lo*hi, FP32 accumulation */
   SLQ_PREC_BF16X2 = 3  /* matrix split hi+lo, vectors BF16: hi*hi + lo*hi           */

@@ -3,16 +3,19 @@
 // contraction W[p][i] = sum_m A[i][m] V[p][m] on the matrix cores.
 //
 // FP32 path, D[i][p] on the matrix cores (rows = output elements, columns =
-// probes), in three forms (which one: launch_f32):
+// probes), in three forms (which one: F32Plan,
+// matvec_plan.h):
 //
 //  * workgroup form (more than 32 probes): 128 rows x 64 or 128 probes, six
-//    products of three BF16 parts per factor (k_matvec_f32); the probes' parts and the
-//    matrix tiles (or the tile's points) pass through LDS, an entry is formed
-//    once and used for every probe;
-//  * wave form (RBF, up to 32 probes): the same products, four waves sharing
-//    32 rows by tiles, no LDS sharing and no barrier in the loop;
+//    products of three BF16 parts per factor (k_matvec_f32); the probes' parts
+//    and the matrix tiles (or the tile's points) pass through LDS, an entry is
+//    formed once and used for every probe;
+//  * wave form (RBF, up to 32 probes, and small problems of more): the same
+//    products, four waves sharing 32 rows by tiles, no LDS sharing and no
+//    barrier in the loop;
 //  * stream form (stored matrix, up to 32 probes): v_mfma_f32_32x32x2f32 with
 //    the matrix loaded to LDS by a wave of its own.
+// A fourth, k_matvec_f32_units, is taken where a decomposition is differentiated.
 //
 // RBF: K_im = exp2(c |x_i - x_m|^2), c = -log2(e) / (2 l^2); the nugget
 // s2 * v is added in FP32 in the epilogue (never folded into a tile).
@@ -516,12 +519,12 @@ __device__ floatx16 f32_block(const float* __restrict__ A, const RBFParams& prm,
 // rounded to nearest): a bias of one sign in every output, which a recursion
 // adds up (a decomposition's start-vector cotangent lost a factor of five).
 // So the planes hold V and -V in turns of kSignRun tiles, whose products are
-// added with that sign, and the biases cancel.  Sums are kept in levels (a
-// tile or a pair of tiles, 16 tiles, the slice), smallest products first:
-// against 64 bits the result is 1.2x (n = 1001) to 3x (n = 32768) nearer than
+// added with that sign, and the biases cancel (in the wave form between its
+// waves).  Sums are kept in levels, smallest products first: a tile, kTileRun
+// tiles, the slice (the RBF workgroup form: a pair of tiles, the slice).
+// Against 64 bits the result is 1.2x (n = 1001) to 3x (n = 32768) nearer than
 // the FP32 MFMA chain's.
 constexpr int kTileRun = 16;
-
 
 // Workgroup form, for more than 32 probes: 128 rows x 32 NACC probes, 32 rows
 // per wave.  The matrix cores bound it (48 products of 32 cycles a tile and

@@ -183,10 +183,12 @@ struct F32Plan {
     // splitting in the waves 0.2 us per 1000 columns).
     if (form == kWorkgroup || (form == kWave && nacc == 1 && n >= 4096)) input = kPlanes;
     // The stream form's tiles are written by the producer of the input where
-    // there is one, in a launch of about 3.5 us otherwise.  With up to 16
-    // probes most of a tile is padding, and its lines cost more than the rows'
-    // (15001, 16 probes: 199 -> 208 us); up to n = 8400 the launch costs what
-    // the tiles save.
+    // there is one, in a launch of about 3.5 us otherwise.  With few probes
+    // most of a tile is padding, and its lines cost more than the rows' (a
+    // product with that launch, rows and tiles: n = 10413, 16 probes 99.1 and
+    // 105.9 us, 24: 105.3 and 105.8, 25: 108.2 and 105.3, 32: 114.0 and 109.9);
+    // for less than n = 9000 the launch costs more than the tiles save (8600, 32
+    // probes: 71.4 and 73.7; 8961: 88.5 and 81.6).
     if (form == kStream && n > 8960 && P > 24) input = kTiles;
     S = choose_splitk_f32(n, P, rbf, planed);
     even = 0;
