@@ -1546,6 +1546,88 @@ __global__ void __launch_bounds__(kThreads)
   store_out<NACC, false, false>(Wout, V, P, n, i0w, p0, acc, 0.f);
 }
 
+// The same sums for up to 32 probes of a small matrix, where the rows give a
+// few workgroups and each is a serial chain of a slice's tiles (1024 cycles of
+// matrix core each, 8 to 15 tiles): a workgroup of 32 rows deals the tiles to
+// eight waves, which leave their sums in LDS, and adds those in the order of the
+// tiles (bit for bit the form above).  No barrier before that: a wave reads its
+// rows and probes straight from memory, at most two tiles, all loads ahead.
+// Decomposition with its reverse pass, form above -> this one: n = 512, 1 probe,
+// depth 32 2.12 -> 1.80 ms; 768, 2, 30: 2.28 -> 1.86; 1500, 1, 32: 2.63 -> 2.18;
+// 2048, 32, 32: 2.86 -> 2.68; beyond two workgroups a CU 2500, 16, 32: 3.40 ->
+// 3.58; 4096, 32, 32: 4.20 -> 5.07.
+constexpr int kUnitsWaves = 8;
+constexpr int kUnitsTiles = 2 * kUnitsWaves;  // tiles of a slice, 4 KB of LDS each
+constexpr int kUnitsDealt = 512;              // workgroups it is taken up to
+
+__global__ void __launch_bounds__(64 * kUnitsWaves)
+    k_matvec_f32_units_dealt(const float* __restrict__ A, const float* __restrict__ V, int64_t P,
+                             int64_t n, float* __restrict__ W) {
+  extern __shared__ __attribute__((aligned(16))) float units_sums[];  // [tile][16][64]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, h = lane >> 5;
+  const int64_t i0 = int64_t(blockIdx.x) * 32;
+  const int64_t all_tiles = (n + BK - 1) / BK;
+  const int64_t kt_begin = all_tiles * blockIdx.z / gridDim.z;
+  const int ntiles = int(all_tiles * (blockIdx.z + 1) / gridDim.z - kt_begin);
+  // rows past n and probes past P as the last (not stored)
+  const float* arow = A + (i0 + r < n ? i0 + r : n - 1) * n;
+  const float* vrow = V + (r < P ? r : P - 1) * n;
+  auto load4 = [&](const float* base, int64_t m, bool whole) {
+    if (whole) return load4u(base + m);
+    return make_float4(m + 0 < n ? base[m + 0] : 0.f, m + 1 < n ? base[m + 1] : 0.f,
+                       m + 2 < n ? base[m + 2] : 0.f, m + 3 < n ? base[m + 3] : 0.f);
+  };
+  float4 a[2][4], v[2][4];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int kt = wave + j * kUnitsWaves;
+    if (kt < ntiles) {
+      const int64_t m0 = (kt_begin + kt) * BK;
+      const bool whole = m0 + BK <= n;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        a[j][g] = load4(arow, m0 + 16 * h + 4 * g, whole);
+        v[j][g] = load4(vrow, m0 + 16 * h + 4 * g, whole);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int kt = wave + j * kUnitsWaves;
+    if (kt < ntiles) {
+      floatx16 tmp;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) tmp[e] = 0.f;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float fa[4] = {a[j][g].x, a[j][g].y, a[j][g].z, a[j][g].w};
+        const float fb[4] = {v[j][g].x, v[j][g].y, v[j][g].z, v[j][g].w};
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          tmp = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[u], fb[u], tmp, 0, 0, 0);
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) units_sums[(kt * 16 + e) * 64 + lane] = tmp[e];
+    }
+  }
+  __syncthreads();
+  // waves 0 .. 3 sum and store four consecutive rows a lane (store_out's layout)
+  if (wave >= 4 || r >= P) return;
+  float o[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int kt = 0; kt < ntiles; ++kt)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] += units_sums[(kt * 16 + 4 * wave + e) * 64 + lane];
+  const int64_t i = i0 + 8 * wave + 4 * h;
+  float* out = W + (int64_t(blockIdx.z) * P + r) * n + i;
+  if (i + 4 <= n) {
+    store4u(out, make_float4(o[0], o[1], o[2], o[3]));
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (i + e < n) out[e] = o[e];
+  }
+}
+
 // RBF exponents for the BF16 kernels.  The base-2 exponent of a 32 x 32 tile,
 //   arg[m][i] = c |x_m|^2 + c |x_i|^2 + sum_d x_m,d (-2c x_i,d),
 // is a short sum of products of FP32 numbers.  Each factor f is split into
@@ -3039,8 +3121,13 @@ hipError_t launch_matvec(hipStream_t s, const slq_operator& op, const float* V, 
     const dim3 grid(unsigned((n + BI - 1) / BI), unsigned((P + 32 * nacc - 1) / (32 * nacc)),
                     unsigned(S));
     float* out = S > 1 ? partial : W;
+    const int64_t slice = ((n + BK - 1) / BK + S - 1) / S;  // tiles of the longest
     if (ev0) (void)hipEventRecord(ev0, s);
-    if (nacc == 1)
+    if (nacc == 1 && slice <= kUnitsTiles && (n + 31) / 32 * S <= kUnitsDealt)
+      hipLaunchKernelGGL(k_matvec_f32_units_dealt,
+                         dim3(unsigned((n + 31) / 32), 1, unsigned(S)), dim3(64 * kUnitsWaves),
+                         size_t(slice) * 4096, s, op.matrix, V, P, n, out);
+    else if (nacc == 1)
       hipLaunchKernelGGL(k_matvec_f32_units<1>, grid, dim3(kThreads), 0, s, op.matrix, V, P, n, out);
     else if (nacc == 2)
       hipLaunchKernelGGL(k_matvec_f32_units<2>, grid, dim3(kThreads), 0, s, op.matrix, V, P, n, out);

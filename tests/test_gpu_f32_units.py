@@ -27,3 +27,20 @@ def test_relation_of_the_matrix_cores_products(cuda, n, P):
     rhs = H.transpose(1, 2) @ Q
     rhs[:, -1] += r
     assert float((Q @ A.double() - rhs).norm(dim=2).max() / norm) < 1e-5
+
+
+# one, a few, eight, nine and fifteen tiles a slice; 1 to 8 slices; up to 2048
+# dealt to waves for up to 32 probes and not beyond, or with more probes
+@pytest.mark.parametrize("n", [1, 31, 96, 255, 257, 480, 511, 513, 991, 1500, 2047, 2048])
+@pytest.mark.parametrize("P", [1, 31, 32])
+def test_few_probes_take_the_same_sums(cuda, n, P):
+    """A probe's decomposition does not depend on how many there are: the tiles'
+    sums are added in one order, bit for bit."""
+    gen = torch.Generator().manual_seed(n)
+    A = (torch.randn((n, n), generator=gen) / n**0.5).to(cuda).requires_grad_()
+    V = torch.randn((33, n), generator=gen).to(cuda)
+    many, few = (decomp.hessenberg(min(n, 3), reortho="full").batched(
+        operators.dense_matvec, x, A) for x in (V, V[:P]))
+    for a, b in zip(few, many):
+        assert torch.isfinite(a).all()
+        assert torch.equal(a, b[:P])
